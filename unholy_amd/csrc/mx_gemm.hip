@@ -664,16 +664,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 // The same workgroup shape as mx_gemm_pipe_kernel (256 threads, one tile x 256 output columns, wave w owns columns
 // 64 w .. 64 w + 63 over all rows, 16x16x32 bf16 MFMAs, one per 32-input block), but the activations arrive as bf16:
 // they go from LDS straight into the MFMA with no conversion, and only the weights are dequantized (half a
-// conversion per MFMA instead of one and a half). Stages are 64 inputs, three ring slots of 24.5 KB (73.5 KB, two
-// workgroups per CU), two stages in flight. Per stage a slot holds
-//   A  16 KB: 128 rows x 64 bf16, row r's 16-byte piece p at slot r * 8 + (p ^ lds_swz(r));
-//   B   8 KB: 8 blocks of 1 KB = (projection or column half q, 32-column block c), slot h * 32 + n <- piece 2n + h;
+// conversion per MFMA instead of one and a half). Stages are 64 inputs. Per stage a slot holds
+//   A  4 KB per 32 live rows: rows x 64 bf16, row r's 16-byte piece p at slot r * 8 + (p ^ lds_swz(r));
+//   B  8 KB: 8 blocks of 1 KB = (projection or column half q, 32-column block c), slot h * 32 + n <- piece 2n + h;
 //   Bs 512 B: the e8m0 weight scales of projection q at q * 256 in their global order.
-// Every wave issues 4 A, 2 B and 1 scale load per stage (7 vm operations).
+// The ring is shaped by the tile's live rows (GbRing): only they are loaded, and the LDS that short tiles leave holds
+// more stages.
 constexpr int kSkinnyMaxRows = 64;  // mx_grouped_gemm's max_rows bound for the GEMV route
-constexpr int GB_KS = 64, GB_A = 128 * 128, GB_B = 8 * 1024, GB_BS = 512;
-constexpr int GB_STAGE = GB_A + GB_B + GB_BS;
-constexpr int GB_S = 3, GB_RING = GB_S * GB_STAGE;
+constexpr int GB_KS = 64, GB_B = 8 * 1024, GB_BS = 512;
+constexpr int GB_RING = 3 * (16 * 1024 + GB_B + GB_BS);  // 73.5 KB: two workgroups per CU
+
+// The ring of a tile of RB live 16-row blocks: NA activation loads per wave and stage, S slots (S - 1 stages in
+// flight). Every wave issues NA A, 2 B and 1 scale load per stage.
+template <int RB>
+struct GbRing {
+  static constexpr int NA = (RB + 1) / 2, A = NA * 4096, STAGE = A + GB_B + GB_BS;
+  static constexpr int S = GB_RING / STAGE, NL = NA + 3;
+  static_assert(S >= 3 && (S - 2) * NL < 64);
+};
 static_assert(GP_C1 <= GB_RING && GP_C2 + GP_ROWS <= GB_RING && 64 * (256 + 4) * 4 <= GB_RING,
               "the C tiles reuse the ring");
 
@@ -685,87 +693,103 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   if (by >= a.ntiles || (a.ntiles_dev && by >= *a.ntiles_dev)) return;
   const Exl3Tile tile = a.tiles[by];
   if (tile.rows <= 0) return;
-  const uint8_t* wq[2];
-  const uint8_t* sq[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    wq[q] = a.w_tab[NP == 2 ? q : 0][tile.expert];
-    sq[q] = a.s_tab[NP == 2 ? q : 0][tile.expert];
-    if (!wq[q] || !sq[q]) return;
-  }
-  const int K = a.K, KS = K / GB_KS, N = a.N, ntn = N / 16;
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // column quarter
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);  // column quarter
   const int cq = wave, q_own = cq >> 1;
+  const int K = a.K, KS = K / GB_KS, N = a.N, ntn = N / 16;
   // NP 1: columns bx 256 .. + 255 as two 128-column halves; the last block of a matrix with N % 256 == 128 has only
   // the first half, and its second-half waves stream that half again (their results are not stored).
   const int colq0 = NP == 2 ? bx * 128 : bx * 256, colq_step = NP == 2 || colq0 + 128 >= N ? 0 : 128;
+  const uint8_t *wsrc, *ssrc;  // the wave's weight blocks (2 KB of a stage's 8) and scales (128 bytes of 512), stage 0
+  {
+    const uint8_t* wq[2];
+    const uint8_t* sq[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      wq[q] = a.w_tab[NP == 2 ? q : 0][tile.expert];
+      sq[q] = a.s_tab[NP == 2 ? q : 0][tile.expert];
+      if (!wq[q] || !sq[q]) return;
+    }
+    const size_t nt0 = size_t(colq0 + q_own * colq_step) / 16;
+    wsrc = reinterpret_cast<const uint8_t*>(uniform_ptr(wq[q_own] + nt0 * 512 + (wave & 1) * 2048));
+    ssrc = reinterpret_cast<const uint8_t*>(uniform_ptr(sq[q_own] + nt0 * 32 + (wave & 1) * 128));
+  }
   const size_t cslab = size_t(ntn) * 512, sslab = size_t(ntn) * 32;
   const uint32_t lds0 = lds_addr(smem);
-  const uint32_t boff = uint32_t((l32 * 2 + h) * 16);  // B block: slot h*32+n <- piece 2n+h
-  const int m16 = lane & 15, g = lane >> 4;
-  // A piece of row rb * 16 + m16, inputs 32 b + 8 g .. + 7 (piece 4b + g): byte a_lane[b] + rb * 2048 of the stage
-  // (lds_swz(rb * 16 + m16) == lds_swz(m16)).
-  const uint32_t a_lane0 = uint32_t(m16 * 128 + ((g ^ lds_swz(m16)) << 4));
-  const uint32_t a_lane1 = uint32_t(m16 * 128 + (((4 + g) ^ lds_swz(m16)) << 4));
-  // B word of column block cb, block b: byte b_lane + (cb >> 1) * 1024 + b * 512 + (cb & 1) * 256; the two scales
-  // of column block cb (b = 0, 1) the u16 at s_lane + cb * 32.
-  const uint32_t b_lane = uint32_t(GB_A + q_own * 4096 + (cq & 1) * 2048 + m16 * 16 + 4 * g);
-  const uint32_t s_lane = uint32_t(GB_A + GB_B + q_own * 256 + (cq & 1) * 128 + m16 * 2);
 
   for (int rg = 0; rg < tile.rows; rg += 128) {
     const int M = min(128, tile.rows - rg);
     const size_t row0 = size_t(tile.row0) + rg;
     __syncthreads();  // the previous row group's LDS use is over
-    // Each lane's A source in 16-byte units from a.xa (a gathered row's byte offset can pass 4 GiB).
-    uint32_t a16[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int slot = (wave * 4 + i) * 64 + lane, r = slot >> 3, p = (slot & 7) ^ lds_swz(r);
-      const int rr = min(r, M - 1);  // rows past the tile repeat its last
-      a16[i] = uint32_t(a.x_rows ? a.x_rows[row0 + rr] : int(row0 + rr)) * uint32_t(K / 8) + uint32_t(p);
-    }
-    const auto issue = [&](int s) {
-      const uint32_t st = __builtin_amdgcn_readfirstlane(lds0 + uint32_t((s % GB_S) * GB_STAGE));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dma16_g(a.xa + s * 64, a16[i], st + uint32_t(wave * 4 + i) * 1024);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int u = wave * 2 + i, q = u >> 2, c = u & 3;
-        const uint8_t* bb = wq[q] + size_t(s) * cslab + size_t((colq0 + q * colq_step) / 16) * 512 + c * 1024;
-        dma16_nt(bb, boff, st + uint32_t(GB_A + u * 1024));
-      }
-      {  // scales: wave w copies bytes 128 w .. + 127 (projection w / 2), 8 lanes of 16 bytes
-        const int q = wave >> 1;
-        const uint8_t* sb = sq[q] + size_t(s) * sslab + size_t((colq0 + q * colq_step) / 16) * 32 + (wave & 1) * 128;
-        if (lane < 8) dma16(sb, uint32_t(lane) * 16, st + uint32_t(GB_A + GB_B + wave * 128));
-      }
-    };
-    issue(0);
-    if (KS > 1) issue(1);
 
     const auto tile_body = [&](auto nrb) {
       constexpr int RB = decltype(nrb)::value;
+      using T = GbRing<RB>;
+      constexpr int NA = T::NA, S = T::S, NL = T::NL;
+      // Opaque per body, so that the lane addresses of the eight bodies are not all formed (and spilled) ahead of them.
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+      const uint32_t boff = uint32_t((l32 * 2 + h) * 16);  // B block: slot h*32+n <- piece 2n+h
+      const int m16 = lane & 15, g = lane >> 4;
+      // A piece of row rb * 16 + m16, inputs 32 b + 8 g .. + 7 (piece 4b + g): byte a_lane[b] + rb * 2048 of the stage
+      // (lds_swz(rb * 16 + m16) == lds_swz(m16)).
+      const uint32_t a_lane0 = uint32_t(m16 * 128 + ((g ^ lds_swz(m16)) << 4));
+      const uint32_t a_lane1 = uint32_t(m16 * 128 + (((4 + g) ^ lds_swz(m16)) << 4));
+      // B word of column block cb, block b: byte A + b_lane + (cb >> 1) * 1024 + b * 512 + (cb & 1) * 256; the two scales
+      // of column block cb (b = 0, 1) the u16 at A + s_lane + cb * 32.
+      const uint32_t b_lane = uint32_t(q_own * 4096 + (cq & 1) * 2048 + m16 * 16 + 4 * g);
+      const uint32_t s_lane = uint32_t(GB_B + q_own * 256 + (cq & 1) * 128 + m16 * 2);
+      // Each lane's A source in 16-byte units from a.xa (a gathered row's byte offset can pass 4 GiB).
+      uint32_t a16[NA];
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const int slot = (wave * NA + i) * 64 + lane, r = slot >> 3, p = (slot & 7) ^ lds_swz(r);
+        const int rr = min(r, M - 1);  // rows past the tile repeat its last
+        a16[i] = uint32_t(a.x_rows ? a.x_rows[row0 + rr] : int(row0 + rr)) * uint32_t(K / 8) + uint32_t(p);
+      }
+      const auto issue = [&](int s) {
+        const uint32_t st = __builtin_amdgcn_readfirstlane(lds0 + uint32_t((s % S) * T::STAGE));
+        // The stage index as an opaque scalar: its source addresses are then formed in scalar registers here, not
+        // carried through the loop in vector registers (whose spills would wait for every load in flight).
+        int ss = s;
+        asm volatile("" : "+s"(ss));
+#pragma unroll
+        for (int i = 0; i < NA; ++i) dma16_g(a.xa + size_t(ss) * 64, a16[i], st + uint32_t(wave * NA + i) * 1024);
+        const uint8_t* const wb = wsrc + size_t(ss) * cslab;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma16_nt(wb + i * 1024, boff, st + uint32_t(T::A + (wave * 2 + i) * 1024));
+        if (lane < 8)  // scales: 8 lanes of 16 bytes
+          dma16(ssrc + size_t(ss) * sslab, uint32_t(lane) * 16, st + uint32_t(T::A + GB_B + wave * 128));
+      };
+#pragma unroll
+      for (int s = 0; s < S - 1; ++s)
+        if (s < KS) issue(s);
       v4f acc[RB][4];
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) acc[rb][cb] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
       for (int s = 0; s < KS; ++s) {
-        if (s + 1 < KS) wait_vm<7>();  // stage s has landed; stage s + 1 may still be in flight
+        // Stage s has landed when only the loads of the stages issued after it are in flight.
+        const int after = KS - 1 - s;
+        if (after >= S - 2) wait_vm<(S - 2) * NL>();
+        else if (S > 4 && after >= 3) wait_vm<(S > 4 ? 3 : 0) * NL>();
+        else if (S > 3 && after >= 2) wait_vm<(S > 3 ? 2 : 0) * NL>();
+        else if (after >= 1) wait_vm<NL>();
         else wait_vm<0>();
-        __syncthreads();  // every wave's part of stage s has landed; slot (s + 2) % 3 (stage s - 1) is free
-        if (s + 2 < KS) issue(s + 2);
-        const uint8_t* stb = smem + (s % GB_S) * GB_STAGE;
+        __syncthreads();  // every wave's part of stage s has landed; the slot of stage s - 1 is free
+        if (s + S - 1 < KS) issue(s + S - 1);
+        const uint8_t* stb = smem + (s % S) * T::STAGE;
         uint32_t bsc[4], bw[2][4];
         bf16x8 af[2][RB];
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) bsc[cb] = *reinterpret_cast<const uint16_t*>(stb + s_lane + cb * 32);
+        for (int cb = 0; cb < 4; ++cb) bsc[cb] = *reinterpret_cast<const uint16_t*>(stb + T::A + s_lane + cb * 32);
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int cb = 0; cb < 4; ++cb)
-            bw[b][cb] = *reinterpret_cast<const uint32_t*>(stb + b_lane + (cb >> 1) * 1024 + b * 512 + (cb & 1) * 256);
+            bw[b][cb] = *reinterpret_cast<const uint32_t*>(stb + T::A + b_lane + (cb >> 1) * 1024 + b * 512 +
+                                                           (cb & 1) * 256);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) af[0][rb] = *reinterpret_cast<const bf16x8*>(stb + a_lane0 + rb * 2048);
         __builtin_amdgcn_sched_barrier(0);  // the stage's first reads all issued before any use
