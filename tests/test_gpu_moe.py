@@ -306,3 +306,28 @@ def test_forward_matches_composed_entry_points(T, E, K, D, I):
     call("uh_moe_combine", pair, b["pidx"], None, comp, T, K, D, None)
     synchronize()
     assert np.array_equal(out.download((T, D), np.uint16), comp.download((T, D), np.uint16))
+
+
+@pytest.mark.parametrize("T,E,K,D,I", [(9, 16, 2, 256, 128), (40, 32, 6, 512, 256), (64, 64, 8, 256, 128),
+                                       (40, 16, 2, 256, 256), (380, 80, 2, 512, 256), (380, 16, 2, 512, 256)])
+def test_moe_forward_tile_sizes(T, E, K, D, I):
+    """The forward's GEMM steps over skewed routing: experts with 1 to 130 rows (every count of 16-row blocks of a
+    workgroup, a tile past 64 rows where the few-rows kernel takes two groups, tiles past 128 rows), the one-block and
+    the many-block dispatch, 2 I > D (no room for hh in the workspace of a small step: the GEMVs). Against the oracle,
+    max-rel <= 1e-2 per element as test_moe_forward_vs_oracle."""
+    rng = np.random.default_rng(T + E + K + I)
+    experts, bufs, tab, x, logits = _moe_case(rng, T, E, K, D, I)
+    t0 = 0
+    for e, n in enumerate((130, 65, 64, 49, 33, 17, 16, 1)):
+        logits[t0:t0 + n, e] += 12.0  # the first pick of the next n tokens
+        t0 += n
+    sel_ref, wt_ref = oracle.route_softmax(logits, K)
+    out_ref, _ = oracle.moe_forward(x, sel_ref, wt_ref, experts, D, I, 10.0)
+    ws_bytes = call("uh_mx_moe_workspace_size", T, K, E, D, I)
+    ws, out = DeviceBuffer(ws_bytes), DeviceBuffer(T * D * 2)
+    sel, wt = DeviceBuffer(T * K * 4), DeviceBuffer(T * K * 4)
+    call("uh_mx_moe_forward", dev(x), dev(logits), T, K, E, D, I, tab.ptr, 10.0, ws.ptr, ws_bytes, out.ptr, sel.ptr,
+         wt.ptr, None)
+    synchronize()
+    assert np.array_equal(sel.download((T, K), np.int32), sel_ref)
+    assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2

@@ -96,17 +96,17 @@ struct MoeWs {
   int32_t *count, *off, *fill, *plan, *tiles, *eidx, *row_expert, *pidx, *sel;
   float *ewt, *wt;
   uint8_t *xq, *xs, *hq, *hs;
-  bf16 *xa, *hh;  // prefill: fake-quantized token rows [T, D] (in xq's bytes) and SwiGLU rows [P, I]
+  bf16 *xa, *hh;  // GEMM steps: fake-quantized token rows [T, D] (in xq's bytes) and SwiGLU rows [P, I]
   bf16* h;  // raw SwiGLU rows [P, I] (T <= 64 path); shares xq's bytes (P * D >= P * I * 2), which only prefill uses
   bf16* pair_out;
   size_t bytes;
-  int max_tiles, tile_rows;
+  int max_tiles;
 };
 MoeWs carve(char* base, int T, int K, int E, int D, int I) {
   MoeWs w{};
   const size_t P = size_t(T) * K;
-  w.tile_rows = T <= 64 ? 16 : k::kExl3TileRows;
-  w.max_tiles = int(std::min<size_t>(P, size_t(E) + P / size_t(w.tile_rows) + 1));
+  const int tile_rows = T <= 64 ? 16 : k::kExl3TileRows;  // (a GEMM step of up to 64 tokens has fewer tiles)
+  w.max_tiles = int(std::min<size_t>(P, size_t(E) + P / size_t(tile_rows) + 1));
   size_t o = 0;
   auto take = [&](size_t bytes) {
     char* p = base ? base + o : nullptr;
@@ -130,8 +130,14 @@ MoeWs carve(char* base, int T, int K, int E, int D, int I) {
   w.xs = reinterpret_cast<uint8_t*>(take(P * (D / 128)));
   w.hq = reinterpret_cast<uint8_t*>(take(P * I));
   w.hs = reinterpret_cast<uint8_t*>(take(P * (I / 128)));
+  char* const codes_end = base ? base + o : nullptr;  // xq, xs, hq and hs lie one after another
   w.xa = reinterpret_cast<bf16*>(w.xq);  // T * D * 2 <= P * D
-  w.hh = T > 64 ? reinterpret_cast<bf16*>(take(P * I * 2)) : nullptr;
+  if (T > 64) {
+    w.hh = reinterpret_cast<bf16*>(take(P * I * 2));
+  } else if (base) {  // behind xa, in the bytes that only the fp8-code GEMMs use (K = 6, I = D / 2: room for it)
+    char* const hh = reinterpret_cast<char*>(w.xq) + (size_t(T) * D * 2 + 255) / 256 * 256;
+    if (size_t(D) >= size_t(I) * 2 && hh + P * I * 2 <= codes_end) w.hh = reinterpret_cast<bf16*>(hh);
+  }
   w.pair_out = reinterpret_cast<bf16*>(take(P * D * 2));
   w.bytes = o;
   return w;
@@ -819,7 +825,16 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     // Dispatch in one single-block launch up to 512 picks; the routing in that launch too while every token has a
     // wave of its own (T <= 8), else a wave per token over many workgroups first.
     const bool one_block = P <= k::kMoeMidMaxPicks, route_in = one_block && T <= 8;
-    if (!route_in) k::route_softmax(logits, s_sel, s_wt, T, E, K, st);
+    // The GEMM on bf16 rows from 9 tokens on, the GEMV below it (us per forward, GEMV / GEMM, K = 6: E = 256, D = 4096,
+    // I = 2048: T = 8 111 / 114, 9 125 / 121, 16 181 / 171, 64 353 / 337; E = 32: T = 8 76 / 73, 16 86 / 79, 64
+    // 127 / 92; E = 64, D = 2048, I = 1024: T = 8 33 / 38, 16 52 / 45). Up to 64 tokens the fp8-code and
+    // block-scaled GEMMs are not used, whatever the switches say, and a workspace without room for hh keeps the GEMV.
+    const bool bf16_rows = !prefill_fp8() && k::mx_gemm_exact();
+    const bool rows16 = bf16_rows && (T > 64 || (T > 8 && w.hh && k::mx_gemm_pipe_on())), gemv = T <= 64 && !rows16;
+    const int tile_rows = gemv ? 16 : k::kExl3TileRows;
+    const bool few_rows = size_t(P) <= size_t(10) * E;  // at most 10 rows per expert on average: tiles of few rows
+    if (rows16) k::launch_route_xform(logits, s_sel, s_wt, T, E, K, x, w.xa, D, st);
+    else if (!route_in) k::route_softmax(logits, s_sel, s_wt, T, E, K, st);
     const int* ntd = &reinterpret_cast<const k::MoePlan*>(w.plan)->n_local_tiles;
     k::Exl3Tile* tiles = reinterpret_cast<k::Exl3Tile*>(w.tiles);
     if (one_block) {
@@ -831,7 +846,7 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
       a.E = E;
       a.P = P;
       a.max_tiles = w.max_tiles;
-      a.tile_rows = w.tile_rows;
+      a.tile_rows = tile_rows;
       a.plan = reinterpret_cast<k::MoePlan*>(w.plan);
       a.lt = tiles;
       a.eidx = w.eidx;
@@ -841,51 +856,48 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
       a.softmax_logits = route_in ? logits : nullptr;
       k::moe_dispatch_mid(a, st);
     } else {
-      k::launch_zero_words(w.count, size_t(E), st);  // a kernel: no memset node if the caller captures a graph
-      k::moe_count(s_sel, T, K, w.count, E, st);
-      k::moe_plan(w.count, nullptr, E, P, reinterpret_cast<k::MoePlan*>(w.plan), tiles, nullptr, w.off, w.fill,
-                  w.max_tiles, st, w.tile_rows);
-      k::moe_scatter_e(s_sel, s_wt, T, K, E, w.off, w.eidx, w.ewt, w.row_expert, w.pidx, st);
+      k::launch_moe_dispatch_all(s_sel, s_wt, T, K, E, reinterpret_cast<k::MoePlan*>(w.plan), tiles, w.max_tiles,
+                                 tile_rows, w.eidx, w.ewt, w.row_expert, w.pidx, st);
     }
     mark(1);
     const k::MxGlu glu{w.ewt, w.row_expert, t(2, 1), nullptr, limit, nullptr, w.hq, w.hs};
-    if (T <= 64) {
+    if (gemv) {
       // Both GEMVs quantize their inputs while staging them: x rows per 128 for w1 / w3, and for w2 the raw SwiGLU
       // rows h, whose act_quant codes are exactly those of the fake-quantized hh. A tile holds at most one row per
       // token, so min(tile_rows, T) rows bound the staging.
       k::MxGlu gh = glu;
       gh.hq = gh.hs = nullptr;
       gh.h = w.h;
-      const int rows = std::min(w.tile_rows, T);
+      const int rows = std::min(tile_rows, T);
       mark(2);
       k::mx_grouped_gemv_x(x, D, w.eidx, D, tiles, w.max_tiles, t(0, 0), t(0, 1), nullptr, I, I, st, ntd, t(1, 0),
                            t(1, 1), nullptr, rows, gh);
       mark(3);
       k::mx_grouped_gemv_x(w.h, I, nullptr, I, tiles, w.max_tiles, t(2, 0), t(2, 1), w.pair_out, D, D, st, ntd,
                            nullptr, nullptr, nullptr, rows, k::MxGlu{});
-    } else if (!prefill_fp8() && k::mx_gemm_exact()) {
+    } else if (rows16) {
       // Each token row fake-quantized once to bf16 (exact e4m3 x 2^k values; its K picks would otherwise be
       // quantized K times); the w1 / w3 GEMM gathers the pair rows through eidx and writes the fake-quantized
       // SwiGLU rows hh, the w2 GEMM's bf16 input.
-      k::mx_xform_in(x, D, nullptr, nullptr, w.xa, T, D, st, nullptr);
       mark(2);
       k::MxGlu gb = glu;
       gb.hq = gb.hs = nullptr;
       gb.hh = w.hh;
-      k::mx_grouped_gemm_rows(w.xa, w.eidx, D, tiles, w.max_tiles, t(0, 0), t(0, 1), nullptr, I, I, st, ntd, t(1, 0),
-                              t(1, 1), nullptr, gb);
+      k::launch_mx_gemm_rows(w.xa, w.eidx, D, tiles, w.max_tiles, t(0, 0), t(0, 1), nullptr, I, I, st, ntd, t(1, 0),
+                             t(1, 1), nullptr, gb, few_rows);
       mark(3);
-      k::mx_grouped_gemm_rows(w.hh, nullptr, I, tiles, w.max_tiles, t(2, 0), t(2, 1), w.pair_out, D, D, st, ntd);
+      k::launch_mx_gemm_rows(w.hh, nullptr, I, tiles, w.max_tiles, t(2, 0), t(2, 1), w.pair_out, D, D, st, ntd, nullptr,
+                             nullptr, nullptr, k::MxGlu{}, few_rows);
     } else {
       // Each token row quantized once (its K picks would otherwise be quantized K times); the GEMM's loads gather
       // the pair rows' codes through eidx.
       k::mx_xform_in_fp8(x, D, nullptr, nullptr, w.xq, w.xs, T, D, st, nullptr);
       mark(2);
       k::mx_grouped_gemm_q(w.xq, w.xs, D, tiles, w.max_tiles, t(0, 0), t(0, 1), nullptr, I, I, st, ntd, t(1, 0), t(1, 1),
-                           nullptr, w.tile_rows, glu, w.eidx);
+                           nullptr, tile_rows, glu, w.eidx);
       mark(3);
       k::mx_grouped_gemm_q(w.hq, w.hs, I, tiles, w.max_tiles, t(2, 0), t(2, 1), w.pair_out, D, D, st, ntd, nullptr,
-                           nullptr, nullptr, w.tile_rows);
+                           nullptr, nullptr, tile_rows);
     }
     mark(4);
     k::moe_combine(w.pair_out, w.pidx, nullptr, out, T, K, D, st);

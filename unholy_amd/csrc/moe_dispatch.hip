@@ -118,13 +118,12 @@ __global__ __launch_bounds__(PLAN_NT) void moe_plan_kernel(int32_t* count, const
 // selection order). A thread per token, SC_NT tokens per pass (one block scan); the next pass's picks are loaded
 // before this pass's scan, so their latency overlaps it.
 constexpr int SC_NT = 1024;
-__global__ __launch_bounds__(SC_NT) void moe_scatter_kernel(const int32_t* __restrict__ sel, const float* __restrict__ wt,
-                                                            int T, int K, const int32_t* __restrict__ off,
-                                                            int32_t* eidx, float* ewt, int32_t* row_expert,
-                                                            int32_t* pidx) {
-  __shared__ int lds[SC_NT / 64 + 1];
-  const int e = blockIdx.x;
-  int run = 0, base_row = -1;
+// base_row < 0: read from *off once a pick needs it (an expert without picks never reads it).
+__device__ __forceinline__ void scatter_expert(const int32_t* __restrict__ sel, const float* __restrict__ wt, int T,
+                                               int K, int e, int base_row, int32_t* eidx, float* ewt,
+                                               int32_t* row_expert, int32_t* pidx, int* lds,
+                                               const int32_t* off = nullptr) {
+  int run = 0;
   int cur[kMaxK], nxt[kMaxK];
   const auto load = [&](int t, int (&v)[kMaxK]) {
 #pragma unroll
@@ -143,7 +142,7 @@ __global__ __launch_bounds__(SC_NT) void moe_scatter_kernel(const int32_t* __res
     int tot;
     const int pre = block_exclusive_scan<SC_NT>(c, &tot, lds);
     if (c) {
-      if (base_row < 0) base_row = off[e];
+      if (base_row < 0) base_row = *off;
       int d = 0;
 #pragma unroll
       for (int j = 0; j < kMaxK; ++j)
@@ -160,6 +159,65 @@ __global__ __launch_bounds__(SC_NT) void moe_scatter_kernel(const int32_t* __res
 #pragma unroll
     for (int j = 0; j < kMaxK; ++j) cur[j] = nxt[j];
   }
+}
+__global__ __launch_bounds__(SC_NT) void moe_scatter_kernel(const int32_t* __restrict__ sel, const float* __restrict__ wt,
+                                                            int T, int K, const int32_t* __restrict__ off,
+                                                            int32_t* eidx, float* ewt, int32_t* row_expert,
+                                                            int32_t* pidx) {
+  __shared__ int lds[SC_NT / 64 + 1];
+  scatter_expert(sel, wt, T, K, blockIdx.x, -1, eidx, ewt, row_expert, pidx, lds, off + blockIdx.x);
+}
+
+// moe_count + moe_plan + moe_scatter in one launch, every expert resident (the forward's steps past one block of
+// picks). Block e counts all picks per expert in LDS (every block repeats the counting: sel is read from L2, and that
+// costs less than the three launches that would share one count: 203 tokens 15 us as four launches, count clearing
+// included), takes its own first row as the sum of the counts below e, then scatters its picks as
+// moe_scatter_kernel does. The tiles are written longest first (full tiles in expert order, then the remainders by
+// falling row count, ties to the lower expert): a GEMM's workgroups start in tile order, so its last round is of
+// short tiles. The order of tiles decides no result.
+struct DispatchAllArgs {
+  const int32_t* sel;
+  const float* wt;
+  int T, K, E, max_tiles, tile_rows;
+  MoePlan* plan;
+  Exl3Tile* tiles;
+  int32_t* eidx;
+  float* ewt;
+  int32_t *row_expert, *pidx;
+};
+__global__ __launch_bounds__(SC_NT) void moe_dispatch_all_kernel(DispatchAllArgs a) {
+  __shared__ int bins[1024], lds[SC_NT / 64 + 1], part[5][SC_NT / 64];
+  const int e = blockIdx.x, tid = threadIdx.x, E = a.E, T = a.T, K = a.K, n = T * K;
+  for (int i = tid; i < E; i += SC_NT) bins[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < n; i += SC_NT) atomicAdd(&bins[a.sel[i]], 1);
+  __syncthreads();
+  // Thread i stands for expert i (E <= SC_NT). Sums over the experts: rows and full tiles below e, full tiles in all,
+  // remainder tiles ahead of e's, remainder tiles in all.
+  const int own = bins[e], rem = own % a.tile_rows;
+  const int c = tid < E ? bins[tid] : 0, f = c / a.tile_rows, r = c % a.tile_rows;
+  int v[5] = {tid < e ? c : 0, tid < e ? f : 0, f, (r > rem || (r == rem && tid < e)) && r ? 1 : 0, r ? 1 : 0};
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
+    if ((tid & 63) == 0) part[q][tid >> 6] = v[q];
+  }
+  __syncthreads();
+  int sum[5];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+    sum[q] = 0;
+    for (int w = 0; w < SC_NT / 64; ++w) sum[q] += part[q][w];
+  }
+  const int row0 = sum[0], full = own / a.tile_rows;
+  for (int i = tid; i < full; i += SC_NT)
+    if (sum[1] + i < a.max_tiles) a.tiles[sum[1] + i] = Exl3Tile{e, row0 + i * a.tile_rows, a.tile_rows};
+  if (tid == 0 && rem && sum[2] + sum[3] < a.max_tiles)
+    a.tiles[sum[2] + sum[3]] = Exl3Tile{e, row0 + full * a.tile_rows, rem};
+  if (e == 0 && tid == 0) *a.plan = MoePlan{n, n, min(sum[2] + sum[4], a.max_tiles), 0, 0};
+  if (!own) return;  // uniform
+  scatter_expert(a.sel, a.wt, T, K, e, row0, a.eidx, a.ewt, a.row_expert, a.pidx, lds);
 }
 
 // ---- routers: a wave per token ---------------------------------------------------------------------------------------
@@ -259,7 +317,7 @@ __device__ __forceinline__ void route_wave(const float* lr, const float* bias, c
 }
 
 // mode 0: DSV4 (sqrt-softplus + bias, hash tid2eid, bias_vl for image ids), 1: GLM sigmoid, 2: softmax top-K.
-template <int MODE>
+template <int MODE, int NV>
 __global__ __launch_bounds__(256) void route_wave_kernel(const float* __restrict__ logits, const float* bias0,
                                                          const int32_t* tid2eid0, const int32_t* ids, int32_t* sel,
                                                          float* weights, int T, int E, int K, float route_scale,
@@ -269,8 +327,43 @@ __global__ __launch_bounds__(256) void route_wave_kernel(const float* __restrict
   const bool image = MODE == 0 && bias_vl && ids[t] >= vocab;
   const float* bias = image ? bias_vl : bias0;
   const int32_t* hash_row = MODE == 0 && !image && tid2eid0 ? tid2eid0 + size_t(ids[t]) * K : nullptr;
-  route_wave<MODE, 16>(logits + size_t(t) * E, bias, hash_row, E, K, route_scale, sel + size_t(t) * K,
+  route_wave<MODE, NV>(logits + size_t(t) * E, bias, hash_row, E, K, route_scale, sel + size_t(t) * K,
                        weights + size_t(t) * K, nullptr, nullptr);
+}
+
+// Softmax routing and the forward's input transform (each token row fake-quantized to bf16, mx_xform_in) in one
+// launch: neither reads the other's output. Blocks below rblocks route 4 tokens each, the others quantize 8 values per
+// thread, 16 consecutive threads one 128-block.
+template <int NV>
+__global__ __launch_bounds__(256) void route_xform_kernel(const float* __restrict__ logits, int32_t* sel,
+                                                          float* weights, int T, int E, int K, int rblocks,
+                                                          const bf16* __restrict__ x, bf16* __restrict__ xa, int D) {
+  if (int(blockIdx.x) < rblocks) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t < T)
+      route_wave<2, NV>(logits + size_t(t) * E, nullptr, nullptr, E, K, 1.0f, sel + size_t(t) * K,
+                        weights + size_t(t) * K, nullptr, nullptr);
+    return;
+  }
+  const size_t items = size_t(T) * (D / 8), step = size_t(gridDim.x - rblocks) * 256;
+  for (size_t base = size_t(blockIdx.x - rblocks) * 256; base < items; base += step) {  // uniform: whole 16-lane groups
+    const size_t it = min(base + threadIdx.x, items - 1);
+    const uint4 raw = *reinterpret_cast<const uint4*>(x + it * 8);
+    const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
+    float v[8], am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(rw[i] << 16);
+      v[2 * i + 1] = __uint_as_float(rw[i] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(v[i]));
+    const Fp8Block b = fp8_block_scale(row16_max(am));
+    if (base + threadIdx.x >= items) continue;
+    uint32_t c[2];
+    fp8_codes8(v, b, c[0], c[1]);
+    *reinterpret_cast<uint4*>(xa + it * 8) = __builtin_bit_cast(uint4, fp8x8_to_bf16(c[0], c[1], b.sc));
+  }
 }
 
 // The reference's one-thread-per-token DSV4 router (ref_moe.hip:14-60): the same picks and weights as the wave
@@ -975,13 +1068,26 @@ void moe_scatter(const int32_t* sel, const float* wt, int T, int K, const int32_
   moe_scatter_e(sel, wt, T, K, PLAN_NT, off, eidx, ewt, row_expert, pidx, st);
 }
 
-__global__ void zero_words_kernel(int32_t* p, size_t n) {
-  for (size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x) p[i] = 0;
+void launch_moe_dispatch_all(const int32_t* sel, const float* wt, int T, int K, int E, MoePlan* plan, Exl3Tile* tiles,
+                             int max_tiles, int tile_rows, int32_t* eidx, float* ewt, int32_t* row_expert,
+                             int32_t* pidx, hipStream_t st) {
+  if (T <= 0) return;
+  if (E <= 0 || E > SC_NT) throw std::runtime_error("moe_plan: E must be in [1, 1024]");
+  if (tile_rows <= 0 || tile_rows > kExl3TileRows) throw std::runtime_error("moe_plan: tile_rows in [1, 128]");
+  if (K <= 0 || K > kMaxK) throw std::runtime_error("moe_scatter: K in [1, 8], E > 0");
+  moe_dispatch_all_kernel<<<unsigned(E), SC_NT, 0, st>>>(
+      DispatchAllArgs{sel, wt, T, K, E, max_tiles, tile_rows, plan, tiles, eidx, ewt, row_expert, pidx});
+  UH_CHECK_LAUNCH();
 }
 
-void launch_zero_words(int32_t* p, size_t n, hipStream_t st) {
-  if (!n) return;
-  zero_words_kernel<<<unsigned(std::min<size_t>(cdiv(n, 256), 1024)), 256, 0, st>>>(p, n);
+void launch_route_xform(const float* logits, int32_t* sel, float* weights, int T, int E, int K, const bf16* x, bf16* xa,
+                        int D, hipStream_t st) {
+  if (T <= 0) return;
+  if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_softmax: E <= 1024, K in [1, 8]");
+  if (D % 128) throw std::runtime_error("mx transform: K % 128");
+  const unsigned rb = cdiv(size_t(T), 4), xb = unsigned(std::min<size_t>(cdiv(size_t(T) * (D / 8), 256), 8192));
+  auto* kern = E <= 256 ? &route_xform_kernel<4> : &route_xform_kernel<16>;
+  kern<<<rb + xb, 256, 0, st>>>(logits, sel, weights, T, E, K, int(rb), x, xa, D);
   UH_CHECK_LAUNCH();
 }
 
@@ -1140,7 +1246,7 @@ void route_fast(const float* logits, const float* bias, const int32_t* tid2eid, 
                 int vocab) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_fast: E <= 1024, K in [1, 8]");
-  route_wave_kernel<0><<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, tid2eid, ids, sel, weights, T, E, K,
+  (E <= 256 ? &route_wave_kernel<0, 4> : &route_wave_kernel<0, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, tid2eid, ids, sel, weights, T, E, K,
                                                             route_scale, bias_vl, vocab);
   UH_CHECK_LAUNCH();
 }
@@ -1148,14 +1254,14 @@ void route_glm(const float* logits, const float* bias, int32_t* sel, float* weig
                float route_scale, hipStream_t st) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_glm: E <= 1024, K in [1, 8]");
-  route_wave_kernel<1><<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, nullptr, nullptr, sel, weights, T, E, K,
+  (E <= 256 ? &route_wave_kernel<1, 4> : &route_wave_kernel<1, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, nullptr, nullptr, sel, weights, T, E, K,
                                                             route_scale, nullptr, 0);
   UH_CHECK_LAUNCH();
 }
 void route_softmax(const float* logits, int32_t* sel, float* weights, int T, int E, int K, hipStream_t st) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_softmax: E <= 1024, K in [1, 8]");
-  route_wave_kernel<2><<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, nullptr, nullptr, nullptr, sel, weights, T, E, K,
+  (E <= 256 ? &route_wave_kernel<2, 4> : &route_wave_kernel<2, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, nullptr, nullptr, nullptr, sel, weights, T, E, K,
                                                             1.0f, nullptr, 0);
   UH_CHECK_LAUNCH();
 }

@@ -359,8 +359,8 @@ static_assert(GP_C1 <= GP_RING, "the bf16 C tile reuses the ring");
 constexpr int GP_ROWS = 1024;  // the SwiGLU epilogue's per-row weights and flags, after the C tiles
 
 // The bf16 / fp32 / SwiGLU epilogue of the pipelined kernels. each(f) calls f(row, column within the wave's 64, value)
-// for every accumulator element; the ring is reused as the C tile.
-template <int NP, class Each>
+// for every accumulator element; the ring is reused as the C tile (of ROWS rows).
+template <int NP, int ROWS = 128, class Each>
 __device__ __forceinline__ void gp_epilogue(const MxGemvArgs& a, uint8_t* smem, int M, size_t row0, int bx, int cq,
                                             int tid, const Each& each) {
   const int N = a.N, q_own = cq >> 1;
@@ -403,10 +403,10 @@ __device__ __forceinline__ void gp_epilogue(const MxGemvArgs& a, uint8_t* smem, 
     // Each row's routing weight and whether its expert's w2 is here, loaded once per row (threads 0..127) into LDS
     // beside the tiles, so that the loop below has no dependent global loads.
     uint16_t* const tg = reinterpret_cast<uint16_t*>(smem);
-    uint16_t* const tu = tg + 128 * GP_LDC2;
+    uint16_t* const tu = tg + ROWS * GP_LDC2;
     uint16_t* const mine = q_own ? tu : tg;
-    float* const rw_lds = reinterpret_cast<float*>(smem + GP_C2);
-    int* const live_lds = reinterpret_cast<int*>(smem + GP_C2 + 512);
+    float* const rw_lds = reinterpret_cast<float*>(smem + 2 * ROWS * GP_LDC2 * 2);
+    int* const live_lds = reinterpret_cast<int*>(rw_lds + 128);
     float rw_t = 0.0f;
     int live_t = 1;
     if (tid < M) {
@@ -672,21 +672,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 // more stages.
 constexpr int kSkinnyMaxRows = 64;  // mx_grouped_gemm's max_rows bound for the GEMV route
 constexpr int GB_KS = 64, GB_B = 8 * 1024, GB_BS = 512;
-constexpr int GB_RING = 3 * (16 * 1024 + GB_B + GB_BS);  // 73.5 KB: two workgroups per CU
+// MRB: the most 16-row blocks a workgroup takes at a time, 8 or 4 (a longer tile is done in groups of 16 MRB rows, each
+// streaming the weights again). 8: two workgroups per CU; 4: half the accumulators, so three, whose barriers and
+// operand waits overlap better while a stage holds few MFMAs. Whole forward at E = 256, D = 4096, I = 2048, 4 against 8
+// (us): T = 65 333 / 347, 128 419 / 433, 203 472 / 488, 400 556 / 570, 500 581 / 585, 700 656 / 642, 1000 742 / 722.
+constexpr int gb_ring(int mrb) { return mrb == 8 ? 3 * (16 * 1024 + GB_B + GB_BS) : 50 * 1024; }
+constexpr int gb_wgs(int mrb) { return mrb == 8 ? 2 : 3; }
 
 // The ring of a tile of RB live 16-row blocks: NA activation loads per wave and stage, S slots (S - 1 stages in
 // flight). Every wave issues NA A, 2 B and 1 scale load per stage.
-template <int RB>
+template <int RB, int MRB>
 struct GbRing {
   static constexpr int NA = (RB + 1) / 2, A = NA * 4096, STAGE = A + GB_B + GB_BS;
-  static constexpr int S = GB_RING / STAGE, NL = NA + 3;
+  static constexpr int S = gb_ring(MRB) / STAGE, NL = NA + 3, ROWS = 16 * MRB;
   static_assert(S >= 3 && (S - 2) * NL < 64);
+  static_assert(ROWS * GP_LDC1 * 2 <= gb_ring(MRB) && 2 * ROWS * GP_LDC2 * 2 + GP_ROWS <= gb_ring(MRB) &&
+                    gb_wgs(MRB) * gb_ring(MRB) <= 160 * 1024,
+                "the C tiles reuse the ring");
 };
-static_assert(GP_C1 <= GB_RING && GP_C2 + GP_ROWS <= GB_RING && 64 * (256 + 4) * 4 <= GB_RING,
-              "the C tiles reuse the ring");
 
-template <int NP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mx_gemm_pipe_bf16_kernel(MxGemvArgs a) {
+template <int NP, int MRB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gb_wgs(MRB)))) void mx_gemm_pipe_bf16_kernel(
+    MxGemvArgs a) {
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
   tile_block(gridDim.x, bx, by);
@@ -716,14 +723,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   const size_t cslab = size_t(ntn) * 512, sslab = size_t(ntn) * 32;
   const uint32_t lds0 = lds_addr(smem);
 
-  for (int rg = 0; rg < tile.rows; rg += 128) {
-    const int M = min(128, tile.rows - rg);
+  for (int rg = 0; rg < tile.rows; rg += 16 * MRB) {
+    const int M = min(16 * MRB, tile.rows - rg);
     const size_t row0 = size_t(tile.row0) + rg;
     __syncthreads();  // the previous row group's LDS use is over
 
     const auto tile_body = [&](auto nrb) {
       constexpr int RB = decltype(nrb)::value;
-      using T = GbRing<RB>;
+      using T = GbRing<RB, MRB>;
       constexpr int NA = T::NA, S = T::S, NL = T::NL;
       // Opaque per body, so that the lane addresses of the eight bodies are not all formed (and spilled) ahead of them.
       int tid = threadIdx.x;
@@ -808,7 +815,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             for (int cb = 0; cb < 4; ++cb) acc[rb][cb] = mfma_bf16(af[b][rb], bf[cb], acc[rb][cb]);
         }
       }
-      gp_epilogue<NP>(a, smem, M, row0, bx, cq, tid, [&](const auto& f) {
+      gp_epilogue<NP, 16 * MRB>(a, smem, M, row0, bx, cq, tid, [&](const auto& f) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -819,14 +826,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     };
     {
       const int rb16 = __builtin_amdgcn_readfirstlane((M + 15) / 16);
-      if (rb16 == 8) tile_body(std::integral_constant<int, 8>{});
-      else if (rb16 == 7) tile_body(std::integral_constant<int, 7>{});
-      else if (rb16 == 6) tile_body(std::integral_constant<int, 6>{});
-      else if (rb16 == 5) tile_body(std::integral_constant<int, 5>{});
-      else if (rb16 == 4) tile_body(std::integral_constant<int, 4>{});
+      if constexpr (MRB == 8) {
+        if (rb16 == 8) tile_body(std::integral_constant<int, 8>{});
+        else if (rb16 == 7) tile_body(std::integral_constant<int, 7>{});
+        else if (rb16 == 6) tile_body(std::integral_constant<int, 6>{});
+        else if (rb16 == 5) tile_body(std::integral_constant<int, 5>{});
+      }
+      if (rb16 == 4) tile_body(std::integral_constant<int, 4>{});
       else if (rb16 == 3) tile_body(std::integral_constant<int, 3>{});
       else if (rb16 == 2) tile_body(std::integral_constant<int, 2>{});
-      else tile_body(std::integral_constant<int, 1>{});
+      else if (rb16 == 1) tile_body(std::integral_constant<int, 1>{});
     }
   }
 }
@@ -843,10 +852,10 @@ void launch_pipe_t(const MxGemvArgs& a, int ntiles, hipStream_t st) {
   UH_CHECK_LAUNCH();
 }
 
-template <int NP>
+template <int NP, int MRB>
 void launch_pipe_bf16_t(const MxGemvArgs& a, int ntiles, hipStream_t st) {
-  const size_t lds = GB_RING;
-  auto* kern = &mx_gemm_pipe_bf16_kernel<NP>;
+  const size_t lds = gb_ring(MRB);
+  auto* kern = &mx_gemm_pipe_bf16_kernel<NP, MRB>;
   UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(lds)));
   MxGemvArgs b = a;
@@ -870,12 +879,12 @@ void launch_gemm_t(const MxGemvArgs& a, int ntiles, hipStream_t st) {
 }  // namespace
 
 // UH_GEMM_PIPE=0 selects the register-staged kernel for fp8 codes too (comparison runs).
-static bool pipe_disabled() {
-  static const bool off = [] {
+bool mx_gemm_pipe_on() {
+  static const bool on = [] {
     const char* e = std::getenv("UH_GEMM_PIPE");
-    return e && e[0] == '0';
+    return !(e && e[0] == '0');
   }();
-  return off;
+  return on;
 }
 
 
@@ -883,7 +892,7 @@ void launch_mx_gemm(const MxGemvArgs& a, int ntiles, int amode, hipStream_t st) 
   if (ntiles <= 0) return;
   // bf16 activation rows (amode 1) take the 64-input-stage pipelined kernel: K % 64 as the reference asks
   // (mx_moe.hip:1045); the other kernels stage 128 inputs at a time.
-  const bool pipe16 = amode == 1 && !pipe_disabled() && a.N % 128 == 0 && a.K % GB_KS == 0 && !a.out32;
+  const bool pipe16 = amode == 1 && mx_gemm_pipe_on() && a.N % 128 == 0 && a.K % GB_KS == 0 && !a.out32;
   if (a.K <= 0 || a.N <= 0 || a.N % 128 || (!pipe16 && a.K % GM_KS))
     throw std::runtime_error("mx_grouped_gemm: K % 128 (K % 64 for bf16 rows) or N % 128");
   const bool np2 = a.w_tab[1] != nullptr, glu = a.hh || a.hq;
@@ -911,12 +920,17 @@ void launch_mx_gemm(const MxGemvArgs& a, int ntiles, int amode, hipStream_t st) 
   (amode == 2   ? launch_gemm_t<NP, 2>(a, ntiles, st)                   \
    : amode == 1 ? launch_gemm_t<NP, 1>(a, ntiles, st)                   \
                 : launch_gemm_t<NP, 0>(a, ntiles, st))
-  const bool pipe = amode == 0 && a.K / GM_KS <= GP_MAX_KS && !pipe_disabled();
+  const bool pipe = amode == 0 && a.K / GM_KS <= GP_MAX_KS && mx_gemm_pipe_on();
   if (amode == 0 && a.x_rows && (!pipe || (!glu && a.N % 256)))
     throw std::runtime_error("mx_grouped_gemm_q: x_rows needs the pipelined kernel (K <= 14336, N % 256 without glu)");
   if (pipe16) {
-    if (glu) launch_pipe_bf16_t<2>(a, ntiles, st);
-    else launch_pipe_bf16_t<1>(a, ntiles, st);
+    if (a.few_rows) {
+      if (glu) launch_pipe_bf16_t<2, 4>(a, ntiles, st);
+      else launch_pipe_bf16_t<1, 4>(a, ntiles, st);
+      return;
+    }
+    if (glu) launch_pipe_bf16_t<2, 8>(a, ntiles, st);
+    else launch_pipe_bf16_t<1, 8>(a, ntiles, st);
   } else if (glu) {
     if (pipe) launch_pipe_t<2>(a, ntiles, st);
     else UH_GM(2);
@@ -1036,16 +1050,24 @@ void mx_grouped_gemm_x(const bf16* x, int ldx, const int32_t* x_rows, int K, con
   launch_mx_gemm(a, ntiles, 2, st);
 }
 
+void launch_mx_gemm_rows(const bf16* xa, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
+                         const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
+                         hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
+                         const uint8_t* const* s_tab2, bf16* out2, const MxGlu& glu, bool few_rows) {
+  MxGemvArgs a = gemm_args(xa, nullptr, nullptr, K, tiles, w_tab, s_tab, out, ldo, N, ntiles_dev, w_tab2, s_tab2, out2,
+                           glu);
+  a.x_rows = x_rows;
+  a.few_rows = few_rows;
+  if (x_rows && (!mx_gemm_pipe_on() || K % GB_KS || N % 128))
+    throw std::runtime_error("mx_grouped_gemm_rows: x_rows needs the pipelined kernel (K % 64, N % 128)");
+  launch_mx_gemm(a, ntiles, 1, st);
+}
 void mx_grouped_gemm_rows(const bf16* xa, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
                           const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
                           hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
                           const uint8_t* const* s_tab2, bf16* out2, const MxGlu& glu) {
-  MxGemvArgs a = gemm_args(xa, nullptr, nullptr, K, tiles, w_tab, s_tab, out, ldo, N, ntiles_dev, w_tab2, s_tab2, out2,
-                           glu);
-  a.x_rows = x_rows;
-  if (x_rows && (pipe_disabled() || K % GB_KS || N % 128))
-    throw std::runtime_error("mx_grouped_gemm_rows: x_rows needs the pipelined kernel (K % 64, N % 128)");
-  launch_mx_gemm(a, ntiles, 1, st);
+  launch_mx_gemm_rows(xa, x_rows, K, tiles, ntiles, w_tab, s_tab, out, ldo, N, st, ntiles_dev, w_tab2, s_tab2, out2,
+                      glu, false);
 }
 
 void mx_grouped_gemm_glu(const bf16* xa, int K, const Exl3Tile* tiles, int ntiles, const uint8_t* const* w1_tab,

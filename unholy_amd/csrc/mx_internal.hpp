@@ -37,6 +37,7 @@ struct MxGemvArgs {
   // > 0: one matrix, two column streams per wave: projection 1 is projection 0's matrix from 16-column tile `split`
   // on (codes, scales and outputs offset by split tiles); the grid covers split tiles.
   int split;
+  bool few_rows = false;  // GEMM on bf16 rows: most tiles hold at most 64 rows (a choice of kernel, not a bound)
 };
 
 // amode: 0 e4m3 codes + scales, 1 fake-quantized bf16 rows, 2 raw bf16 token rows (act_quant in the kernel).
@@ -47,13 +48,25 @@ unsigned long long fp8_check_encode(unsigned long long* total);
 // Exhaustive check of the hardware bf16 rounding against f32_to_bf16 over all fp32 bit patterns; returns the
 // mismatches at non-NaN inputs (*nan_bad: at NaN inputs).
 unsigned long long bf16_check_encode(unsigned long long* nan_bad);
-// Zeroes n int32 words (a kernel, so that a captured graph records no memset node).
-void launch_zero_words(int32_t* p, size_t n, hipStream_t st);
 struct MoePlan;
+// moe_count + moe_plan + moe_scatter of a step whose experts are all resident, in one launch; the tiles longest first.
+void launch_moe_dispatch_all(const int32_t* sel, const float* wt, int T, int K, int E, MoePlan* plan, Exl3Tile* tiles,
+                             int max_tiles, int tile_rows, int32_t* eidx, float* ewt, int32_t* row_expert,
+                             int32_t* pidx, hipStream_t st);
+// route_softmax and mx_xform_in of the token rows x [T, D] (fake-quantized into xa) in one launch.
+void launch_route_xform(const float* logits, int32_t* sel, float* weights, int T, int E, int K, const uint16_t* x,
+                        uint16_t* xa, int D, hipStream_t st);
 // remote_combine over rows of stride ld (the grid strides over the device-side token count; max_tokens only sizes it).
 void launch_remote_combine(const uint16_t* pair_out, int ld, const int32_t* u2p, const MoePlan* plan, uint16_t* dst,
                            int K, int dim, int max_tokens, hipStream_t st);
 void launch_mx_gemm(const MxGemvArgs& a, int ntiles, int amode, hipStream_t st);
+// mx_grouped_gemm_rows with MxGemvArgs::few_rows; the pipelined GEMMs (UH_GEMM_PIPE) are on.
+struct MxGlu;
+void launch_mx_gemm_rows(const uint16_t* xa, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
+                         const uint8_t* const* w_tab, const uint8_t* const* s_tab, uint16_t* out, int ldo, int N,
+                         hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
+                         const uint8_t* const* s_tab2, uint16_t* out2, const MxGlu& glu, bool few_rows);
+bool mx_gemm_pipe_on();
 void launch_mx_transform(int mode, const uint16_t* x, int ldx, const int32_t* x_rows, const uint16_t* u,
                          const float* w, float limit, const int32_t* row_expert, const uint8_t* const* s_tab,
                          uint16_t* out, uint8_t* q, uint8_t* qs, int K, int P, hipStream_t st);
