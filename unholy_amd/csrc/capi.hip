@@ -124,14 +124,15 @@ MoeWs carve(char* base, int T, int K, int E, int D, int I) {
   w.sel = reinterpret_cast<int32_t*>(take(P * 4));
   w.ewt = reinterpret_cast<float*>(take(P * 4));
   w.wt = reinterpret_cast<float*>(take(P * 4));
-  w.xq = reinterpret_cast<uint8_t*>(take(P * D));
+  // also the bf16 rows xa of a GEMM step (with one pick per token they are the larger)
+  w.xq = reinterpret_cast<uint8_t*>(take(T > 64 ? std::max(P * D, size_t(T) * D * 2) : P * D));
   w.h = reinterpret_cast<bf16*>(w.xq);
   if (size_t(D) < size_t(I) * 2) w.h = reinterpret_cast<bf16*>(take(P * I * 2));
   w.xs = reinterpret_cast<uint8_t*>(take(P * (D / 128)));
   w.hq = reinterpret_cast<uint8_t*>(take(P * I));
   w.hs = reinterpret_cast<uint8_t*>(take(P * (I / 128)));
   char* const codes_end = base ? base + o : nullptr;  // xq, xs, hq and hs lie one after another
-  w.xa = reinterpret_cast<bf16*>(w.xq);  // T * D * 2 <= P * D
+  w.xa = reinterpret_cast<bf16*>(w.xq);
   if (T > 64) {
     w.hh = reinterpret_cast<bf16*>(take(P * I * 2));
   } else if (base) {  // behind xa, in the bytes that only the fp8-code GEMMs use (K = 6, I = D / 2: room for it)
