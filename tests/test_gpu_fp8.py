@@ -209,3 +209,29 @@ def test_fp8_gemm_refuses_narrow_ldc():
     c = DeviceBuffer(M * N * 2)
     with pytest.raises(Exception, match="ldc < N"):
         call("uh_gemm_fp8_f32s", q, sa, w, sw, c, N - 32, M, N, K, None)
+
+
+# The K-part kernel's forms (2 x 1 .. 6 x 4 row x column blocks of 16): row and column remainders, fewer 128-blocks than
+# waves, uneven parts, two sets of scales (K > 4096); and the tiled kernel's block mapping (1, 3, 5, 8 and 9 row tiles).
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("M,N,K", [(17, 48, 128), (33, 80, 1152), (47, 4096, 256), (100, 4096, 256), (250, 4096, 256),
+                                   (300, 4096, 384), (384, 4096, 256), (65, 192, 8192), (18, 32, 5248),
+                                   (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256), (1100, 1024, 256)])
+def test_fp8_mid_sizes(M, N, K, f32):
+    """gemm_w8a8_wmma / gemm_fp8_f32s past 16 rows against the oracle within the bf16 bar, C with a row stride past N
+    and its columns past N untouched."""
+    rng = np.random.default_rng(M + N + K)
+    x = randn_bf16(rng, (M, K))
+    wq, sw = _w8a8_weights(rng, N, K)
+    if f32:
+        q, sa = oracle.act_quant_fp8_f32s(x)
+        sw = (rng.random(sw.shape, np.float32) + 0.5) * np.float32(2.0 ** -6)
+    else:
+        q, sa = oracle.act_quant_fp8(x)
+    ldc = N + 8
+    c = dev(np.full((M, ldc), 0x7FC1, np.uint16))
+    call("uh_gemm_fp8_f32s" if f32 else "uh_gemm_w8a8_wmma", dev(q), dev(sa), dev(wq), dev(sw), c, ldc, M, N, K, None)
+    g = c.download((M, ldc), np.uint16)
+    assert np.all(g[:, N:] == 0x7FC1)
+    ref16, _ = oracle.gemm_w8a8(q, sa, wq, sw)
+    assert max_rel(from_bf16(g[:, :N]), from_bf16(ref16)) <= 1e-2

@@ -39,11 +39,16 @@ void launch_fp8_gemv(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts* parts
 // 16 < M <= 256 with fp32 scales: one workgroup per 32 x 32 output tile over the whole of K (N % 32, K <= 8192).
 bool fp8_rows_fits(const Fp8GemmArgs& a);
 void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st);
-// M > 64: the LDS-ring MFMA GEMM (N % 256, K % 128, ldc % 8; fp8_tiled_fits says whether a shape qualifies).
+// The LDS-ring MFMA GEMM (N % 128, K % 128, ldc % 8; fp8_tiled_fits says whether a shape qualifies).
 bool fp8_tiled_fits(const Fp8GemmArgs& a);
 void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st);
-// Picks the row-tile kernel (fp32 scales, 16 < M <= 256, where it fits), the small-M kernel (M <= 64), the tiled GEMM,
-// or the row-group kernel for shapes the tiled one does not take.
+// 16 < M: a workgroup per output tile of up to 96 x 64, K split over its waves (N % 16, K <= 8192); its estimated time.
+bool fp8_kpart_fits(const Fp8GemmArgs& a);
+double fp8_kpart_us(const Fp8GemmArgs& a);
+void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st);
+double fp8_tiled_us(const Fp8GemmArgs& a);
+// M <= 16: the GEMV; past it the K-part kernel or the tiled GEMM, by their estimated times; where neither fits the row
+// tiles, the GEMV (M <= 64) or the row-group kernel.
 void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st);
 
 }  // namespace unholy::kernels

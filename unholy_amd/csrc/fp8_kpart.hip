@@ -1,0 +1,252 @@
+// Dense fp8 GEMM for 16 < M up to the low thousands: C[M, N] (bf16) = A[M, K] (e4m3) x W[N, K]^T (e4m3), per-128 scales
+// (e8m0 or fp32, as fp8_tiled.hip).
+//
+// What bounds these sizes is getting each CU's share of W and A to it: 4096 x 4096 weights are 64 KB per CU, and a
+// tile of R x C outputs reads (R + C) K bytes, mostly from L2. A grid of about one workgroup per CU therefore wants the
+// largest tile that still makes 256 workgroups, with many bytes in flight and no barrier to wait at.
+// - A workgroup = 8 waves over one tile of 16 RB rows x 16 CB columns; wave w takes the w-th eighth of K's 128-blocks
+//   and computes the whole tile over it. The waves share nothing (each has its own LDS slot and no barrier) until their
+//   partial tiles are added through LDS in wave order.
+// - Operands go through LDS by direct loads of 8 rows x 128 bytes with consecutive lanes along a row. Loads straight
+//   into MFMA operand order (lane l: row l % 16) read at most 9.5 TB/s from L2, whatever is in flight: four
+//   consecutive lanes lie in four rows; with consecutive lanes along a row L2 delivers 25-33 TB/s (a read-only probe,
+//   all CUs). 64 x 4096 x 4096 step 14.2 us with the register loads, 12.1 with these; 300 rows 29 / 21.8.
+// - A lane's 16 bytes of an operand row feed two 16x16x32 bf16 MFMAs as they stand (the same input permutation on
+//   both sides), converted exactly. e8m0 scales are folded into the conversions (exact); with fp32 scales each
+//   block's MFMA chain starts from zero and is folded as acc += raw * (sa * sw).
+// Steps (act_quant + GEMM, us, 4096 x 4096) against the kernels that ran before it: e8m0 M = 32 15.5 -> 11.1, 64 20.0 ->
+// 12.1, 128 38.5 -> 15.2, 256 41.6 -> 19.9, 300 41.3 -> 21.8, 512 42.3 -> 32.0; fp32 M = 64 13.6 -> 11.9, 256 34.6 ->
+// 20.2, 300 43.5 -> 23.3. 32768 x 1024, e8m0, M = 64: 97 -> 19.
+#include <algorithm>
+#include <stdexcept>
+
+#include "common.hpp"
+#include "numerics.hpp"
+#include "fp8_internal.hpp"
+#include "pipe.hpp"
+
+namespace unholy::kernels {
+
+using namespace uh;
+using namespace pipe;
+
+namespace {
+
+constexpr int KP_WAVES = 8;
+constexpr int NSET = 2;  // scale registers per row block: NSET sets of 4 128-input blocks
+
+template <bool F32S, int RB, int CB>
+__global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp8_kpart_kernel(
+    Fp8GemmArgs a, int row_tiles, int tile_rows) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int M = a.M, K = a.K, KS = K / 128;
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Work item = column block x row tiles + row tile; XCD x takes the x-th eighth of the items, so that the row tiles of
+  // a column block share one L2.
+  const int nw = gridDim.x, lin = blockIdx.x;
+  const int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
+  const int row0 = (wi % row_tiles) * tile_rows, col0 = (wi / row_tiles) * (16 * CB);
+  const int Mt = min(tile_rows, M - row0);
+  const int per = (KS + KP_WAVES - 1) / KP_WAVES, b0 = min(KS, wave * per), n = min(KS, b0 + per) - b0;  // blocks
+
+  // Scales of the wave's blocks in registers. Lane group g holds block g (NSET sets of 4): the rows' of row block rb
+  // in lane l16 = row; the weights' (16 CB columns lie in one 128-row weight block) of block l in lane l.
+  float sav[NSET][RB], swv = 0.0f;
+  const auto sa_at = [&](int r, int kb) {
+    const size_t i = size_t(row0 + min(r, Mt - 1)) * KS + min(kb, KS - 1);
+    return F32S ? a.sa32[i] : e8m0_to_f32(a.sa8[i]);
+  };
+#pragma unroll
+  for (int q = 0; q < NSET; ++q)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) sav[q][rb] = q * 4 < per ? sa_at(rb * 16 + l16, b0 + 4 * q + g) : 0.0f;
+  {
+    const size_t i = size_t(col0 / 128) * KS + min(b0 + (lane & 7), KS - 1);
+    swv = F32S ? a.sw32[i] : e8m0_to_f32(a.sw8[i]);
+  }
+
+  // The wave's slot in LDS: one 128-input block, RB row blocks then CB column blocks of 16 rows x 128 bytes. A direct
+  // load covers 8 rows x 128 bytes; the 16-byte piece p of row r sits at p ^ ((r >> 1) & 7).
+  constexpr int SLOT = (RB + CB) * 2048, NL = 2 * (RB + CB);
+  uint8_t* const slot = smem + wave * SLOT;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(slot));
+  uint32_t off[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int r = 8 * i + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
+    off[i] = (i < 2 * RB ? uint32_t(row0 + min(r, Mt - 1)) : uint32_t(col0 + r - 16 * RB)) * uint32_t(K) + uint32_t(p * 16);
+  }
+  const auto issue = [&](int c) {
+    const size_t k = size_t(b0 + c) * 128;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) dma16(i < 2 * RB ? a.a + k : a.w + k, off[i], lds0 + uint32_t(i * 1024));
+  };
+  if (n > 0) issue(0);
+  v4f acc[RB][CB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  // The scales are waited for here, once (with the first block's loads behind them), not in the loop.
+  asm volatile("" : "+v"(swv));
+#pragma unroll
+  for (int q = 0; q < NSET; ++q)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) asm volatile("" : "+v"(sav[q][rb]));
+
+  const uint8_t* const rd = slot + l16 * 128;
+  const int p0 = (g ^ ((l16 >> 1) & 7)) * 16, p1 = ((4 + g) ^ ((l16 >> 1) & 7)) * 16;
+#pragma unroll 1  // run from a cold instruction cache: small beats unrolled
+  for (int c = 0; c < n; ++c) {
+    wait_vm<0>();
+    asm volatile("" ::: "memory");
+    v4i aq[RB][2], bq[CB][2];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      bq[cb][0] = *reinterpret_cast<const v4i*>(rd + (RB + cb) * 2048 + p0);
+      bq[cb][1] = *reinterpret_cast<const v4i*>(rd + (RB + cb) * 2048 + p1);
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      aq[rb][0] = *reinterpret_cast<const v4i*>(rd + rb * 2048 + p0);
+      aq[rb][1] = *reinterpret_cast<const v4i*>(rd + rb * 2048 + p1);
+    }
+    if (c + 1 < n) {  // the next block into the slot as soon as it has been read: in flight under this block's MFMAs
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      issue(c + 1);
+    }
+    const float sw = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(__float_as_uint(swv)), c & 7)));
+    const auto sa_of = [&](int rb, int row) {  // the scale of row `row` of the row block in block c
+      const float v = c >= 4 ? sav[1][rb] : sav[0][rb];
+      return __uint_as_float(uint32_t(__builtin_amdgcn_ds_bpermute(((c & 3) * 16 + row) * 4, int(__float_as_uint(v)))));
+    };
+    bf16x8 bf[CB][4];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        bf[cb][t] = fp8x8_to_bf16(uint32_t(bq[cb][t >> 1][2 * (t & 1)]), uint32_t(bq[cb][t >> 1][2 * (t & 1) + 1]),
+                                  F32S ? 1.0f : sw);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const float asc = F32S ? 1.0f : sa_of(rb, l16);
+      v4f raw[CB];
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) raw[cb] = F32S ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : acc[rb][cb];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bf16x8 af = fp8x8_to_bf16(uint32_t(aq[rb][t >> 1][2 * (t & 1)]),
+                                        uint32_t(aq[rb][t >> 1][2 * (t & 1) + 1]), asc);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) raw[cb] = mfma_bf16(af, bf[cb][t], raw[cb]);
+      }
+      if constexpr (F32S) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float f = sa_of(rb, 4 * g + i) * sw;
+#pragma unroll
+          for (int cb = 0; cb < CB; ++cb) acc[rb][cb][i] += raw[cb][i] * f;
+        }
+      } else {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = raw[cb];
+      }
+    }
+  }
+
+  // The 8 partial tiles added in wave order, PB column blocks at a time (the partials of a pass fit 128 KB of LDS).
+  constexpr int PB = RB * CB <= 16 ? CB : CB / 2, NV = RB * PB;
+  v4f* const red = reinterpret_cast<v4f*>(smem);
+#pragma unroll
+  for (int p = 0; p < CB; p += PB) {
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < PB; ++cb) red[(wave * NV + rb * PB + cb) * 64 + lane] = acc[rb][p + cb];
+    __syncthreads();
+    for (int v = wave; v < NV; v += KP_WAVES) {
+      v4f s = red[v * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < KP_WAVES; ++w) s += red[(w * NV + v) * 64 + lane];
+      const int r = (v / PB) * 16 + 4 * g, col = col0 + (p + v % PB) * 16 + l16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (r + i < Mt) a.c[size_t(row0 + r + i) * a.ldc + col] = f32_to_bf16(s[i]);
+    }
+  }
+}
+
+template <bool F32S, int RB, int CB>
+void launch_t(const Fp8GemmArgs& a, hipStream_t st) {
+  constexpr int NV = RB * (RB * CB <= 16 ? CB : CB / 2);
+  constexpr size_t lds = std::max<size_t>(size_t(KP_WAVES) * NV * 64 * 16, size_t(KP_WAVES) * (RB + CB) * 2048);
+  static_assert(lds <= 160 * 1024);
+  const int rt = (a.M + 16 * RB - 1) / (16 * RB), tile_rows = ((a.M + rt - 1) / rt + 15) / 16 * 16;
+  auto* kern = &fp8_kpart_kernel<F32S, RB, CB>;
+  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               int(lds)));
+  kern<<<dim3(unsigned(a.N / (16 * CB)) * unsigned(rt)), 64 * KP_WAVES, lds, st>>>(a, rt, tile_rows);
+  UH_CHECK_LAUNCH();
+}
+
+}  // namespace
+
+namespace {
+// The forms (16-row blocks x 16-column blocks), and what a launch of each takes (us, 16 < M <= 1024 and the shapes of
+// the model's projections, with act_quant): every round of 256 workgroups reads (RB + CB) rows and columns of K; a round
+// past the first adds its start-up and the reduction, less where two or three workgroups share a CU. 64 x 4096 x 4096
+// (M x N x K) 12.1 measured, 300 x 4096 x 4096 22.2, 512 32.8, 768 46.4, 600 x 4096 x 8192 60, 200 x 8192 x 1024 16.3,
+// 20 x 32768 x 1024 14.2 as 2 x 2 and 17.9 as 4 x 4.
+struct KpForm {
+  int rb, cb;
+  double read, next;  // RB + CB, more where the registers leave less in flight; the cost of a further round
+};
+constexpr KpForm kForms[] = {{2, 1, 3.0, 1.0}, {2, 2, 4.0, 1.2}, {4, 2, 6.0, 3.0},
+                             {4, 4, 9.0, 3.5}, {5, 4, 10.5, 3.5}, {6, 4, 13.0, 3.5}};
+double form_us(const Fp8GemmArgs& a, const KpForm& f) {
+  const size_t wg = size_t((a.M + 16 * f.rb - 1) / (16 * f.rb)) * (a.N / (16 * f.cb));
+  const double rounds = double((wg + 255) / 256);
+  return 7.0 + (rounds - 1.0) * f.next + rounds * f.read * a.K * 0.00034;
+}
+int best_form(const Fp8GemmArgs& a) {
+  const int forms = a.sa32 ? 5 : 6;  // 6 x 4 with fp32 scales spills
+  int best = 0;
+  for (int i = 1; i < forms; ++i)
+    if (a.N % (16 * kForms[i].cb) == 0 && form_us(a, kForms[i]) < form_us(a, kForms[best])) best = i;
+  return best;
+}
+}  // namespace
+
+bool fp8_kpart_fits(const Fp8GemmArgs& a) {
+  return a.M > 16 && a.N > 0 && a.N % 16 == 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET &&
+         (a.sa32 ? a.sw32 != nullptr : a.sa8 && a.sw8) && size_t(a.M) * a.K < (size_t(1) << 32) &&
+         size_t(a.N) * a.K < (size_t(1) << 32);
+}
+double fp8_kpart_us(const Fp8GemmArgs& a) { return form_us(a, kForms[best_form(a)]); }
+
+void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
+  if (!fp8_kpart_fits(a)) throw std::runtime_error("fp8 kpart: shape");
+  if (!a.a || !a.w || !a.c) throw std::runtime_error("fp8 gemm: null operand");
+  if (a.sa32) {
+    switch (best_form(a)) {
+      case 0: return launch_t<true, 2, 1>(a, st);
+      case 1: return launch_t<true, 2, 2>(a, st);
+      case 2: return launch_t<true, 4, 2>(a, st);
+      case 3: return launch_t<true, 4, 4>(a, st);
+      default: return launch_t<true, 5, 4>(a, st);
+    }
+  }
+  switch (best_form(a)) {
+    case 0: return launch_t<false, 2, 1>(a, st);
+    case 1: return launch_t<false, 2, 2>(a, st);
+    case 2: return launch_t<false, 4, 2>(a, st);
+    case 3: return launch_t<false, 4, 4>(a, st);
+    case 4: return launch_t<false, 5, 4>(a, st);
+    default: return launch_t<false, 6, 4>(a, st);
+  }
+}
+
+}  // namespace unholy::kernels

@@ -45,10 +45,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   constexpr int CB = T::CB;
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
-  tile_block(gridDim.x, bx, by);
   const int K = a.K, KS = K / 128, M = a.M;
+  if (!dense_block(a.N / TN, (M + 127) / 128, bx, by)) return;
   const int row0 = by * 128;
-  if (row0 >= M) return;  // padding of the grid's row-tile count
   const int Mt = min(128, M - row0), col0 = bx * TN;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,13 +236,12 @@ void launch_tiled_t(const Fp8GemmArgs& a, hipStream_t st) {
   auto* kern = &fp8_tiled_kernel<F32S, TN>;
   UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(lds)));
-  kern<<<tile_grid(a.N / TN, (a.M + 127) / 128), 256, lds, st>>>(a);
+  kern<<<dense_grid(a.N / TN, (a.M + 127) / 128), 256, lds, st>>>(a);
   UH_CHECK_LAUNCH();
 }
 // 64-column tiles while 128-column ones would leave fewer than 256 workgroups: twice the workgroups on the same
-// serial K loop each. 4096 x 4096 step, 128 / 64 columns: M = 384 55.9 / 52.7 us, 512 56.6 / 53.0, 768 57.4 / 55.6,
-// 1024 (256 workgroups of 128 columns) 61.0 / 60.1, 2048 96.1 / 112.5. (A 4-slot ring of 64-column stages, three in
-// flight, ran 80 us at M = 384-768: not kept.)
+// serial K loop each. 4096 x 4096 step, 128 / 64 columns (measured with one row tile's workgroups on one XCD): M = 384
+// 55.9 / 52.7 us, 512 56.6 / 53.0, 768 57.4 / 55.6, 1024 (256 workgroups of 128 columns) 61.0 / 60.1, 2048 96.1 / 112.5.
 bool tiled_narrow(const Fp8GemmArgs& a) { return size_t(a.N / 128) * ((a.M + 127) / 128) < 256; }
 template <bool F32S>
 void launch_tiled_f(const Fp8GemmArgs& a, hipStream_t st) {
@@ -256,6 +254,19 @@ void launch_tiled_f(const Fp8GemmArgs& a, hipStream_t st) {
 bool fp8_tiled_fits(const Fp8GemmArgs& a) {
   // two workgroups per CU: 80 KB of LDS each
   return a.N % 128 == 0 && a.K % 128 == 0 && a.ldc % 8 == 0 && FpTile<128>::lds(a.K, a.sa32 != nullptr) <= 80 * 1024;
+}
+
+// What a launch takes (us, with act_quant, K = 1024..8192; fp32 scales x 1.07): per 128-input stage 0.82 / 1.06 us (64
+// columns, up to / past 256 workgroups), 1.15 (128 columns, 256 workgroups), 1.75 up to 512, 2.06 per 512 past that.
+// 512 x 4096 x 4096 (M x N x K) 33.9 measured, 768 41.2, 1000 43.7, 1500 64.2, 2000 71.5, 300 x 8192 x 1024 14.8.
+double fp8_tiled_us(const Fp8GemmArgs& a) {
+  const size_t w = size_t(a.N / 128) * ((a.M + 127) / 128);
+  const double stage = w <= 128   ? 0.82
+                       : w < 256  ? 1.06
+                       : w == 256 ? 1.15
+                       : w < 512  ? 1.75
+                                  : 2.06 * double((w + 511) / 512);
+  return 7.0 + a.K / 128 * stage * (a.sa32 ? 1.07 : 1.0);
 }
 
 void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st) {
