@@ -95,3 +95,21 @@ def test_grouped_fp8w_shape_errors():
         call("uh_gemv_grouped_fp8w", da, dw, dsw, c, 33, 2, 128, 256, None, None, None, None)
     call("uh_gemm_grouped_fp8w_wmma", da, dw, dsw, c, 0, 2, 128, 256, None)  # M = 0: nothing to do
 
+
+
+# The K-part kernel's forms (1 x 1 .. 8 x 4 row x column blocks of 16, 128- and 64-input slots) at the sizes that select
+# them: row remainders, R a multiple of 16 or 32 only, one 128-block, uneven K parts, more than eight blocks a wave
+# (K = 9,216); the tiled kernel past it with row tiles that do and do not divide over the XCDs.
+@pytest.mark.parametrize("M,G,R,K", [(9, 8, 512, 256), (16, 8, 1024, 128), (30, 8, 1024, 256), (61, 8, 1024, 384),
+                                     (100, 8, 1024, 128), (180, 8, 1024, 128), (250, 8, 1024, 256), (23, 5, 48, 1152),
+                                     (70, 3, 96, 640), (12, 2, 16, 9216), (600, 8, 1024, 256), (1030, 16, 512, 128),
+                                     (1000, 8, 1024, 128)])
+def test_grouped_fp8w_mid_sizes(M, G, R, K):
+    rng = np.random.default_rng(M * 5 + G * R + K)
+    a, w, sw = _case(rng, M, G, R, K)
+    ref16, _ = oracle.gemm_grouped_fp8w(a, w, sw, G, R)
+    c = dev(np.full((M * G * R + 64,), 0x7FC1, np.uint16))
+    call("uh_gemm_grouped_fp8w_wmma", dev(a), dev(w), dev(sw), c, M, G, R, K, None)
+    got = c.download((M * G * R + 64,), np.uint16)
+    assert np.all(got[M * G * R:] == 0x7FC1)
+    assert max_rel(from_bf16(got[:M * G * R].reshape(M, G, R)), from_bf16(ref16)) <= 1e-2

@@ -47,6 +47,11 @@ bool fp8_kpart_fits(const Fp8GemmArgs& a);
 double fp8_kpart_us(const Fp8GemmArgs& a);
 void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st);
 double fp8_tiled_us(const Fp8GemmArgs& a);
+// The same for the grouped projection (R % 16, K <= 65536).
+bool grouped_kpart_fits(int M, int G, int R, int K);
+double grouped_kpart_us(int M, int G, int R, int K);
+void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
+                          hipStream_t st);
 // M <= 16: the GEMV; past it the K-part kernel or the tiled GEMM, by their estimated times; where neither fits the row
 // tiles, the GEMV (M <= 64) or the row-group kernel.
 void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st);

@@ -35,6 +35,36 @@ namespace {
 constexpr int KP_WAVES = 8;
 constexpr int NSET = 2;  // scale registers per row block: NSET sets of 4 128-input blocks
 
+// The waves' partial tiles added in wave order through LDS (every wave is past its own LDS use after the first barrier),
+// PB column blocks at a time, so that a pass's partials fit 128 KB; store(row, column, sum) of each output.
+template <int RB, int CB>
+constexpr int kp_pass() { return RB * CB <= 16 ? CB : CB / 2; }
+template <int RB, int CB>
+constexpr size_t kp_reduce_lds() { return size_t(KP_WAVES) * RB * kp_pass<RB, CB>() * 64 * 16; }
+template <int RB, int CB, class Store>
+__device__ __forceinline__ void kp_reduce(const v4f (&acc)[RB][CB], uint8_t* smem, const Store& store) {
+  constexpr int PB = kp_pass<RB, CB>(), NV = RB * PB;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  v4f* const red = reinterpret_cast<v4f*>(smem);
+#pragma unroll
+  for (int p = 0; p < CB; p += PB) {
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < PB; ++cb) red[(wave * NV + rb * PB + cb) * 64 + lane] = acc[rb][p + cb];
+    __syncthreads();
+    for (int v = wave; v < NV; v += KP_WAVES) {
+      v4f s = red[v * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < KP_WAVES; ++w) s += red[(w * NV + v) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) store((v / PB) * 16 + 4 * g + i, (p + v % PB) * 16 + l16, s[i]);
+    }
+  }
+}
+
 template <bool F32S, int RB, int CB>
 __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp8_kpart_kernel(
     Fp8GemmArgs a, int row_tiles, int tile_rows) {
@@ -156,39 +186,133 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
     }
   }
 
-  // The 8 partial tiles added in wave order, PB column blocks at a time (the partials of a pass fit 128 KB of LDS).
-  constexpr int PB = RB * CB <= 16 ? CB : CB / 2, NV = RB * PB;
-  v4f* const red = reinterpret_cast<v4f*>(smem);
-#pragma unroll
-  for (int p = 0; p < CB; p += PB) {
-    __syncthreads();
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < PB; ++cb) red[(wave * NV + rb * PB + cb) * 64 + lane] = acc[rb][p + cb];
-    __syncthreads();
-    for (int v = wave; v < NV; v += KP_WAVES) {
-      v4f s = red[v * 64 + lane];
-#pragma unroll
-      for (int w = 1; w < KP_WAVES; ++w) s += red[(w * NV + v) * 64 + lane];
-      const int r = (v / PB) * 16 + 4 * g, col = col0 + (p + v % PB) * 16 + l16;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (r + i < Mt) a.c[size_t(row0 + r + i) * a.ldc + col] = f32_to_bf16(s[i]);
-    }
-  }
+  kp_reduce(acc, smem, [&](int r, int col, float v) {
+    if (r < Mt) a.c[size_t(row0 + r) * a.ldc + col0 + col] = f32_to_bf16(v);
+  });
 }
 
 template <bool F32S, int RB, int CB>
 void launch_t(const Fp8GemmArgs& a, hipStream_t st) {
-  constexpr int NV = RB * (RB * CB <= 16 ? CB : CB / 2);
-  constexpr size_t lds = std::max<size_t>(size_t(KP_WAVES) * NV * 64 * 16, size_t(KP_WAVES) * (RB + CB) * 2048);
+  constexpr size_t lds = std::max<size_t>(kp_reduce_lds<RB, CB>(), size_t(KP_WAVES) * (RB + CB) * 2048);
   static_assert(lds <= 160 * 1024);
   const int rt = (a.M + 16 * RB - 1) / (16 * RB), tile_rows = ((a.M + rt - 1) / rt + 15) / 16 * 16;
   auto* kern = &fp8_kpart_kernel<F32S, RB, CB>;
   UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(lds)));
   kern<<<dim3(unsigned(a.N / (16 * CB)) * unsigned(rt)), 64 * KP_WAVES, lds, st>>>(a, rt, tile_rows);
+  UH_CHECK_LAUNCH();
+}
+
+// The same for the grouped projection c[m][g][r] = sum_k a[m][g][k] w[g R + r][k]: bf16 rows as they are (twice the
+// bytes of the weights' rows), e8m0 weight scales per 128 x 128 folded into the conversions. KB inputs per step and
+// slot: 128 (A 16 rows x 256 bytes, W 16 rows x 128 bytes per block), or 64 for the forms whose 128-input slots do not
+// fit (A 16 x 128, W 16 x 64).
+template <int RB, int CB, int KB>
+struct GKp {
+  static constexpr int AB = 16 * KB * 2, WB = 16 * KB, SLOT = RB * AB + CB * WB, NA = RB * AB / 1024, NW = CB * WB / 1024;
+  static constexpr int AR = 1024 / (2 * KB), WR = 1024 / KB;  // rows per direct load
+  // Piece (16 bytes) p of row r of a block: the 16 rows that an operand read covers touch each LDS bank once.
+  static __device__ __forceinline__ int aswz(int r) { return KB == 128 ? r : (r >> 1) & 7; }
+  static __device__ __forceinline__ int wswz(int r) { return KB == 128 ? (r >> 1) & 7 : (r >> 2) & 3; }
+  static constexpr size_t lds() { return std::max<size_t>(kp_reduce_lds<RB, CB>(), size_t(KP_WAVES) * SLOT); }
+};
+template <int RB, int CB, int KB>
+__global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void grouped_kpart_kernel(
+    const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K, int row_tiles,
+    int tile_rows) {
+  using T = GKp<RB, CB, KB>;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int KS = K / 128, N = G * R;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int nw = gridDim.x, lin = blockIdx.x;
+  const int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
+  const int row0 = (wi % row_tiles) * tile_rows, col0 = (wi / row_tiles) * (16 * CB), grp = col0 / R;  // R % (16 CB) == 0
+  const int Mt = min(tile_rows, M - row0);
+  const int per = (KS + KP_WAVES - 1) / KP_WAVES, b0 = min(KS, wave * per), n = (min(KS, b0 + per) - b0) * (128 / KB);
+  // The scale of the wave's block l in lane l (the host: at most 64 blocks a wave).
+  float swv = e8m0_to_f32(sw[size_t(col0 / 128) * KS + min(b0 + lane, KS - 1)]);
+  uint8_t* const slot = smem + wave * T::SLOT;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(slot));
+  uint32_t aoff[T::NA], woff[T::NW];
+#pragma unroll
+  for (int i = 0; i < T::NA; ++i) {
+    constexpr int PR = 64 / T::AR;  // pieces per row
+    const int r = T::AR * i + lane / PR, p = (lane % PR) ^ T::aswz(r & 15);
+    aoff[i] = (uint32_t(row0 + min(r, Mt - 1)) * uint32_t(G) + uint32_t(grp)) * uint32_t(K) * 2u + uint32_t(p * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < T::NW; ++i) {
+    constexpr int PR = 64 / T::WR;
+    const int r = T::WR * i + lane / PR, p = (lane % PR) ^ T::wswz(r & 15);
+    woff[i] = uint32_t(col0 + r) * uint32_t(K) + uint32_t(p * 16);
+  }
+  const auto issue = [&](int s) {
+    const size_t k = size_t(b0) * 128 + size_t(s) * KB;
+#pragma unroll
+    for (int i = 0; i < T::NW; ++i) dma16(w + k, woff[i], lds0 + uint32_t(RB * T::AB + i * 1024));
+#pragma unroll
+    for (int i = 0; i < T::NA; ++i) dma16(a + k, aoff[i], lds0 + uint32_t(i * 1024));
+  };
+  if (n > 0) issue(0);
+  v4f acc[RB][CB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("" : "+v"(swv));  // waited for here, once, not in the loop
+  constexpr int H = KB / 64;     // 64-input halves: one 16-byte piece of W and two of A per lane
+#pragma unroll 1
+  for (int s = 0; s < n; ++s) {
+    wait_vm<0>();
+    asm volatile("" ::: "memory");
+    v4i wq[CB][H];
+    bf16x8 aq[RB][2 * H];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int x = 0; x < H; ++x)
+        wq[cb][x] = *reinterpret_cast<const v4i*>(slot + RB * T::AB + cb * T::WB + l16 * KB +
+                                                  ((4 * x + g) ^ T::wswz(l16)) * 16);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int t = 0; t < 2 * H; ++t)  // inputs 64 (t / 2) + 16 g + 8 (t % 2) .. + 7, as W's conversion t
+        aq[rb][t] = *reinterpret_cast<const bf16x8*>(slot + rb * T::AB + l16 * KB * 2 +
+                                                     ((8 * (t >> 1) + 2 * g + (t & 1)) ^ T::aswz(l16)) * 16);
+    if (s + 1 < n) {  // the next step into the slot as soon as it has been read
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      issue(s + 1);
+    }
+    const float sc = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(__float_as_uint(swv)), s * KB / 128)));
+#pragma unroll
+    for (int t = 0; t < 2 * H; ++t) {
+      bf16x8 wf[CB];
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+        wf[cb] = fp8x8_to_bf16(uint32_t(wq[cb][t >> 1][2 * (t & 1)]), uint32_t(wq[cb][t >> 1][2 * (t & 1) + 1]), sc);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mfma_bf16(aq[rb][t], wf[cb], acc[rb][cb]);
+    }
+  }
+  kp_reduce(acc, smem, [&](int r, int col, float v) {
+    if (r < Mt) c[size_t(row0 + r) * N + col0 + col] = f32_to_bf16(v);
+  });
+}
+template <int RB, int CB, int KB>
+void launch_g(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
+              hipStream_t st) {
+  constexpr size_t lds = GKp<RB, CB, KB>::lds();
+  static_assert(lds <= 160 * 1024);
+  const int rt = (M + 16 * RB - 1) / (16 * RB), tile_rows = ((M + rt - 1) / rt + 15) / 16 * 16;
+  auto* kern = &grouped_kpart_kernel<RB, CB, KB>;
+  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               int(lds)));
+  kern<<<dim3(unsigned(G * R / (16 * CB)) * unsigned(rt)), 64 * KP_WAVES, lds, st>>>(a, w, sw, c, M, G, R, K, rt,
+                                                                                     tile_rows);
   UH_CHECK_LAUNCH();
 }
 
@@ -246,6 +370,44 @@ void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
     case 3: return launch_t<false, 4, 4>(a, st);
     case 4: return launch_t<false, 5, 4>(a, st);
     default: return launch_t<false, 6, 4>(a, st);
+  }
+}
+
+// ---- grouped ---------------------------------------------------------------------------------------------------------
+namespace {
+// The forms and what a launch takes (us): every round of 256 workgroups reads 16 (2 RB + CB) K bytes a workgroup. G R =
+// 8192, K = 4096: M = 16 10.1 measured (1 x 2), 32 12.9 (2 x 2), 64 14.7 (2 x 4), 128 19.6 (4 x 4), 256 30.9 (8 x 4), 512
+// 54.9 (8 x 4, two rounds).
+constexpr KpForm kGForms[] = {{1, 1, 3.0, 0.0}, {1, 2, 4.0, 0.0},  {2, 2, 6.0, 0.0}, {2, 4, 8.0, 0.0},
+                              {4, 4, 12.0, 0.0}, {6, 4, 16.0, 0.0}, {8, 4, 20.0, 0.0}};
+double gform_us(int M, int N, int K, const KpForm& f) {
+  const size_t wg = size_t((M + 16 * f.rb - 1) / (16 * f.rb)) * (N / (16 * f.cb));
+  return 4.8 + double((wg + 255) / 256) * f.read * K * 0.00032;
+}
+int best_gform(int M, int G, int R, int K) {
+  int best = 0;
+  for (int i = 1; i < 7; ++i)
+    if (R % (16 * kGForms[i].cb) == 0 && gform_us(M, G * R, K, kGForms[i]) < gform_us(M, G * R, K, kGForms[best])) best = i;
+  return best;
+}
+}  // namespace
+
+bool grouped_kpart_fits(int M, int G, int R, int K) {
+  return M > 0 && R > 0 && R % 16 == 0 && K > 0 && K % 128 == 0 && K <= 128 * KP_WAVES * 64 &&
+         size_t(M) * G * K * 2 < (size_t(1) << 32) && size_t(G) * R * K < (size_t(1) << 32);
+}
+double grouped_kpart_us(int M, int G, int R, int K) { return gform_us(M, G * R, K, kGForms[best_gform(M, G, R, K)]); }
+void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
+                          hipStream_t st) {
+  if (!grouped_kpart_fits(M, G, R, K)) throw std::runtime_error("grouped kpart: shape");
+  switch (best_gform(M, G, R, K)) {
+    case 0: return launch_g<1, 1, 128>(a, w, sw, c, M, G, R, K, st);
+    case 1: return launch_g<1, 2, 128>(a, w, sw, c, M, G, R, K, st);
+    case 2: return launch_g<2, 2, 128>(a, w, sw, c, M, G, R, K, st);
+    case 3: return launch_g<2, 4, 128>(a, w, sw, c, M, G, R, K, st);
+    case 4: return launch_g<4, 4, 64>(a, w, sw, c, M, G, R, K, st);
+    case 5: return launch_g<6, 4, 64>(a, w, sw, c, M, G, R, K, st);
+    default: return launch_g<8, 4, 64>(a, w, sw, c, M, G, R, K, st);
   }
 }
 

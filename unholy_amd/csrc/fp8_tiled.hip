@@ -46,7 +46,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
   const int K = a.K, KS = K / 128, M = a.M;
-  if (!dense_block(a.N / TN, (M + 127) / 128, bx, by)) return;
+  const int rt = (M + 127) / 128;
+  if (!dense_block(a.N / TN, rt, rt == 8, bx, by)) return;  // eight row tiles: one per XCD
   const int row0 = by * 128;
   const int Mt = min(128, M - row0), col0 = bx * TN;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;

@@ -28,6 +28,7 @@
 
 #include "common.hpp"
 #include "numerics.hpp"
+#include "fp8_internal.hpp"
 #include "pipe.hpp"
 #include "unholy/kernels/gemm_wmma.hpp"
 #include "unholy/kernels/gemv.hpp"
@@ -365,9 +366,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   using T = GroupedTile<TN>;
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
-  tile_block(gridDim.x, bx, by);
+  // Row tiles on XCDs of their own where they divide evenly (M = 4096, G R = 8192: 259 us against 263).
+  const int rt = (M + 127) / 128;
+  if (!dense_block(G * R / TN, rt, rt % 8 == 0, bx, by)) return;
   const int row0 = by * 128;
-  if (row0 >= M) return;  // padding of the grid's row-tile count
   const int KS = K / 64, N = G * R, Mt = min(128, M - row0), col0 = bx * TN, grp = col0 / R;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -502,7 +504,7 @@ void launch_tiled_t(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c,
   auto* kern = &grouped_fp8w_tiled_kernel<TN>;
   UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(lds)));
-  kern<<<tile_grid(G * R / TN, (M + 127) / 128), 256, lds, st>>>(a, w, sw, c, M, G, R, K);
+  kern<<<dense_grid(G * R / TN, (M + 127) / 128), 256, lds, st>>>(a, w, sw, c, M, G, R, K);
   UH_CHECK_LAUNCH();
 }
 void launch_tiled(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
@@ -513,6 +515,29 @@ void launch_tiled(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, i
     launch_tiled_t<256>(a, w, sw, c, M, G, R, K, st);
   else
     launch_tiled_t<128>(a, w, sw, c, M, G, R, K, st);
+}
+
+// What a tiled launch takes (us, K = 4096, per 64-input stage): 1.13 up to 448 workgroups of 128 columns, 1.27 up to
+// 512, with 256 columns 1.75 up to 384 and 1.96 per 512 past that. G R = 8192: M = 512 78.8 measured, 800 79.6, 1024
+// 88.4, 1500 118, 2000 133.
+double tiled_us(int M, int G, int R, int K) {
+  const size_t rt = size_t(M + 127) / 128, w128 = rt * (size_t(G) * R / 128), w256 = w128 / 2;
+  const double stage = R % 256 == 0 && w256 > 256 ? (w256 <= 384 ? 1.75 : 1.96 * double((w256 + 511) / 512))
+                                                  : (w128 <= 448 ? 1.13 : 1.27 * double((w128 + 511) / 512));
+  return 7.0 + K / 64 * stage;
+}
+// Up to 8 rows the row tiles' 32-column form while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part
+// kernel, 8 9.28 / 9.43, 16 10.9 / 10.1); else the K-part kernel or the tiled GEMM by their estimated times; then the
+// kernels for what neither takes (operands past 4 GiB, R % 16 != 0).
+void launch_fast(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
+                 hipStream_t st) {
+  const bool few = M <= 8 && size_t(G) * R / 32 >= 256 && rows_fits(M, G, R, K), tiled = tiled_fits(G, R, K);
+  if (!few && grouped_kpart_fits(M, G, R, K) && (!tiled || grouped_kpart_us(M, G, R, K) < tiled_us(M, G, R, K)))
+    launch_grouped_kpart(a, w, sw, c, M, G, R, K, st);
+  else if (rows_fits(M, G, R, K)) launch_rows(a, w, sw, c, M, G, R, K, st);
+  else if (gemv_fits(M, R) && !grouped_kpart_fits(M, G, R, K)) launch_gemv(a, w, sw, c, M, G, R, K, st);
+  else if (tiled) launch_tiled(a, w, sw, c, M, G, R, K, st);
+  else launch_ref(a, w, sw, c, M, G, R, K, st);  // shapes the fast kernels do not tile
 }
 
 }  // namespace
@@ -528,10 +553,7 @@ void gemm_grouped_fp8w_wmma(const bf16* a, const uint8_t* w, const uint8_t* sw, 
                             hipStream_t st) {
   check_args("gemm_grouped_fp8w_wmma", a, w, sw, c, M, G, R, K);
   if (M == 0) return;
-  if (rows_fits(M, G, R, K)) launch_rows(a, w, sw, c, M, G, R, K, st);
-  else if (gemv_fits(M, R)) launch_gemv(a, w, sw, c, M, G, R, K, st);
-  else if (tiled_fits(G, R, K)) launch_tiled(a, w, sw, c, M, G, R, K, st);
-  else launch_ref(a, w, sw, c, M, G, R, K, st);  // shapes the fast kernels do not tile (R % 128 != 0)
+  launch_fast(a, w, sw, c, M, G, R, K, st);
 }
 
 void gemv_grouped_fp8w(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
@@ -540,9 +562,7 @@ void gemv_grouped_fp8w(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16*
   if (M > 32) throw std::runtime_error("gemv_grouped_fp8w: M > 32");  // the reference's bound (gemv.hip:653)
   if (gq.q && (!gq.qs || (size_t(G) * R) % 128)) throw std::runtime_error("gemv_grouped_fp8w: quantization shape");
   if (M == 0) return;
-  if (rows_fits(M, G, R, K)) launch_rows(a, w, sw, c, M, G, R, K, st);
-  else if (gemv_fits(M, R)) launch_gemv(a, w, sw, c, M, G, R, K, st);
-  else launch_ref(a, w, sw, c, M, G, R, K, st);
+  launch_fast(a, w, sw, c, M, G, R, K, st);
   // act_quant_fp8 (block 128) of the bf16 outputs, the values the reference's last blocks quantize (a second launch
   // here instead of its per-segment counters, which stay zero).
   if (gq.q) act_quant_fp8(c, G * R, gq.q, gq.qs, M, G * R, 128, st);
