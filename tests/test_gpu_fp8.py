@@ -211,14 +211,16 @@ def test_fp8_gemm_refuses_narrow_ldc():
         call("uh_gemm_fp8_f32s", q, sa, w, sw, c, N - 32, M, N, K, None)
 
 
-# The K-part kernel's forms (2 x 1 .. 6 x 4 row x column blocks of 16): row and column remainders, fewer 128-blocks than
-# waves, uneven parts, two sets of scales (K > 4096); and the tiled kernel's block mapping (1, 3, 5, 8 and 9 row tiles).
+# The K-part kernel's forms (1 x 1 .. 6 x 4 row x column blocks of 16): row and column remainders, fewer 128-blocks than
+# waves, uneven parts, two sets of scales (K > 4096); the tiled kernel's block mapping (1, 3, 5, 8 and 9 row tiles); and
+# K > 8192, which the GEMV takes.
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("M,N,K", [(17, 48, 128), (33, 80, 1152), (47, 4096, 256), (100, 4096, 256), (250, 4096, 256),
                                    (300, 4096, 384), (384, 4096, 256), (65, 192, 8192), (18, 32, 5248),
-                                   (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256), (1100, 1024, 256)])
+                                   (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256), (1100, 1024, 256),
+                                   (1, 200, 640), (16, 48, 8192), (9, 32768, 128), (70, 200, 256), (20, 64, 9216)])
 def test_fp8_mid_sizes(M, N, K, f32):
-    """gemm_w8a8_wmma / gemm_fp8_f32s past 16 rows against the oracle within the bf16 bar, C with a row stride past N
+    """gemm_w8a8_wmma / gemm_fp8_f32s against the oracle within the bf16 bar, C with a row stride past N
     and its columns past N untouched."""
     rng = np.random.default_rng(M + N + K)
     x = randn_bf16(rng, (M, K))
@@ -235,3 +237,23 @@ def test_fp8_mid_sizes(M, N, K, f32):
     assert np.all(g[:, N:] == 0x7FC1)
     ref16, _ = oracle.gemm_w8a8(q, sa, wq, sw)
     assert max_rel(from_bf16(g[:, :N]), from_bf16(ref16)) <= 1e-2
+
+
+@pytest.mark.parametrize("M,K", [(1, 256), (20, 1152), (3, 9216)])
+def test_gemv_w8a8_parts_matches_single_ranges(M, K):
+    """Column ranges (one ragged) of gemv_w8a8_parts bit for bit as gemv_w8a8 on each range: one and two row blocks, uneven
+    K parts, and K > 8192 (the GEMV kernel)."""
+    rng = np.random.default_rng(M + K)
+    Ns = (128, 200)
+    q, sa = oracle.act_quant_fp8(randn_bf16(rng, (M, K)))
+    dq, dsa = dev(q), dev(sa)
+    ws = [tuple(dev(v) for v in _w8a8_weights(rng, n, K)) for n in Ns]
+    outs = [DeviceBuffer(M * n * 2) for n in Ns]
+    wp, sp, cp = (np.array([b.ptr for b in v], np.uint64) for v in ([w for w, _ in ws], [s for _, s in ws], outs))
+    n_a = np.array(Ns, np.int32)
+    call("uh_gemv_w8a8_parts", dq, dsa, wp.ctypes.data, sp.ctypes.data, cp.ctypes.data, n_a.ctypes.data,
+         n_a.ctypes.data, 2, M, K, None)
+    for (w, s), n, o in zip(ws, Ns, outs):
+        single = DeviceBuffer(M * n * 2)
+        call("uh_gemv_w8a8", dq, dsa, w, s, single, n, M, n, K, None)
+        assert np.array_equal(single.download((M, n), np.uint16), o.download((M, n), np.uint16))

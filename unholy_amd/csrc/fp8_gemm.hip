@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void gemm_a8w4_ref_kernel(const uint8_t* a, co
   c[size_t(m) * ldc + n] = f32_to_bf16(acc);
 }
 
-// ---- fp8 dense, skinny (rows in groups of <= 16 staged in LDS) -------------------------------------------------------
+// ---- fp8 dense, skinny (rows in groups of <= 16 staged in LDS) ----
 // A workgroup = 4 waves x DN_TN 16-column tiles. Per 128-input step lane l takes 32 code bytes of weight row
 // n0 + l % 16 at inputs 32 (l / 16) .. + 31 (four lanes cover one row's 128 contiguous bytes), dequantizes them and
 // the matching activation inputs exactly to bf16 and issues four bf16 MFMAs per column tile. e8m0 scales are
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(DN_NT) void fp8_skinny_kernel(Fp8GemmArgs a) {
   }
 }
 
-// ---- fp8 dense, small M (<= 64 rows): bandwidth-shaped --------------------------------------------------------------
+// ---- fp8 dense, small M (<= 64 rows), what the K-part kernel does not take (K > 8192): bandwidth-shaped ----
 // One workgroup per 16-column tile; its 8 waves split K (wave w takes 128-blocks w * per .. + per - 1), so the grid
 // covers every CU and each CU keeps 8 waves x 64 lanes x 128 B of weights in flight (four 128-blocks per wave are
 // loaded before any is used). Lane (nl, g) reads 32 weight bytes of column n0 + nl at inputs 32g .. + 31 of a block
@@ -433,6 +433,7 @@ __global__ __launch_bounds__(64 * FV_WAVES) void fp8_gemv_kernel(Fp8GemmArgs a, 
 }
 
 void launch_fp8_gemv_xq(const Fp8GemmArgs& a, hipStream_t st) {
+  if (fp8_kpart_fits(a)) return launch_fp8_kpart_xq(a, st);
   const size_t lds = size_t(a.M) * a.K + size_t(a.M) * (a.K / 128) * 4;
   auto* kern = &fp8_gemv_kernel<true, 1, true>;
   UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -450,7 +451,7 @@ void launch_fp8_gemv_t(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts& pp)
 }
 
 
-// ---- fp8 dense, 16 < M <= 256 with fp32 scales: row tiles ------------------------------------------------------------
+// ---- fp8 dense, 16 < M <= 256 with fp32 scales, weights past 4 GiB (else the K-part kernel): row tiles ----
 // A workgroup per 32 columns x 32 rows over the whole of K (<= 8,192), bf16 C written directly, one launch:
 // - 16 waves = 16 K parts of one 32 x 32 output tile (bf16 MFMA 32x32x16); part p takes block p of every 2,048-input
 //   chunk;
@@ -753,7 +754,8 @@ void launch_fp8_gemv(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts* parts
   if (!a.a) throw std::runtime_error("fp8 gemm: null operand");
   const bool f32s = a.sa32 != nullptr;
   if (!parts && (f32s ? !a.sw32 : (!a.sa8 || !a.sw8))) throw std::runtime_error("fp8 gemm: scales");
-  if (f32s) launch_fp8_gemv_t<true>(a, st, pp);
+  if (parts && fp8_kpart_parts_fits(a, pp)) launch_fp8_kpart_parts(a, pp, st);
+  else if (f32s) launch_fp8_gemv_t<true>(a, st, pp);
   else launch_fp8_gemv_t<false>(a, st, pp);
 }
 

@@ -42,17 +42,21 @@ void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st);
 // The LDS-ring MFMA GEMM (N % 128, K % 128, ldc % 8; fp8_tiled_fits says whether a shape qualifies).
 bool fp8_tiled_fits(const Fp8GemmArgs& a);
 void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st);
-// 16 < M: a workgroup per output tile of up to 96 x 64, K split over its waves (N % 16, K <= 8192); its estimated time.
+// A workgroup per output tile of up to 96 x 64, K split over its waves (K <= 8192), and its estimated time; the column
+// ranges of gemv_w8a8_parts (M <= 32), and bf16 rows quantized in the kernel (fp32 scales, M <= 16).
 bool fp8_kpart_fits(const Fp8GemmArgs& a);
 double fp8_kpart_us(const Fp8GemmArgs& a);
 void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st);
+bool fp8_kpart_parts_fits(const Fp8GemmArgs& a, const Fp8Parts& pp);
+void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_t st);
+void launch_fp8_kpart_xq(const Fp8GemmArgs& a, hipStream_t st);
 double fp8_tiled_us(const Fp8GemmArgs& a);
 // The same for the grouped projection (R % 16, K <= 65536).
 bool grouped_kpart_fits(int M, int G, int R, int K);
 double grouped_kpart_us(int M, int G, int R, int K);
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st);
-// M <= 16: the GEMV; past it the K-part kernel or the tiled GEMM, by their estimated times; where neither fits the row
+// The K-part kernel or the tiled GEMM, by their estimated times; where neither fits (operands past 4 GiB, K > 8192) the row
 // tiles, the GEMV (M <= 64) or the row-group kernel.
 void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st);
 

@@ -1,4 +1,4 @@
-// Dense fp8 GEMM for 16 < M up to the low thousands: C[M, N] (bf16) = A[M, K] (e4m3) x W[N, K]^T (e4m3), per-128 scales
+// Dense fp8 GEMM for up to ~700 rows: C[M, N] (bf16) = A[M, K] (e4m3) x W[N, K]^T (e4m3), per-128 scales
 // (e8m0 or fp32, as fp8_tiled.hip).
 //
 // What bounds these sizes is getting each CU's share of W and A to it: 4096 x 4096 weights are 64 KB per CU, and a
@@ -16,7 +16,8 @@
 //   block's MFMA chain starts from zero and is folded as acc += raw * (sa * sw).
 // Steps (act_quant + GEMM, us, 4096 x 4096) against the kernels that ran before it: e8m0 M = 32 15.5 -> 11.1, 64 20.0 ->
 // 12.1, 128 38.5 -> 15.2, 256 41.6 -> 19.9, 300 41.3 -> 21.8, 512 42.3 -> 32.0; fp32 M = 64 13.6 -> 11.9, 256 34.6 ->
-// 20.2, 300 43.5 -> 23.3. 32768 x 1024, e8m0, M = 64: 97 -> 19.
+// 20.2, 300 43.5 -> 23.3. 32768 x 1024, e8m0, M = 64: 97 -> 19. Decode rows (before: every lane 32 bytes of its own row):
+// e8m0 M = 1 10.5 -> 8.7, 16 12.2 -> 9.6, 16 x 32768 x 1024 36 -> 14; the fused form M = 1 7.2 -> 6.3, 4 10.5 -> 8.7.
 #include <algorithm>
 #include <stdexcept>
 
@@ -65,9 +66,14 @@ __device__ __forceinline__ void kp_reduce(const v4f (&acc)[RB][CB], uint8_t* sme
   }
 }
 
-template <bool F32S, int RB, int CB>
+// XQ (fp32 scales, one row block): A arrives as bf16 rows (a.xa), quantized here as act_quant_fp8_f32s does (s = max(amax,
+// 1e-4) * fp32(1/448), codes e4m3(x / s); 8 values per lane, a block's amax a DPP row max over 16 lanes). Each wave
+// quantizes the rows of its own K part into its own LDS, behind its first weight loads: no wave waits for another.
+// pp.n > 0 (gemv_w8a8_parts: e8m0 scales, one row tile, CB = 1): column ranges, each with its weights and output.
+template <bool F32S, int RB, int CB, bool XQ = false>
 __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp8_kpart_kernel(
-    Fp8GemmArgs a, int row_tiles, int tile_rows) {
+    Fp8GemmArgs a, Fp8Parts pp, int row_tiles, int tile_rows) {
+  static_assert(!XQ || (F32S && RB == 1));
   extern __shared__ __align__(16) uint8_t smem[];
   const int M = a.M, K = a.K, KS = K / 128;
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
@@ -75,8 +81,19 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
   // Work item = column block x row tiles + row tile; XCD x takes the x-th eighth of the items, so that the row tiles of
   // a column block share one L2.
   const int nw = gridDim.x, lin = blockIdx.x;
-  const int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
-  const int row0 = (wi % row_tiles) * tile_rows, col0 = (wi / row_tiles) * (16 * CB);
+  int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
+  if constexpr (!F32S && CB == 1)
+    if (pp.n) {
+      int p = 0;
+      while (p + 1 < pp.n && wi >= pp.t0[p + 1]) ++p;
+      wi -= pp.t0[p];
+      a.w = pp.w[p];
+      a.sw8 = pp.sw[p];
+      a.c = pp.c[p];
+      a.ldc = pp.ldc[p];
+      a.N = pp.N[p];
+    }
+  const int N = a.N, row0 = (wi % row_tiles) * tile_rows, col0 = (wi / row_tiles) * (16 * CB);
   const int Mt = min(tile_rows, M - row0);
   const int per = (KS + KP_WAVES - 1) / KP_WAVES, b0 = min(KS, wave * per), n = min(KS, b0 + per) - b0;  // blocks
 
@@ -90,7 +107,7 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
   for (int q = 0; q < NSET; ++q)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) sav[q][rb] = q * 4 < per ? sa_at(rb * 16 + l16, b0 + 4 * q + g) : 0.0f;
+    for (int rb = 0; rb < RB; ++rb) sav[q][rb] = !XQ && q * 4 < per ? sa_at(rb * 16 + l16, b0 + 4 * q + g) : 0.0f;
   {
     const size_t i = size_t(col0 / 128) * KS + min(b0 + (lane & 7), KS - 1);
     swv = F32S ? a.sw32[i] : e8m0_to_f32(a.sw8[i]);
@@ -98,21 +115,69 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
 
   // The wave's slot in LDS: one 128-input block, RB row blocks then CB column blocks of 16 rows x 128 bytes. A direct
   // load covers 8 rows x 128 bytes; the 16-byte piece p of row r sits at p ^ ((r >> 1) & 7).
-  constexpr int SLOT = (RB + CB) * 2048, NL = 2 * (RB + CB);
+  // XQ: the weights' blocks only; the quantized rows of all the wave's blocks lie behind the slots, [per][16][128] codes
+  // (pieces as above) and [per][16] fp32 scales.
+  constexpr int AB = XQ ? 0 : RB, SLOT = (AB + CB) * 2048, NL = 2 * (AB + CB);
   uint8_t* const slot = smem + wave * SLOT;
+  uint8_t* const xcodes = smem + KP_WAVES * SLOT + wave * (per * (2048 + 64));
+  float* const xscale = reinterpret_cast<float*>(xcodes + per * 2048);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(slot));
   uint32_t off[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int r = 8 * i + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
-    off[i] = (i < 2 * RB ? uint32_t(row0 + min(r, Mt - 1)) : uint32_t(col0 + r - 16 * RB)) * uint32_t(K) + uint32_t(p * 16);
+    // rows and columns past the tile repeat its last (their results are not stored)
+    off[i] = (i < 2 * AB ? uint32_t(row0 + min(r, Mt - 1)) : uint32_t(min(col0 + r - 16 * AB, N - 1))) * uint32_t(K) +
+             uint32_t(p * 16);
   }
   const auto issue = [&](int c) {
     const size_t k = size_t(b0 + c) * 128;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) dma16(i < 2 * RB ? a.a + k : a.w + k, off[i], lds0 + uint32_t(i * 1024));
+    for (int i = 0; i < NL; ++i) dma16(i < 2 * AB ? a.a + k : a.w + k, off[i], lds0 + uint32_t(i * 1024));
   };
+  // Item it = (row, block, piece of 8 values), 16 lanes a block.
+  const int xitems = M * n * 16;
+  const auto x_src = [&](int it) {
+    const int c = min(it, xitems - 1), r = c / (16 * n), rem = c % (16 * n);
+    return a.xa + size_t(r) * a.ldx + size_t(b0) * 128 + rem * 8;
+  };
+  const auto quant_item = [&](int it, const v4i raw) {
+    const int r = it / (16 * n), rem = it % (16 * n), blk = rem >> 4, l = rem & 15;
+    float v[8], am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(uint32_t(raw[i]) << 16);
+      v[2 * i + 1] = __uint_as_float(uint32_t(raw[i]) & 0xffff0000u);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(v[i]));
+    am = row16_max(am);
+    if (it >= xitems) return;
+    const float sc = fmaxf(am, 1e-4f) * (1.0f / 448.0f);
+    uint32_t c0, c1;
+    fp8_codes8(v, sc, c0, c1);
+    *reinterpret_cast<uint2*>(xcodes + blk * 2048 + r * 128 + ((l >> 1) ^ ((r >> 1) & 7)) * 16 + (l & 1) * 8) =
+        make_uint2(c0, c1);
+    if (l == 0) xscale[blk * 16 + r] = sc;
+  };
+  v4i x0 = {0, 0, 0, 0};
+  if constexpr (XQ)
+    if (n > 0) x0 = vload16(x_src(lane));
   if (n > 0) issue(0);
+  if constexpr (XQ)
+    if (n > 0) {
+      wait_vm<NL>();  // the rows' first pass; the weights stay in flight
+      asm volatile("" : "+v"(x0));
+      quant_item(lane, x0);
+      for (int base = 64; base < xitems; base += 256) {  // uniform bound: 16-lane groups stay whole; 4 passes' loads at once
+        v4i x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const v4i*>(x_src(base + 64 * i + lane));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (base + 64 * i < xitems) quant_item(base + 64 * i + lane, x[i]);
+      }
+    }
   v4f acc[RB][CB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
@@ -134,13 +199,14 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
     v4i aq[RB][2], bq[CB][2];
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
-      bq[cb][0] = *reinterpret_cast<const v4i*>(rd + (RB + cb) * 2048 + p0);
-      bq[cb][1] = *reinterpret_cast<const v4i*>(rd + (RB + cb) * 2048 + p1);
+      bq[cb][0] = *reinterpret_cast<const v4i*>(rd + (AB + cb) * 2048 + p0);
+      bq[cb][1] = *reinterpret_cast<const v4i*>(rd + (AB + cb) * 2048 + p1);
     }
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      aq[rb][0] = *reinterpret_cast<const v4i*>(rd + rb * 2048 + p0);
-      aq[rb][1] = *reinterpret_cast<const v4i*>(rd + rb * 2048 + p1);
+      const uint8_t* const ra = XQ ? xcodes + c * 2048 + l16 * 128 : rd + rb * 2048;
+      aq[rb][0] = *reinterpret_cast<const v4i*>(ra + p0);
+      aq[rb][1] = *reinterpret_cast<const v4i*>(ra + p1);
     }
     if (c + 1 < n) {  // the next block into the slot as soon as it has been read: in flight under this block's MFMAs
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -149,6 +215,7 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
     }
     const float sw = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(__float_as_uint(swv)), c & 7)));
     const auto sa_of = [&](int rb, int row) {  // the scale of row `row` of the row block in block c
+      if constexpr (XQ) return xscale[c * 16 + row];
       const float v = c >= 4 ? sav[1][rb] : sav[0][rb];
       return __uint_as_float(uint32_t(__builtin_amdgcn_ds_bpermute(((c & 3) * 16 + row) * 4, int(__float_as_uint(v)))));
     };
@@ -187,19 +254,23 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
   }
 
   kp_reduce(acc, smem, [&](int r, int col, float v) {
-    if (r < Mt) a.c[size_t(row0 + r) * a.ldc + col0 + col] = f32_to_bf16(v);
+    if (r < Mt && col0 + col < N) a.c[size_t(row0 + r) * a.ldc + col0 + col] = f32_to_bf16(v);
   });
 }
 
-template <bool F32S, int RB, int CB>
-void launch_t(const Fp8GemmArgs& a, hipStream_t st) {
-  constexpr size_t lds = std::max<size_t>(kp_reduce_lds<RB, CB>(), size_t(KP_WAVES) * (RB + CB) * 2048);
-  static_assert(lds <= 160 * 1024);
+template <bool F32S, int RB, int CB, bool XQ = false>
+void launch_t(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts& pp = Fp8Parts{}) {
+  constexpr size_t red = kp_reduce_lds<RB, CB>(), slots = size_t(KP_WAVES) * ((XQ ? 0 : RB) + CB) * 2048;
+  static_assert(std::max(red, slots) <= 160 * 1024);
+  const size_t rows = XQ ? size_t(KP_WAVES) * ((a.K / 128 + KP_WAVES - 1) / KP_WAVES) * (2048 + 64) : 0;
+  const size_t lds = std::max(red, slots + rows);
   const int rt = (a.M + 16 * RB - 1) / (16 * RB), tile_rows = ((a.M + rt - 1) / rt + 15) / 16 * 16;
-  auto* kern = &fp8_kpart_kernel<F32S, RB, CB>;
-  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(lds)));
-  kern<<<dim3(unsigned(a.N / (16 * CB)) * unsigned(rt)), 64 * KP_WAVES, lds, st>>>(a, rt, tile_rows);
+  auto* kern = &fp8_kpart_kernel<F32S, RB, CB, XQ>;
+  if (lds > 65536)
+    UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 int(lds)));
+  const unsigned cols = pp.n ? unsigned(pp.t0[pp.n]) : cdiv(size_t(a.N), 16 * CB);
+  kern<<<dim3(cols * unsigned(rt)), 64 * KP_WAVES, lds, st>>>(a, pp, rt, tile_rows);
   UH_CHECK_LAUNCH();
 }
 
@@ -328,27 +399,37 @@ struct KpForm {
   int rb, cb;
   double read, next;  // RB + CB, more where the registers leave less in flight; the cost of a further round
 };
-constexpr KpForm kForms[] = {{2, 1, 3.0, 1.0}, {2, 2, 4.0, 1.2}, {4, 2, 6.0, 3.0},
+constexpr KpForm kForms[] = {{1, 1, 2.0, 0.8}, {2, 1, 3.0, 1.0}, {2, 2, 4.0, 1.2}, {4, 2, 6.0, 3.0},
                              {4, 4, 9.0, 3.5}, {5, 4, 10.5, 3.5}, {6, 4, 13.0, 3.5}};
 double form_us(const Fp8GemmArgs& a, const KpForm& f) {
-  const size_t wg = size_t((a.M + 16 * f.rb - 1) / (16 * f.rb)) * (a.N / (16 * f.cb));
+  const size_t wg = size_t((a.M + 16 * f.rb - 1) / (16 * f.rb)) * cdiv(size_t(a.N), 16 * f.cb);
   const double rounds = double((wg + 255) / 256);
   return 7.0 + (rounds - 1.0) * f.next + rounds * f.read * a.K * 0.00034;
 }
 int best_form(const Fp8GemmArgs& a) {
-  const int forms = a.sa32 ? 5 : 6;  // 6 x 4 with fp32 scales spills
+  const int forms = a.sa32 ? 6 : 7;  // 6 x 4 with fp32 scales spills
   int best = 0;
   for (int i = 1; i < forms; ++i)
-    if (a.N % (16 * kForms[i].cb) == 0 && form_us(a, kForms[i]) < form_us(a, kForms[best])) best = i;
+    if (form_us(a, kForms[i]) < form_us(a, kForms[best])) best = i;
   return best;
 }
 }  // namespace
 
 bool fp8_kpart_fits(const Fp8GemmArgs& a) {
-  return a.M > 16 && a.N > 0 && a.N % 16 == 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET &&
-         (a.sa32 ? a.sw32 != nullptr : a.sa8 && a.sw8) && size_t(a.M) * a.K < (size_t(1) << 32) &&
+  return a.M > 0 && a.N > 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET &&
+         (a.sa32 || a.xa ? a.sw32 != nullptr : a.sa8 && a.sw8) && size_t(a.M) * a.K < (size_t(1) << 32) &&
          size_t(a.N) * a.K < (size_t(1) << 32);
 }
+bool fp8_kpart_parts_fits(const Fp8GemmArgs& a, const Fp8Parts& pp) {
+  for (int i = 0; i < pp.n; ++i)
+    if (size_t(pp.N[i]) * a.K >= (size_t(1) << 32)) return false;
+  return a.M > 0 && a.M <= 32 && a.K <= 128 * KP_WAVES * 4 * NSET;
+}
+void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_t st) {
+  if (a.M <= 16) launch_t<false, 1, 1>(a, st, pp);
+  else launch_t<false, 2, 1>(a, st, pp);
+}
+void launch_fp8_kpart_xq(const Fp8GemmArgs& a, hipStream_t st) { launch_t<true, 1, 1, true>(a, st); }
 double fp8_kpart_us(const Fp8GemmArgs& a) { return form_us(a, kForms[best_form(a)]); }
 
 void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
@@ -356,19 +437,21 @@ void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
   if (!a.a || !a.w || !a.c) throw std::runtime_error("fp8 gemm: null operand");
   if (a.sa32) {
     switch (best_form(a)) {
-      case 0: return launch_t<true, 2, 1>(a, st);
-      case 1: return launch_t<true, 2, 2>(a, st);
-      case 2: return launch_t<true, 4, 2>(a, st);
-      case 3: return launch_t<true, 4, 4>(a, st);
+      case 0: return launch_t<true, 1, 1>(a, st);
+      case 1: return launch_t<true, 2, 1>(a, st);
+      case 2: return launch_t<true, 2, 2>(a, st);
+      case 3: return launch_t<true, 4, 2>(a, st);
+      case 4: return launch_t<true, 4, 4>(a, st);
       default: return launch_t<true, 5, 4>(a, st);
     }
   }
   switch (best_form(a)) {
-    case 0: return launch_t<false, 2, 1>(a, st);
-    case 1: return launch_t<false, 2, 2>(a, st);
-    case 2: return launch_t<false, 4, 2>(a, st);
-    case 3: return launch_t<false, 4, 4>(a, st);
-    case 4: return launch_t<false, 5, 4>(a, st);
+    case 0: return launch_t<false, 1, 1>(a, st);
+    case 1: return launch_t<false, 2, 1>(a, st);
+    case 2: return launch_t<false, 2, 2>(a, st);
+    case 3: return launch_t<false, 4, 2>(a, st);
+    case 4: return launch_t<false, 4, 4>(a, st);
+    case 5: return launch_t<false, 5, 4>(a, st);
     default: return launch_t<false, 6, 4>(a, st);
   }
 }
