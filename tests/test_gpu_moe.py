@@ -333,3 +333,21 @@ def test_moe_forward_tile_sizes(T, E, K, D, I):
     synchronize()
     assert np.array_equal(sel.download((T, K), np.int32), sel_ref)
     assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2
+
+
+@pytest.mark.parametrize("T,E,K,D,I", [(1, 16, 6, 1024, 512), (1, 8, 2, 4096, 256), (3, 24, 6, 4096, 2048),
+                                       (2, 16, 6, 1024, 512)])
+def test_moe_forward_few_tokens(T, E, K, D, I):
+    """Steps of one to three tokens, whose w1 / w3 launch takes 4-wave workgroups by the number it makes (at most 128 of
+    8 waves; 257 to 384 with K >= 4096) and whose w2 launch is split over K or not by its column tiles: the oracle,
+    max-rel <= 1e-2 per element."""
+    rng = np.random.default_rng(T + E + D)
+    experts, bufs, tab, x, logits = _moe_case(rng, T, E, K, D, I)
+    sel_ref, wt_ref = oracle.route_softmax(logits, K)
+    out_ref, _ = oracle.moe_forward(x, sel_ref, wt_ref, experts, D, I, 10.0)
+    ws_bytes = call("uh_mx_moe_workspace_size", T, K, E, D, I)
+    ws, out = DeviceBuffer(ws_bytes), DeviceBuffer(T * D * 2)
+    call("uh_mx_moe_forward", dev(x), dev(logits), T, K, E, D, I, tab.ptr, 10.0, ws.ptr, ws_bytes, out.ptr, None, None,
+         None)
+    synchronize()
+    assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2

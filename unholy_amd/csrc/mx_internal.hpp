@@ -37,6 +37,7 @@ struct MxGemvArgs {
   // > 0: one matrix, two column streams per wave: projection 1 is projection 0's matrix from 16-column tile `split`
   // on (codes, scales and outputs offset by split tiles); the grid covers split tiles.
   int split;
+  int tiles_hint = 0;     // GEMV: the tiles expected to be live, of ntiles (0: all; a choice of kernel, not a bound)
   bool few_rows = false;  // GEMM on bf16 rows: most tiles hold at most 64 rows (a choice of kernel, not a bound)
 };
 
@@ -67,6 +68,11 @@ void launch_mx_gemm_rows(const uint16_t* xa, const int32_t* x_rows, int K, const
                          hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
                          const uint8_t* const* s_tab2, uint16_t* out2, const MxGlu& glu, bool few_rows);
 bool mx_gemm_pipe_on();
+// mx_grouped_gemv_x with MxGemvArgs::tiles_hint.
+void launch_mx_gemv_x(const uint16_t* x, int ldx, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
+                      const uint8_t* const* w_tab, const uint8_t* const* s_tab, uint16_t* out, int ldo, int N,
+                      hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
+                      const uint8_t* const* s_tab2, uint16_t* out2, int max_rows, const MxGlu& glu, int tiles_hint);
 void launch_mx_transform(int mode, const uint16_t* x, int ldx, const int32_t* x_rows, const uint16_t* u,
                          const float* w, float limit, const int32_t* row_expert, const uint8_t* const* s_tab,
                          uint16_t* out, uint8_t* q, uint8_t* qs, int K, int P, hipStream_t st);

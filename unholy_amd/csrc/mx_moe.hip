@@ -585,28 +585,19 @@ static bool ksplit_enabled() {
   return on;
 }
 
-// Workgroup shape: 8 waves (128 outputs) for every launch. A requantizing epilogue needs a whole 128-output block;
-// for the others 8-wave workgroups measured 1% (decode) to 3% (verify) faster than 4-wave ones, whose smaller work
-// items were expected to balance better.
+// Workgroup shape: 8 waves (128 outputs), one workgroup per CU by its registers. 4 waves (three per CU) where 8-wave
+// workgroups would leave half the CUs idle, or make a second round for at most half of them: up to 128, and 257 to 384
+// with K >= 4096 (whole forward, w1 / w3 with 8 / 4 waves, us, E = 256, D = 4096, I = 2048: T = 1 (96 workgroups of 8)
+// 32.9 / 29.8, 2 (192) 41.8 / 44.6, 3 (281) 61.7 / 58.2, 4 (366) 70.4 / 66.6, 5 (453) 77.3 / 80.9, 8 110 / 115; D =
+// 2048, I = 1024, E = 64, T = 8 (278) 32.5 / 33.3). A requantizing epilogue needs a whole 128-output block.
 template <int NP, int GM, int AM, int W>
-void launch_gemv_w(const MxGemvArgs& a, int ntiles, hipStream_t st) {
-  const size_t lds = size_t(a.rows_cap) * (a.K + GV_PAD) + size_t(a.rows_cap) * (a.K / 128);
+void launch_gemv_w(const MxGemvArgs& a, int ntiles, size_t lds, hipStream_t st) {
   const size_t ntn = a.split ? size_t(a.split) : size_t(a.N) / 16;
-  if constexpr (GM == 0 && NP == 1) {
-    // A launch of fewer than 256 workgroups (one per CU) is latency-bound: split each tile's K over its waves.
-    if (size_t(ntiles) * cdiv(ntn, W) < 256 && a.K % (128 * W) == 0 && !a.out32 && ksplit_enabled()) {
-      auto* kern = &mx_gemv_kernel<NP, GM, AM, W, true>;
-      set_lds_limit(kern, std::max<size_t>(lds, size_t(W) * NP * 64 * 16));
-      kern<<<dim3(unsigned(ntn), unsigned(ntiles), 1), 64 * W, std::max<size_t>(lds, size_t(W) * NP * 64 * 16), st>>>(a);
-      UH_CHECK_LAUNCH();
-      return;
-    }
-  }
   const dim3 grid(cdiv(ntn, W), unsigned(ntiles), 1);
-  // bf16 rows when they fit the LDS next to the epilogue's static share (the kernel's registers already hold it to
-  // one 8-wave workgroup per CU)
+  // bf16 rows when they fit the LDS next to the epilogue's static share (with 8 waves the kernel's registers already
+  // hold it to one workgroup per CU; three of 4 waves share the LDS)
   const size_t lds_bf = size_t(a.rows_cap + 1) * (a.K + 8) * 2;
-  if (lds_bf <= 156 * 1024) {
+  if (lds_bf <= (W == 8 ? 156 : 52) * 1024) {
     auto* kern = &mx_gemv_kernel<NP, GM, AM, W, false, true>;
     set_lds_limit(kern, lds_bf);
     kern<<<grid, 64 * W, lds_bf, st>>>(a);
@@ -620,7 +611,29 @@ void launch_gemv_w(const MxGemvArgs& a, int ntiles, hipStream_t st) {
 }
 template <int NP, int GM, int AM>
 void launch_gemv_t(const MxGemvArgs& a, int ntiles, hipStream_t st) {
-  launch_gemv_w<NP, GM, AM, GV_WAVES>(a, ntiles, st);
+  constexpr int W = GV_WAVES;
+  const size_t lds = size_t(a.rows_cap) * (a.K + GV_PAD) + size_t(a.rows_cap) * (a.K / 128);
+  const size_t ntn = a.split ? size_t(a.split) : size_t(a.N) / 16;
+  [[maybe_unused]] const size_t n8 = size_t(ntiles) * cdiv(ntn, W);
+  if constexpr (GM == 0 && NP == 1) {
+    // So few column tiles that one round of workgroups (12 waves per CU) takes a workgroup for each: split each tile's K
+    // over its 8 waves. (Past that the split only multiplies the workgroups' start-ups: the w2 launch of T = 1, 1,536
+    // tiles, took 15 us split and 6 not.)
+    const size_t tiles = size_t(ntiles) * ntn;
+    if (n8 < 256 && tiles * W <= 256 * 12 && a.K % (128 * W) == 0 && !a.out32 && ksplit_enabled()) {
+      auto* kern = &mx_gemv_kernel<NP, GM, AM, W, true>;
+      const size_t l = std::max<size_t>(lds, size_t(W) * NP * 64 * 16);
+      set_lds_limit(kern, l);
+      kern<<<dim3(unsigned(ntn), unsigned(ntiles), 1), 64 * W, l, st>>>(a);
+      UH_CHECK_LAUNCH();
+      return;
+    }
+  }
+  if constexpr (GM == 2) {
+    const size_t live = (a.tiles_hint > 0 ? size_t(a.tiles_hint) : size_t(ntiles)) * cdiv(ntn, W);
+    if (live <= 128 || (live > 256 && live <= 384 && a.K >= 4096)) return launch_gemv_w<NP, GM, AM, 4>(a, ntiles, lds, st);
+  }
+  launch_gemv_w<NP, GM, AM, W>(a, ntiles, lds, st);
 }
 
 // mx_xform_in_q (mx_moe.hip:132-176, kMode 1): rows r in [plan->remote0, plan->P) of a resident expert rebuilt from
@@ -941,16 +954,24 @@ void mx_grouped_gemv_q(const uint8_t* q, const uint8_t* qs, int K, const Exl3Til
                  ntiles, 0, st);
 }
 
-void mx_grouped_gemv_x(const bf16* x, int ldx, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
-                       const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
-                       hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
-                       const uint8_t* const* s_tab2, bf16* out2, int max_rows, const MxGlu& glu) {
+void launch_mx_gemv_x(const bf16* x, int ldx, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
+                      const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
+                      hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
+                      const uint8_t* const* s_tab2, bf16* out2, int max_rows, const MxGlu& glu, int tiles_hint) {
   if ((glu.hh || glu.hq) && ldo != N && (out || out2)) throw std::runtime_error("mx_grouped_gemv_x: glu shape");
   MxGemvArgs a = gemv_args(x, nullptr, nullptr, K, tiles, w_tab, s_tab, out, ldo, N, ntiles_dev, w_tab2, s_tab2, out2,
                            max_rows, glu);
   a.x_rows = x_rows;
   a.ldx = ldx;
+  a.tiles_hint = tiles_hint;
   launch_mx_gemv(a, ntiles, 2, st);
+}
+void mx_grouped_gemv_x(const bf16* x, int ldx, const int32_t* x_rows, int K, const Exl3Tile* tiles, int ntiles,
+                       const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
+                       hipStream_t st, const int* ntiles_dev, const uint8_t* const* w_tab2,
+                       const uint8_t* const* s_tab2, bf16* out2, int max_rows, const MxGlu& glu) {
+  launch_mx_gemv_x(x, ldx, x_rows, K, tiles, ntiles, w_tab, s_tab, out, ldo, N, st, ntiles_dev, w_tab2, s_tab2, out2,
+                   max_rows, glu, 0);
 }
 
 }  // namespace unholy::kernels
