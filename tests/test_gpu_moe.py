@@ -336,18 +336,25 @@ def test_moe_forward_tile_sizes(T, E, K, D, I):
 
 
 @pytest.mark.parametrize("T,E,K,D,I", [(1, 16, 6, 1024, 512), (1, 8, 2, 4096, 256), (3, 24, 6, 4096, 2048),
-                                       (2, 16, 6, 1024, 512)])
+                                       (2, 16, 6, 1024, 512), (1, 300, 8, 256, 128), (2, 24, 5, 384, 640),
+                                       (2, 8, 1, 128, 128), (1, 6, 6, 1152, 2304), (4, 6, 2, 512, 256)])
 def test_moe_forward_few_tokens(T, E, K, D, I):
-    """Steps of one to three tokens, whose w1 / w3 launch takes 4-wave workgroups by the number it makes (at most 128 of
-    8 waves; 257 to 384 with K >= 4096) and whose w2 launch is split over K or not by its column tiles: the oracle,
-    max-rel <= 1e-2 per element."""
+    """Steps of one and two tokens (two launches: the router's wide form past 256 experts, one and eight picks, the same
+    expert for both tokens, units that do not fill the last workgroup, fewer 128-blocks than K parts), and of three and
+    four, whose w1 / w3 launch takes 4-wave workgroups by the number it makes (at most 128 of 8 waves; 257 to 384 with K
+    >= 4096): the oracle, the routing bit-exact, max-rel <= 1e-2 per element, with and without the sel / wt outputs."""
     rng = np.random.default_rng(T + E + D)
     experts, bufs, tab, x, logits = _moe_case(rng, T, E, K, D, I)
     sel_ref, wt_ref = oracle.route_softmax(logits, K)
     out_ref, _ = oracle.moe_forward(x, sel_ref, wt_ref, experts, D, I, 10.0)
     ws_bytes = call("uh_mx_moe_workspace_size", T, K, E, D, I)
     ws, out = DeviceBuffer(ws_bytes), DeviceBuffer(T * D * 2)
-    call("uh_mx_moe_forward", dev(x), dev(logits), T, K, E, D, I, tab.ptr, 10.0, ws.ptr, ws_bytes, out.ptr, None, None,
-         None)
-    synchronize()
-    assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2
+    sel, wt = DeviceBuffer(T * K * 4), DeviceBuffer(T * K * 4)
+    for s, w in ((None, None), (sel, wt)):
+        out.zero()
+        call("uh_mx_moe_forward", dev(x), dev(logits), T, K, E, D, I, tab.ptr, 10.0, ws.ptr, ws_bytes, out.ptr, s, w,
+             None)
+        synchronize()
+        assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2
+    assert np.array_equal(sel.download((T, K), np.int32), sel_ref)
+    np.testing.assert_allclose(wt.download((T, K), np.float32), wt_ref, rtol=2e-6, atol=0)

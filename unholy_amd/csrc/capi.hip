@@ -823,6 +823,17 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     float* s_wt = wt ? wt : w.wt;
     const auto t = [&](int m, int f) { return tab + size_t(2 * m + f) * E; };
     mark(0);
+    const k::MoeTokenArgs tk{x, logits, T, K, E, D, I, tab, limit, s_sel, s_wt, w.row_expert, w.h, out};
+    if (k::moe_token_fits(tk)) {  // one or two tokens: two launches
+      mark(1);
+      mark(2);
+      k::launch_moe_token_up(tk, st);
+      mark(3);
+      k::launch_moe_token_down(tk, st);
+      mark(4);
+      mark(5);
+      return;
+    }
     // Dispatch in one single-block launch up to 512 picks; the routing in that launch too while every token has a
     // wave of its own (T <= 8), else a wave per token over many workgroups first.
     const bool one_block = P <= k::kMoeMidMaxPicks, route_in = one_block && T <= 8;

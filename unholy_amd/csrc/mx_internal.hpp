@@ -82,4 +82,24 @@ void launch_mx_transform(int mode, const uint16_t* x, int ldx, const int32_t* x_
 void launch_swiglu_quant(const uint16_t* g, int ldg, const uint16_t* u, int ldu, int M, int I, float limit,
                          uint16_t* hh, uint8_t* q, uint8_t* qs, hipStream_t st);
 
+// The forward of a step of at most kTokenMaxT tokens in two launches (mx_token.hip): routing + w1 / w3 + SwiGLU into h
+// [T K, I] (each token's picks in ascending expert order, also written to row_expert [T K]), then w2 + combine. sel
+// (may be null, then wt is not written) / wt: the routing. tab: the forward's 6 E pointers.
+constexpr int kTokenMaxT = 2;
+struct MoeTokenArgs {
+  const uint16_t* x;
+  const float* logits;
+  int T, K, E, D, I;
+  const uint8_t* const* tab;
+  float limit;
+  int32_t* sel;
+  float* wt;
+  int32_t* row_expert;
+  uint16_t* h;
+  uint16_t* out;
+};
+bool moe_token_fits(const MoeTokenArgs& a);
+void launch_moe_token_up(const MoeTokenArgs& a, hipStream_t st);
+void launch_moe_token_down(const MoeTokenArgs& a, hipStream_t st);
+
 }  // namespace unholy::kernels
