@@ -54,6 +54,28 @@ def test_fp8_f32_scales(M, N, K):
     assert mr <= 1e-2
 
 
+@pytest.mark.parametrize("M,K,pad", [(3, 128, 0), (65, 4096, 8), (4099, 4096, 0)])
+@pytest.mark.parametrize("f32s", [False, True])
+def test_act_quant_block_magnitudes(M, K, pad, f32s):
+    """Codes and scales against the oracle, bit for bit, for blocks from 1e-30 to 1e30, with -0, values far below their
+    block's scale and exact halves of a code step (the quotient's last bit decides them): one and four items a thread."""
+    rng = np.random.default_rng(M + K)
+    mag = 10.0 ** rng.integers(-30, 31, (M, K // 128)).astype(np.float64)
+    x = rng.standard_normal((M, K)) * np.repeat(mag, 128, 1)
+    x[:, 1::16] = -0.0
+    x[:, 2::16] *= 1e-7
+    x[:, 0::128] = 448 * mag
+    x[:, 3::32] = 17 * np.repeat(mag, 128, 1)[:, 3::32]  # between the codes 16 and 18
+    xb = oracle.f32_to_bf16(x.astype(np.float32))
+    xp = np.zeros((M, K + pad), xb.dtype)
+    xp[:, :K] = xb
+    q, sa = DeviceBuffer(M * K), DeviceBuffer(M * (K // 128) * (4 if f32s else 1))
+    call("uh_act_quant_fp8_f32s" if f32s else "uh_act_quant_fp8", dev(xp), K + pad, q, sa, M, K, 128, None)
+    q_ref, sa_ref = oracle.act_quant_fp8_f32s(xb) if f32s else oracle.act_quant_fp8(xb, 128)
+    assert np.array_equal(sa.download((M, K // 128), np.float32 if f32s else np.uint8), sa_ref)
+    assert np.array_equal(q.download((M, K), np.uint8), q_ref)
+
+
 @pytest.mark.parametrize("M,N,K,pad", [(1, 4096, 4096, 0), (5, 136, 384, 64), (16, 1024, 1024, 8), (3, 200, 256, 0)])
 def test_fp8_f32s_fused_quant_is_bit_identical(M, N, K, pad):
     """gemm_fp8_f32s_x (act_quant_fp8_f32s fused into the GEMV, M <= 16) against the two calls it replaces: the same

@@ -63,43 +63,60 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const bf16* __restrict__
 }
 
 // Block 128 with 8 values per thread: 16 consecutive threads per block (16-byte loads, 8-byte code stores), the amax a
-// DPP row max. The item loop bound is uniform so every 16-lane group is whole. Needs ldx % 8 == 0.
-template <int MODE>
+// DPP row max. U items per thread, their loads issued together: 4 for many rows (a workgroup of one item each lives for
+// little more than its load's latency), 1 while that would leave CUs idle. The item loop bound is uniform so every
+// 16-lane group is whole. Needs ldx % 8 == 0.
+template <int MODE, int U>
 __global__ __launch_bounds__(256) void act_quant8_kernel(const bf16* __restrict__ x, int ldx, uint8_t* __restrict__ q,
                                                          void* __restrict__ s, int rows, int cols) {
   const int nb = cols / 128;
   const size_t per_row = size_t(nb) * 16, items = size_t(rows) * per_row;
-  for (size_t base = size_t(blockIdx.x) * 256; base < items; base += size_t(gridDim.x) * 256) {
-    const size_t it = min(base + threadIdx.x, items - 1);
-    const int r = int(it / per_row), rem = int(it % per_row), b = rem >> 4, l = rem & 15;
-    bf16* xr = const_cast<bf16*>(x) + size_t(r) * ldx + size_t(b) * 128 + 8 * l;
-    const uint4 raw = *reinterpret_cast<const uint4*>(xr);
-    const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
-    float v[8], am = 0.0f;
+  for (size_t base = size_t(blockIdx.x) * (256 * U); base < items; base += size_t(gridDim.x) * (256 * U)) {
+    uint4 raw[U];
+    const auto at = [&](int u, int& r, int& b, int& l) {
+      const size_t it = min(base + size_t(u) * 256 + threadIdx.x, items - 1);
+      const int rem = int(it % per_row);
+      r = int(it / per_row);
+      b = rem >> 4;
+      l = rem & 15;
+      return const_cast<bf16*>(x) + size_t(r) * ldx + size_t(b) * 128 + 8 * l;
+    };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(rw[i] << 16);
-      v[2 * i + 1] = __uint_as_float(rw[i] & 0xffff0000u);
+    for (int u = 0; u < U; ++u) {
+      int r, b, l;
+      raw[u] = *reinterpret_cast<const uint4*>(at(u, r, b, l));
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(v[i]));
-    am = row16_max(am);
-    if (base + threadIdx.x >= items) continue;
-    uint32_t c[2];
-    if constexpr (MODE == 2) {
-      const float sc = fmaxf(am, 1e-4f) * (1.0f / 448.0f);
-      fp8_codes8(v, sc, c[0], c[1]);
-      if (l == 0) static_cast<float*>(s)[size_t(r) * nb + b] = sc;
-    } else {
-      const Fp8Block blk = fp8_block_scale(am);
-      fp8_codes8(v, blk, c[0], c[1]);
-      if constexpr (MODE == 1) {  // the fake-quantized values: the codes decoded back (exact)
-        *reinterpret_cast<uint4*>(xr) = __builtin_bit_cast(uint4, fp8x8_to_bf16(c[0], c[1], blk.sc));
-        continue;
+    for (int u = 0; u < U; ++u) {
+      int r, b, l;
+      bf16* const xr = at(u, r, b, l);
+      const uint32_t rw[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
+      float v[8], am = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(rw[i] << 16);
+        v[2 * i + 1] = __uint_as_float(rw[i] & 0xffff0000u);
       }
-      if (l == 0) static_cast<uint8_t*>(s)[size_t(r) * nb + b] = blk.se;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(v[i]));
+      am = row16_max(am);
+      if (base + size_t(u) * 256 + threadIdx.x >= items) continue;
+      uint32_t c[2];
+      if constexpr (MODE == 2) {
+        const float sc = fmaxf(am, 1e-4f) * (1.0f / 448.0f);
+        fp8_codes8(v, sc, c[0], c[1]);
+        if (l == 0) static_cast<float*>(s)[size_t(r) * nb + b] = sc;
+      } else {
+        const Fp8Block blk = fp8_block_scale(am);
+        fp8_codes8(v, blk, c[0], c[1]);
+        if constexpr (MODE == 1) {  // the fake-quantized values: the codes decoded back (exact)
+          *reinterpret_cast<uint4*>(xr) = __builtin_bit_cast(uint4, fp8x8_to_bf16(c[0], c[1], blk.sc));
+          continue;
+        }
+        if (l == 0) static_cast<uint8_t*>(s)[size_t(r) * nb + b] = blk.se;
+      }
+      *reinterpret_cast<uint2*>(q + size_t(r) * cols + size_t(b) * 128 + 8 * l) = make_uint2(c[0], c[1]);
     }
-    *reinterpret_cast<uint2*>(q + size_t(r) * cols + size_t(b) * 128 + 8 * l) = make_uint2(c[0], c[1]);
   }
 }
 
@@ -109,8 +126,15 @@ void launch_act_quant(const bf16* x, int ldx, uint8_t* q, void* s, int rows, int
   if (block != 32 && block != 64 && block != 128) throw std::runtime_error("act_quant: block in {32, 64, 128}");
   if (cols % block) throw std::runtime_error("act_quant: cols % block");
   if (block == 128 && ldx % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && (MODE == 1 || cols % 8 == 0)) {
-    const unsigned grid = unsigned(std::min<size_t>(cdiv(size_t(rows) * (cols / 8), 256), 8192));
-    act_quant8_kernel<MODE><<<grid, 256, 0, st>>>(x, ldx, q, s, rows, cols);
+    const size_t items = size_t(rows) * (cols / 8);
+    // Four items a thread once that still makes eight workgroups a CU: below, one item each finishes sooner (us at K = 4096,
+    // one / four items: M = 1000 4.5 / 4.9, 2000 6.4 / 6.8, 4096 11.9 / 11.1; fp32 scales 13.7 / 12.5).
+    if (items >= size_t(2048) * 1024) {
+      const unsigned grid = unsigned(std::min<size_t>(cdiv(items, 1024), 8192));
+      act_quant8_kernel<MODE, 4><<<grid, 256, 0, st>>>(x, ldx, q, s, rows, cols);
+    } else {
+      act_quant8_kernel<MODE, 1><<<unsigned(cdiv(items, 256)), 256, 0, st>>>(x, ldx, q, s, rows, cols);
+    }
     UH_CHECK_LAUNCH();
     return;
   }

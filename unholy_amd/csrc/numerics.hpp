@@ -155,9 +155,27 @@ __device__ __forceinline__ void fp8_codes8(const float (&v)[8], const Fp8Block& 
   lo = e4m3x4(clamp448(v[0] * b.inv), clamp448(v[1] * b.inv), clamp448(v[2] * b.inv), clamp448(v[3] * b.inv));
   hi = e4m3x4(clamp448(v[4] * b.inv), clamp448(v[5] * b.inv), clamp448(v[6] * b.inv), clamp448(v[7] * b.inv));
 }
+// v / sc with r = RN(1 / sc): a quotient within an ulp, its exact remainder, and one corrected step, which is the
+// correctly rounded quotient (Markstein, Computation of elementary functions on the IBM RISC System/6000 processor,
+// 1990) wherever the remainder does not underflow; below that both quotients encode to 0. Three operations a value, where
+// the compiler's division takes ten (the quantizer alone, 4096 x 4096: 16.2 us to 13.7).
+__device__ __forceinline__ float div_by(float v, float sc, float r) {
+#pragma clang fp contract(off)
+  const float q = v * r;
+  return __builtin_fmaf(-__builtin_fmaf(q, sc, -v), r, q);  // in this order of signs -0 stays -0
+}
 __device__ __forceinline__ void fp8_codes8(const float (&v)[8], float sc, uint32_t& lo, uint32_t& hi) {
-  lo = e4m3x4(clamp448(v[0] / sc), clamp448(v[1] / sc), clamp448(v[2] / sc), clamp448(v[3] / sc));
-  hi = e4m3x4(clamp448(v[4] / sc), clamp448(v[5] / sc), clamp448(v[6] / sc), clamp448(v[7] / sc));
+  float q[8];
+  if (sc < INFINITY) {
+    const float r = 1.0f / sc;  // sc >= 2^-23: no overflow
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = clamp448(div_by(v[i], sc, r));
+  } else {  // a block with an infinity
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = clamp448(v[i] / sc);
+  }
+  lo = e4m3x4(q[0], q[1], q[2], q[3]);
+  hi = e4m3x4(q[4], q[5], q[6], q[7]);
 }
 
 // act_quant_fp8 (block 128) of compact token rows: item `it` of items = U * dim / 8 is 8 values of row x[u2t[u]]
