@@ -191,7 +191,15 @@ __global__ __launch_bounds__(SC_NT) void moe_dispatch_all_kernel(DispatchAllArgs
   const int e = blockIdx.x, tid = threadIdx.x, E = a.E, T = a.T, K = a.K, n = T * K;
   for (int i = tid; i < E; i += SC_NT) bins[i] = 0;
   __syncthreads();
-  for (int i = tid; i < n; i += SC_NT) atomicAdd(&bins[a.sel[i]], 1);
+  // Eight loads in flight a thread: one at a time their latencies add up (24,576 picks: 24.5 us for the kernel, 20.6 so).
+  for (int i0 = tid; i0 < n; i0 += 8 * SC_NT) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = i0 + u * SC_NT < n ? a.sel[i0 + u * SC_NT] : -1;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (v[u] >= 0) atomicAdd(&bins[v[u]], 1);
+  }
   __syncthreads();
   // Thread i stands for expert i (E <= SC_NT). Sums over the experts: rows and full tiles below e, full tiles in all,
   // remainder tiles ahead of e's, remainder tiles in all.
