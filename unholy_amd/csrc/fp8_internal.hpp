@@ -36,7 +36,8 @@ struct Fp8Parts {
 void launch_fp8_skinny(const Fp8GemmArgs& a, hipStream_t st);
 // M <= 64: one workgroup per 16-column tile, K split over its 8 waves (bandwidth-shaped).
 void launch_fp8_gemv(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts* parts = nullptr);
-// 16 < M <= 256 with fp32 scales: one workgroup per 32 x 32 output tile over the whole of K (N % 32, K <= 8192).
+// 16 < M <= 256 with fp32 scales and weights past 4 GiB: one workgroup per 32 x 32 output tile over the whole of K (N % 32,
+// K <= 8192).
 bool fp8_rows_fits(const Fp8GemmArgs& a);
 void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st);
 // The LDS-ring MFMA GEMM (N % 128, K % 128, ldc % 8; fp8_tiled_fits says whether a shape qualifies).
