@@ -240,7 +240,7 @@ def test_fp8_gemm_refuses_narrow_ldc():
 @pytest.mark.parametrize("M,N,K", [(17, 48, 128), (33, 80, 1152), (47, 4096, 256), (100, 4096, 256), (250, 4096, 256),
                                    (300, 4096, 384), (384, 4096, 256), (65, 192, 8192), (18, 32, 5248),
                                    (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256), (1100, 1024, 256),
-                                   (1, 200, 640), (16, 48, 8192), (9, 32768, 128), (70, 200, 256), (20, 64, 9216)])
+                                   (1, 200, 640), (16, 48, 8192), (9, 32768, 128), (70, 200, 256), (20, 64, 9216), (1170, 4096, 128)])
 def test_fp8_mid_sizes(M, N, K, f32):
     """gemm_w8a8_wmma / gemm_fp8_f32s against the oracle within the bf16 bar, C with a row stride past N
     and its columns past N untouched."""

@@ -103,7 +103,7 @@ def test_grouped_fp8w_shape_errors():
 @pytest.mark.parametrize("M,G,R,K", [(9, 8, 512, 256), (16, 8, 1024, 128), (30, 8, 1024, 256), (61, 8, 1024, 384),
                                      (100, 8, 1024, 128), (180, 8, 1024, 128), (250, 8, 1024, 256), (23, 5, 48, 1152),
                                      (70, 3, 96, 640), (12, 2, 16, 9216), (600, 8, 1024, 256), (1030, 16, 512, 128),
-                                     (1000, 8, 1024, 128)])
+                                     (1000, 8, 1024, 128), (1170, 4, 1024, 128)])
 def test_grouped_fp8w_mid_sizes(M, G, R, K):
     rng = np.random.default_rng(M * 5 + G * R + K)
     a, w, sw = _case(rng, M, G, R, K)
