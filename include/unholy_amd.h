@@ -345,7 +345,9 @@ int uh_mx_moe_forward(const uint16_t* x, const float* logits, int T, int K, int 
                       const uint8_t* const* tab, float limit, void* ws, size_t ws_bytes, uint16_t* out, int32_t* sel,
                       float* wt, void* stream);
 /* The same with stage events (6 hipEvent_t, recorded on `stream` before routing, after routing + dispatch, after
- * the input transform, after w1/w3 + SwiGLU, after w2, after the combine; NULL entries are skipped). */
+ * the input transform, after w1/w3 + SwiGLU, after w2, after the combine; NULL entries are skipped). Stages that share a
+ * launch end with it, so their events are recorded together: a step of one or two tokens may run as two launches,
+ * routing to SwiGLU (events 1, 2 and 3 behind it) and w2 + combine (events 4 and 5). */
 int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, int E, int D, int I,
                          const uint8_t* const* tab, float limit, void* ws, size_t ws_bytes, uint16_t* out, int32_t* sel,
                          float* wt, void* stream, void* const* events);

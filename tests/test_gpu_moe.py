@@ -7,7 +7,7 @@ import pytest
 import oracle
 from tests.helpers import from_bf16, max_abs_rms, max_rel, mx_weights, randn_bf16, rel_l2
 from unholy_amd import call
-from unholy_amd.device import DeviceBuffer, pointer_table, synchronize
+from unholy_amd.device import DeviceBuffer, Event, Stream, fill_random_bytes, pointer_table, synchronize
 
 pytestmark = pytest.mark.gpu
 
@@ -358,3 +358,36 @@ def test_moe_forward_few_tokens(T, E, K, D, I):
         assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2
     assert np.array_equal(sel.download((T, K), np.int32), sel_ref)
     np.testing.assert_allclose(wt.download((T, K), np.float32), wt_ref, rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("T", [1, 2, 3])
+def test_forward_stage_events(T):
+    """Each stage event of uh_mx_moe_forward_ev lies behind the work it stands for. One expert's w1 and w3 (80 MB and
+    more) take longer than their bytes at 8 TB/s, the card's nominal rate, 10 us and more, where two events
+    recorded back to back are 4 to 8 us apart: the event after w1 / w3 + SwiGLU comes later than that, and so does the
+    routing event where one launch routes and forms h (one or two tokens). sel and wt are there once event 1 is."""
+    E, K, D, I = 1, 1, 12288, 8192 if T == 1 else 6144
+    rng = np.random.default_rng(T)
+    keep, ptrs = [], []
+    for n in (D * I // 2, D * I // 32) * 3:
+        b = DeviceBuffer(n)
+        fill_random_bytes(b, n, len(keep), 119, 125)
+        keep.append(b)
+        ptrs.append(b)
+    tab = pointer_table(ptrs)
+    x, logits = dev(randn_bf16(rng, (T, D))), dev(rng.standard_normal((T, E), dtype=np.float32))
+    ws_bytes = call("uh_mx_moe_workspace_size", T, K, E, D, I)
+    ws, out, sel, wt = DeviceBuffer(ws_bytes), DeviceBuffer(T * D * 2), DeviceBuffer(T * K * 4), DeviceBuffer(T * K * 4)
+    ev, st = [Event() for _ in range(6)], Stream()
+    handles = (ctypes.c_void_p * 6)(*[e.handle for e in ev])
+    for _ in range(3):
+        call("uh_memset", sel.ptr, 0xFF, T * K * 4, st.handle)
+        call("uh_memset", wt.ptr, 0xFF, T * K * 4, st.handle)
+        call("uh_mx_moe_forward_ev", x, logits, T, K, E, D, I, tab, 10.0, ws, ws_bytes, out, sel, wt, st.handle, handles)
+        ev[1].synchronize()
+        assert np.array_equal(sel.download((T, K), np.int32), np.zeros((T, K), np.int32))
+        assert np.array_equal(wt.download((T, K), np.float32), np.ones((T, K), np.float32))
+        st.synchronize()
+    at = [ev[0].elapsed_ms(e) for e in ev]
+    assert all(b >= a for a, b in zip(at, at[1:])) and at[5] > 0, at
+    assert at[1 if T <= 2 else 3] > D * I * 17 / 16 / 8e12 * 1e3, at

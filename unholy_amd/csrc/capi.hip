@@ -825,9 +825,9 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     mark(0);
     const k::MoeTokenArgs tk{x, logits, T, K, E, D, I, tab, limit, s_sel, s_wt, w.row_expert, w.h, out};
     if (k::moe_token_fits(tk)) {  // one or two tokens: two launches
+      k::launch_moe_token_up(tk, st);  // routes (sel, wt), quantizes x and forms h: events 1, 2 and 3 follow it
       mark(1);
       mark(2);
-      k::launch_moe_token_up(tk, st);
       mark(3);
       k::launch_moe_token_down(tk, st);
       mark(4);
