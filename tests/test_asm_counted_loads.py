@@ -3,7 +3,8 @@ accounting and wait for them with counted vmcnt waits (unholy_amd/csrc/pipe.hpp 
 safe while the compiled code neither reads nor overwrites a destination register of such a load before a wait has
 retired it, on every path the code can take.
 
-(fp8_tiled_kernel's next-stage activation scale is one such load, issued ahead of the stage's ring loads.) This test
+(fp8_tiled_kernel's next-stage activation scale is one such load, issued ahead of the stage's ring loads; the first
+bf16 row pieces of fp8_kpart_kernel's quantizing form are another, ahead of the weights'.) This test
 compiles the kernels to gfx950 assembly, splits each kernel into basic blocks (labels, branches,
 s_endpgm) and follows every path through them, loop back-edges included, against an in-order model of the
 vector-memory counter: loads (and stores) retire oldest first, `s_waitcnt vmcnt(N)` leaves the newest N
@@ -166,6 +167,7 @@ def test_hazard_model_follows_a_loop_back_edge():
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 @pytest.mark.parametrize("src,name,count,load", [("fp8_gemm.hip", "fp8_rows_kernel", 8, "global_load_dwordx4"),
                                                  ("grouped_fp8w.hip", "grouped_fp8w_rows_kernel", 8, "global_load_dwordx4"),
+                                                 ("fp8_kpart.hip", "fp8_kpart_kernelILb1ELi1ELi1ELb1E", 1, "global_load_dwordx4"),
                                                  ("fp8_tiled.hip", "fp8_tiled_kernel", 4, "global_load_dword ")])
 def test_counted_loads_have_no_early_use(src, name, count, load, tmp_path):
     kernels = _kernel_asm(src, name, tmp_path)

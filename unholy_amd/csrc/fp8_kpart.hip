@@ -160,12 +160,10 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
         make_uint2(c0, c1);
     if (l == 0) xscale[blk * 16 + r] = sc;
   };
-  v4i x0 = {0, 0, 0, 0};
-  if constexpr (XQ)
-    if (n > 0) x0 = vload16(x_src(lane));
-  if (n > 0) issue(0);
-  if constexpr (XQ)
-    if (n > 0) {
+  if (n > 0) {
+    if constexpr (XQ) {  // one block of code from the untracked load to its wait: its register is never merged or moved
+      v4i x0 = vload16(x_src(lane));
+      issue(0);
       wait_vm<NL>();  // the rows' first pass; the weights stay in flight
       asm volatile("" : "+v"(x0));
       quant_item(lane, x0);
@@ -177,7 +175,10 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
         for (int i = 0; i < 4; ++i)
           if (base + 64 * i < xitems) quant_item(base + 64 * i + lane, x[i]);
       }
+    } else {
+      issue(0);
     }
+  }
   v4f acc[RB][CB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
