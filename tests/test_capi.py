@@ -55,6 +55,19 @@ def test_shape_errors_are_reported(call):
     assert msg in _lib.last_error()
 
 
+@pytest.mark.parametrize("T", [1, 2, 8, 16, 64, 100])
+@pytest.mark.parametrize("null", ["x", "tab", "ws", "out"])
+def test_forward_refuses_null_operands(T, null):
+    """Every step refuses a null operand before it launches anything (a kernel would read it)."""
+    K, E, D, I = 2, 8, 256, 128
+    p = {f: 4096 for f in ("x", "logits", "tab", "ws", "out")}  # never read
+    p[null] = None
+    f = _lib.lib().uh_mx_moe_forward
+    rc = f(p["x"], p["logits"], T, K, E, D, I, p["tab"], 10.0, p["ws"], 1 << 40, p["out"], None, None, None)
+    assert rc == -1
+    assert "null operand" in _lib.last_error()
+
+
 def test_cpp_dropin_caller_compiles_and_links(tmp_path):
     """A C++ caller compiles against include/unholy/kernels/*.hpp and links every drop-in symbol it uses from
     libunholy_amd.so (tests/cpp/build.sh into a temporary path; running it needs a GPU: tests/test_gpu_dropin.py)."""

@@ -817,6 +817,9 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     const MoeWs w = carve(static_cast<char*>(ws), T, K, E, D, I);
     if (ws_bytes < w.bytes) throw std::runtime_error("uh_mx_moe_forward: workspace too small");
     if (D % 128 || I % 128) throw std::runtime_error("uh_mx_moe_forward: D % 128, I % 128");
+    // Ahead of every launch: the steps that read x and tab first do so in kernels without checks of their own.
+    if (!x || !tab || !ws || !out) throw std::runtime_error("uh_mx_moe_forward: null operand");
+    if (!logits && T > 8) throw std::runtime_error("uh_mx_moe_forward: null logits");
     const hipStream_t st = S(stream);
     const int P = T * K;
     int32_t* s_sel = sel ? sel : w.sel;
@@ -824,7 +827,7 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     const auto t = [&](int m, int f) { return tab + size_t(2 * m + f) * E; };
     mark(0);
     const k::MoeTokenArgs tk{x, logits, T, K, E, D, I, tab, limit, s_sel, s_wt, w.row_expert, w.h, out};
-    if (k::moe_token_fits(tk)) {  // one or two tokens: two launches
+    if (logits && k::moe_token_fits(tk)) {  // one or two tokens: two launches
       k::launch_moe_token_up(tk, st);  // routes (sel, wt), quantizes x and forms h: events 1, 2 and 3 follow it
       mark(1);
       mark(2);
