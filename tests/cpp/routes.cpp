@@ -1,0 +1,43 @@
+// Prints the kernel that the library's dispatch chooses for each call described on stdin, one per line. Nothing is
+// launched and no pointer is read, so it runs without a GPU (tests/test_routes.py).
+//   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | rows | gemv | skinny
+//   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
+#include <cstdint>
+#include <iostream>
+#include <sstream>
+#include <string>
+
+#include "fp8_internal.hpp"
+
+using namespace unholy::kernels;
+
+static const uint8_t* at(uintptr_t offset) { return reinterpret_cast<const uint8_t*>(0x100000 + offset); }
+
+int main() {
+  static const char* const kDense[] = {"kpart", "tiled", "rows", "gemv", "skinny"};
+  static const char* const kGrouped[] = {"rows", "kpart", "gemv", "tiled", "ref"};
+  for (std::string line; std::getline(std::cin, line);) {
+    std::istringstream in(line);
+    std::string kind;
+    in >> kind;
+    if (kind == "dense") {
+      Fp8GemmArgs a{};
+      int f32 = 0;
+      uintptr_t ao = 0, wo = 0;
+      in >> a.M >> a.N >> a.K >> a.ldc >> f32 >> ao >> wo;
+      a.a = at(ao);
+      a.w = at(wo);
+      a.c = reinterpret_cast<uint16_t*>(0x100000);
+      if (f32) a.sa32 = a.sw32 = reinterpret_cast<const float*>(0x100000);
+      else a.sa8 = a.sw8 = at(0);
+      std::cout << kDense[int(fp8_route(a))] << "\n";
+    } else if (kind == "grouped") {
+      int M, G, R, K;
+      uintptr_t ao = 0, wo = 0;
+      in >> M >> G >> R >> K >> ao >> wo;
+      std::cout << kGrouped[int(grouped_route(at(ao), at(wo), M, G, R, K))] << "\n";
+    } else {
+      return 1;
+    }
+  }
+}

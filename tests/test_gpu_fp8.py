@@ -279,3 +279,43 @@ def test_gemv_w8a8_parts_matches_single_ranges(M, K):
         single = DeviceBuffer(M * n * 2)
         call("uh_gemv_w8a8", dq, dsa, w, s, single, n, M, n, K, None)
         assert np.array_equal(single.download((M, n), np.uint16), o.download((M, n), np.uint16))
+
+
+def _at_offset(a, off):
+    """A device copy of `a` starting `off` bytes past an aligned address: (buffer, address)."""
+    a = np.ascontiguousarray(a)
+    b = DeviceBuffer(a.nbytes + off)
+    call("uh_memcpy_h2d", b.ptr + off, a.ctypes.data, a.nbytes)
+    return b, b.ptr + off
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 200, 256), (16, 256, 4096), (40, 256, 512), (70, 256, 512)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_fp8_unaligned_operands(M, N, K, f32):
+    """Weights or activations 8 bytes off a 16-byte address (a tensor inside a checkpoint's flat buffer): the kernels with
+    plain loads, within the bf16 bar of the oracle; the fused and the multi-range forms on such weights too."""
+    rng = np.random.default_rng(M + K)
+    x = randn_bf16(rng, (M, K))
+    wq, sw = _w8a8_weights(rng, N, K)
+    if f32:
+        q, sa = oracle.act_quant_fp8_f32s(x)
+        sw = (rng.random(sw.shape, np.float32) + 0.5) * np.float32(2.0 ** -6)
+    else:
+        q, sa = oracle.act_quant_fp8(x)
+    ref = from_bf16(oracle.gemm_w8a8(q, sa, wq, sw)[0])
+    c, dsa, dsw = DeviceBuffer(M * N * 2), dev(sa), dev(sw)
+    for ao, wo in ((8, 0), (0, 8)):
+        (qb, qp), (wb, wp) = _at_offset(q, ao), _at_offset(wq, wo)
+        c.zero()
+        call("uh_gemm_fp8_f32s" if f32 else "uh_gemm_w8a8_wmma", qp, dsa, wp, dsw, c, N, M, N, K, None)
+        assert max_rel(from_bf16(c.download((M, N), np.uint16)), ref) <= 1e-2
+    if f32 and M <= 16:
+        c.zero()
+        call("uh_gemm_fp8_f32s_x", dev(x), K, wp, dsw, c, N, M, N, K, None)
+        assert max_rel(from_bf16(c.download((M, N), np.uint16)), ref) <= 1e-2
+    if not f32 and M <= 32:
+        c.zero()
+        arr = [np.array([v], np.uint64) for v in (wp, dsw.ptr, c.ptr)]
+        n = np.array([N], np.int32)
+        call("uh_gemv_w8a8_parts", dev(q), dsa, *[v.ctypes.data for v in arr], n.ctypes.data, n.ctypes.data, 1, M, K, None)
+        assert max_rel(from_bf16(c.download((M, N), np.uint16)), ref) <= 1e-2

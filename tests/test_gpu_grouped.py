@@ -113,3 +113,21 @@ def test_grouped_fp8w_mid_sizes(M, G, R, K):
     got = c.download((M * G * R + 64,), np.uint16)
     assert np.all(got[M * G * R:] == 0x7FC1)
     assert max_rel(from_bf16(got[:M * G * R].reshape(M, G, R)), from_bf16(ref16)) <= 1e-2
+
+
+@pytest.mark.parametrize("M,G,R,K", [(1, 8, 1024, 256), (12, 2, 128, 384), (200, 2, 64, 256), (5, 2, 40, 128)])
+def test_grouped_fp8w_unaligned_operands(M, G, R, K):
+    """Activations or weights 8 bytes off a 16-byte address: the kernels with plain loads."""
+    rng = np.random.default_rng(M + K)
+    a, w, sw = _case(rng, M, G, R, K)
+    ref = from_bf16(oracle.gemm_grouped_fp8w(a, w, sw, G, R)[0])
+    c, dsw = DeviceBuffer(M * G * R * 2), dev(sw)
+    for ao, wo in ((8, 0), (0, 8)):
+        bufs = []
+        for v, o in ((a, ao), (w, wo)):
+            b = DeviceBuffer(v.nbytes + o)
+            call("uh_memcpy_h2d", b.ptr + o, v.ctypes.data, v.nbytes)
+            bufs.append((b, b.ptr + o))
+        c.zero()
+        call("uh_gemm_grouped_fp8w_wmma", bufs[0][1], bufs[1][1], dsw, c, M, G, R, K, None)
+        assert max_rel(from_bf16(c.download((M, G, R), np.uint16)), ref) <= 1e-2

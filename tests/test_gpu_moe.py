@@ -391,3 +391,15 @@ def test_forward_stage_events(T):
     at = [ev[0].elapsed_ms(e) for e in ev]
     assert all(b >= a for a, b in zip(at, at[1:])) and at[5] > 0, at
     assert at[1 if T <= 2 else 3] > D * I * 17 / 16 / 8e12 * 1e3, at
+
+
+def test_forward_unaligned_workspace():
+    """A workspace 8 bytes off a 16-byte address: a step of 9 to 64 tokens keeps the GEMV (plain loads of its rows)."""
+    T, E, K, D, I = 20, 16, 6, 512, 256
+    rng = np.random.default_rng(T)
+    experts, bufs, tab, x, logits = _moe_case(rng, T, E, K, D, I)
+    out_ref, _ = oracle.moe_forward(x, *oracle.route_softmax(logits, K), experts, D, I, 10.0)
+    n = call("uh_mx_moe_workspace_size", T, K, E, D, I)
+    ws, out = DeviceBuffer(n + 8), DeviceBuffer(T * D * 2)
+    call("uh_mx_moe_forward", dev(x), dev(logits), T, K, E, D, I, tab, 10.0, ws.ptr + 8, n, out, None, None, None)
+    assert max_rel(from_bf16(out.download((T, D), np.uint16)), from_bf16(out_ref)) <= 1e-2

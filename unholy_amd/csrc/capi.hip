@@ -137,7 +137,9 @@ MoeWs carve(char* base, int T, int K, int E, int D, int I) {
     w.hh = reinterpret_cast<bf16*>(take(P * I * 2));
   } else if (base) {  // behind xa, in the bytes that only the fp8-code GEMMs use (K = 6, I = D / 2: room for it)
     char* const hh = reinterpret_cast<char*>(w.xq) + (size_t(T) * D * 2 + 255) / 256 * 256;
-    if (size_t(D) >= size_t(I) * 2 && hh + P * I * 2 <= codes_end) w.hh = reinterpret_cast<bf16*>(hh);
+    // (the GEMM loads xa and hh straight into LDS, 16 bytes a lane: a workspace with another alignment keeps the GEMV)
+    if (size_t(D) >= size_t(I) * 2 && hh + P * I * 2 <= codes_end && reinterpret_cast<uintptr_t>(base) % 16 == 0)
+      w.hh = reinterpret_cast<bf16*>(hh);
   }
   w.pair_out = reinterpret_cast<bf16*>(take(P * D * 2));
   w.bytes = o;

@@ -735,6 +735,32 @@ void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st) {
   else launch_fp8_rows_t<1>(a, st);
 }
 
+static size_t skinny_lds(const Fp8GemmArgs& a) {
+  const size_t rows = std::min(a.M, DN_MAXROWS);
+  return rows * (a.K + DN_PAD) + rows * (a.K / 128) * (a.sa32 ? 4 : 1);
+}
+
+Fp8Route fp8_route(const Fp8GemmArgs& a) {
+  const bool aligned = fp8_aligned(a.a, a.w);
+  if (fp8_kpart_fits(a))
+    return !fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a) ? Fp8Route::kpart : Fp8Route::tiled;
+  if (aligned && fp8_rows_fits(a)) return Fp8Route::rows;  // weights past 4 GiB
+  if (a.M <= 64) return Fp8Route::gemv;
+  // (unaligned operands whose rows do not fit the row groups' LDS stay with the tiled GEMM)
+  if (fp8_tiled_fits(a) && (aligned || skinny_lds(a) > 160 * 1024)) return Fp8Route::tiled;
+  return Fp8Route::skinny;
+}
+void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st) {
+  if (a.M > 0 && a.ldc < a.N) throw std::runtime_error("fp8 gemm: ldc < N");
+  switch (fp8_route(a)) {
+    case Fp8Route::kpart: return launch_fp8_kpart(a, st);
+    case Fp8Route::tiled: return launch_fp8_tiled(a, st);
+    case Fp8Route::rows: return launch_fp8_rows(a, st);
+    case Fp8Route::gemv: return launch_fp8_gemv(a, st);
+    case Fp8Route::skinny: return launch_fp8_skinny(a, st);
+  }
+}
+
 void launch_fp8_skinny(const Fp8GemmArgs& a0, hipStream_t st) {
   Fp8GemmArgs a = a0;
   if (a.M <= 0) return;
@@ -743,7 +769,7 @@ void launch_fp8_skinny(const Fp8GemmArgs& a0, hipStream_t st) {
   const bool f32s = a.sa32 != nullptr;
   if (f32s ? !a.sw32 : (!a.sa8 || !a.sw8)) throw std::runtime_error("fp8 gemm: scales");
   a.rows_cap = std::min(a.M, DN_MAXROWS);
-  const size_t lds = size_t(a.rows_cap) * (a.K + DN_PAD) + size_t(a.rows_cap) * (a.K / 128) * (f32s ? 4 : 1);
+  const size_t lds = skinny_lds(a);
   const dim3 grid(cdiv(cdiv(size_t(a.N), 16), DN_WAVES * DN_TN), cdiv(size_t(a.M), size_t(a.rows_cap)));
   if (f32s) {
     if (lds > 65536)

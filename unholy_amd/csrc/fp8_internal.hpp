@@ -57,8 +57,17 @@ bool grouped_kpart_fits(int M, int G, int R, int K);
 double grouped_kpart_us(int M, int G, int R, int K);
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st);
-// The K-part kernel or the tiled GEMM, by their estimated times; where neither fits (operands past 4 GiB, K > 8192) the row
-// tiles, the GEMV (M <= 64) or the row-group kernel.
+// The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits
+// (operands past 4 GiB, K > 8192) the row tiles, the GEMV (M <= 64) or the row-group kernel. The first three load operands
+// straight into LDS, 16 bytes a lane, and are kept to 16-byte aligned operands; the GEMV and the row groups take any.
+enum class Fp8Route { kpart, tiled, rows, gemv, skinny };
+Fp8Route fp8_route(const Fp8GemmArgs& a);
+inline bool fp8_aligned(const void* a, const void* w) {
+  return (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) % 16 == 0;
+}
 void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st);
+// The kernel of a grouped projection (grouped_fp8w.hip).
+enum class GroupedRoute { rows, kpart, gemv, tiled, ref };
+GroupedRoute grouped_route(const void* a, const void* w, int M, int G, int R, int K);
 
 }  // namespace unholy::kernels

@@ -417,13 +417,13 @@ int best_form(const Fp8GemmArgs& a) {
 }  // namespace
 
 bool fp8_kpart_fits(const Fp8GemmArgs& a) {
-  return a.M > 0 && a.N > 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET &&
+  return a.M > 0 && a.N > 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET && fp8_aligned(a.a, a.w) &&
          (a.sa32 || a.xa ? a.sw32 != nullptr : a.sa8 && a.sw8) && size_t(a.M) * a.K < (size_t(1) << 32) &&
          size_t(a.N) * a.K < (size_t(1) << 32);
 }
 bool fp8_kpart_parts_fits(const Fp8GemmArgs& a, const Fp8Parts& pp) {
   for (int i = 0; i < pp.n; ++i)
-    if (size_t(pp.N[i]) * a.K >= (size_t(1) << 32)) return false;
+    if (size_t(pp.N[i]) * a.K >= (size_t(1) << 32) || !fp8_aligned(a.a, pp.w[i])) return false;
   return a.M > 0 && a.M <= 32 && a.K <= 128 * KP_WAVES * 4 * NSET;
 }
 void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_t st) {

@@ -526,18 +526,32 @@ double tiled_us(int M, int G, int R, int K) {
                                                   : (w128 <= 448 ? 1.13 : 1.27 * double((w128 + 511) / 512));
   return 7.0 + K / 64 * stage;
 }
+}  // namespace
+
 // Up to 8 rows the row tiles' 32-column form while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part
 // kernel, 8 9.28 / 9.43, 16 10.9 / 10.1); else the K-part kernel or the tiled GEMM by their estimated times; then the
-// kernels for what neither takes (operands past 4 GiB, R % 16 != 0).
-void launch_fast(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
-                 hipStream_t st) {
+// kernels for what neither takes (operands past 4 GiB, R % 16 != 0). All but the GEMV and the reference order load
+// operands straight into LDS, 16 bytes a lane: operands that are not 16-byte aligned take those two.
+GroupedRoute grouped_route(const void* a, const void* w, int M, int G, int R, int K) {
+  if (!fp8_aligned(a, w)) return R % 16 == 0 ? GroupedRoute::gemv : GroupedRoute::ref;
   const bool few = M <= 8 && size_t(G) * R / 32 >= 256 && rows_fits(M, G, R, K), tiled = tiled_fits(G, R, K);
   if (!few && grouped_kpart_fits(M, G, R, K) && (!tiled || grouped_kpart_us(M, G, R, K) < tiled_us(M, G, R, K)))
-    launch_grouped_kpart(a, w, sw, c, M, G, R, K, st);
-  else if (rows_fits(M, G, R, K)) launch_rows(a, w, sw, c, M, G, R, K, st);
-  else if (gemv_fits(M, R) && !grouped_kpart_fits(M, G, R, K)) launch_gemv(a, w, sw, c, M, G, R, K, st);
-  else if (tiled) launch_tiled(a, w, sw, c, M, G, R, K, st);
-  else launch_ref(a, w, sw, c, M, G, R, K, st);  // shapes the fast kernels do not tile
+    return GroupedRoute::kpart;
+  if (rows_fits(M, G, R, K)) return GroupedRoute::rows;
+  if (gemv_fits(M, R) && !grouped_kpart_fits(M, G, R, K)) return GroupedRoute::gemv;
+  return tiled ? GroupedRoute::tiled : GroupedRoute::ref;
+}
+
+namespace {
+void launch_fast(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
+                 hipStream_t st) {
+  switch (grouped_route(a, w, M, G, R, K)) {
+    case GroupedRoute::rows: return launch_rows(a, w, sw, c, M, G, R, K, st);
+    case GroupedRoute::kpart: return launch_grouped_kpart(a, w, sw, c, M, G, R, K, st);
+    case GroupedRoute::gemv: return launch_gemv(a, w, sw, c, M, G, R, K, st);
+    case GroupedRoute::tiled: return launch_tiled(a, w, sw, c, M, G, R, K, st);
+    case GroupedRoute::ref: return launch_ref(a, w, sw, c, M, G, R, K, st);
+  }
 }
 
 }  // namespace

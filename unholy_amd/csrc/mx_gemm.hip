@@ -941,17 +941,6 @@ void launch_mx_gemm(const MxGemvArgs& a, int ntiles, int amode, hipStream_t st) 
 #undef UH_GM
 }
 
-void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st) {
-  if (a.M > 0 && a.ldc < a.N) throw std::runtime_error("fp8 gemm: ldc < N");
-  if (fp8_kpart_fits(a)) {  // or the tiled GEMM, by the estimated times of the two
-    if (!fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a)) launch_fp8_kpart(a, st);
-    else launch_fp8_tiled(a, st);
-  } else if (fp8_rows_fits(a)) launch_fp8_rows(a, st);  // weights past 4 GiB
-  else if (a.M <= 64) launch_fp8_gemv(a, st);
-  else if (fp8_tiled_fits(a)) launch_fp8_tiled(a, st);
-  else launch_fp8_skinny(a, st);
-}
-
 namespace {
 MxGemvArgs gemm_args(const bf16* xa, const uint8_t* q, const uint8_t* qs, int K, const Exl3Tile* tiles,
                      const uint8_t* const* w_tab, const uint8_t* const* s_tab, bf16* out, int ldo, int N,
