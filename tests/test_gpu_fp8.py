@@ -319,3 +319,29 @@ def test_fp8_unaligned_operands(M, N, K, f32):
         n = np.array([N], np.int32)
         call("uh_gemv_w8a8_parts", dev(q), dsa, *[v.ctypes.data for v in arr], n.ctypes.data, n.ctypes.data, 1, M, K, None)
         assert max_rel(from_bf16(c.download((M, N), np.uint16)), ref) <= 1e-2
+
+
+@pytest.mark.parametrize("M,N,K,off", [(2, 65536, 1024, 0), (16, 256, 1152, 8), (7, 200, 8192, 8), (1, 128, 128, 8)])
+def test_few_rows_same_bits_by_every_kernel(M, N, K, off):
+    """gemm_fp8_f32s_x and gemm_fp8_f32s, gemv_w8a8_parts and gemv_w8a8, bit for bit: at a shape whose estimate is best for
+    the tiled GEMM, and with weights `off` bytes off a 16-byte address in one call of each pair (the GEMV there, the K-part
+    kernel for the aligned copy)."""
+    rng = np.random.default_rng(M + N)
+    x = randn_bf16(rng, (M, K))
+    wq = rng.integers(0, 0x7F, (N, K), dtype=np.uint8)
+    sw32 = (rng.random(((N + 127) // 128, K // 128), np.float32) + 0.5) * np.float32(2.0 ** -6)
+    sw8 = rng.integers(118, 126, sw32.shape, dtype=np.uint8)
+    (b0, w0), (b1, w1) = _at_offset(wq, 0), _at_offset(wq, off)
+    dx, d32, d8 = dev(x), dev(sw32), dev(sw8)
+    c, ref = DeviceBuffer(M * N * 2), DeviceBuffer(M * N * 2)
+    q, sa = DeviceBuffer(M * K), DeviceBuffer(M * (K // 128) * 4)
+    call("uh_act_quant_fp8_f32s", dx, K, q, sa, M, K, 128, None)
+    call("uh_gemm_fp8_f32s", q, sa, w0, d32, ref, N, M, N, K, None)
+    call("uh_gemm_fp8_f32s_x", dx, K, w1, d32, c, N, M, N, K, None)
+    assert np.array_equal(c.download((M, N), np.uint16), ref.download((M, N), np.uint16))
+    call("uh_act_quant_fp8", dx, K, q, sa, M, K, 128, None)
+    call("uh_gemv_w8a8", q, sa, w0, d8, ref, N, M, N, K, None)
+    arr = [np.array([v], np.uint64) for v in (w1, d8.ptr, c.ptr)]
+    n = np.array([N], np.int32)
+    call("uh_gemv_w8a8_parts", q, sa, *[v.ctypes.data for v in arr], n.ctypes.data, n.ctypes.data, 1, M, K, None)
+    assert np.array_equal(c.download((M, N), np.uint16), ref.download((M, N), np.uint16))

@@ -47,3 +47,12 @@ def test_unaligned_operands_avoid_direct_loads(routes):
         assert not bad, bad[:5]
     assert set(routes([f"{l} 0 0" for l in dense])) <= {"kpart", "tiled"}
     assert set(routes([f"{l} 0 16" for l in grouped])) <= DIRECT
+
+
+def test_few_rows_never_change_the_order_of_sums(routes):
+    """gemm_fp8_f32s of up to 16 rows equals gemm_fp8_f32s_x bit for bit, gemv_w8a8 of up to 32 every column range of
+    gemv_w8a8_parts: at no shape may the plain entry points take the tiled GEMM, which adds in another order."""
+    lines = [f"dense {m} {n} {k} {n} {f} 0 0" for f, ms in ((1, (1, 5, 16)), (0, (1, 8, 17, 32))) for m in ms
+             for n in (128, 1024, 4096, 8192, 32768, 65536, 129280) for k in (128, 256, 512, 1024, 2048, 4096, 8192, 9216)]
+    bad = [(l, a) for l, a in zip(lines, routes(lines)) if a not in ("kpart", "gemv")]
+    assert not bad, bad[:5]

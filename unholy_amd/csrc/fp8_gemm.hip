@@ -273,11 +273,12 @@ __global__ __launch_bounds__(DN_NT) void fp8_skinny_kernel(Fp8GemmArgs a) {
 // ---- fp8 dense, small M (<= 64 rows), what the K-part kernel does not take (K > 8192): bandwidth-shaped ----
 // One workgroup per 16-column tile; its 8 waves split K (wave w takes 128-blocks w * per .. + per - 1), so the grid
 // covers every CU and each CU keeps 8 waves x 64 lanes x 128 B of weights in flight (four 128-blocks per wave are
-// loaded before any is used). Lane (nl, g) reads 32 weight bytes of column n0 + nl at inputs 32g .. + 31 of a block
-// and the same inputs of activation row nl (row tile mt: rows 16 mt + nl) from global memory (A is small and
+// loaded before any is used). Lane (nl, g) reads 32 weight bytes of column n0 + nl, inputs 16 g .. + 15 and 64 + 16 g .. + 15
+// of a block, and the same inputs of activation row nl (row tile mt: rows 16 mt + nl) from global memory (A is small and
 // cache-resident), dequantizes both exactly to bf16 (e8m0 scales folded in) and issues 16x16x32 bf16 MFMAs. With fp32
 // scales each block's MFMA chain starts from zero and is folded as acc += raw * (sa * sw). The 8 partial tiles are
-// summed in wave order through LDS.
+// summed in wave order through LDS. K parts, inputs of an MFMA and order of sums are those of fp8_kpart_kernel: the two give
+// the same bits, and a call that one of them takes may be compared with a call that the other takes.
 constexpr int FV_WAVES = 8, FV_CHUNK = 4;
 
 // XQ: A arrives as bf16 rows (a.xa). The workgroup first quantizes its M rows into LDS as act_quant_fp8_f32s does
@@ -306,7 +307,7 @@ __global__ __launch_bounds__(64 * FV_WAVES) void fp8_gemv_kernel(Fp8GemmArgs a, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = tile * 16, n = min(n0 + nl, N - 1), nb = n0 / 128;  // a 16-column tile lies in one 128-block
   const int per = (KS + FV_WAVES - 1) / FV_WAVES, b0 = min(KS, wave * per), b1 = min(KS, b0 + per);
-  const uint8_t* wrow = a.w + size_t(n) * K + g * 32;
+  const uint8_t* wrow = a.w + size_t(n) * K + g * 16;
   v4f acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(64 * FV_WAVES) void fp8_gemv_kernel(Fp8GemmArgs a, 
     for (int u = 0; u < FV_CHUNK; ++u) {
       const int kb = min(kc + u, b1 - 1);
       b[u][0] = *reinterpret_cast<gptr<v4i>>(as_global(wrow + kb * 128));
-      b[u][1] = *reinterpret_cast<gptr<v4i>>(as_global(wrow + kb * 128 + 16));
+      b[u][1] = *reinterpret_cast<gptr<v4i>>(as_global(wrow + kb * 128 + 64));
       swv[u] = F32S ? a.sw32[size_t(nb) * KS + kb] : e8m0_to_f32(a.sw8[size_t(nb) * KS + kb]);
     }
   };
@@ -377,9 +378,9 @@ __global__ __launch_bounds__(64 * FV_WAVES) void fp8_gemv_kernel(Fp8GemmArgs a, 
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           const int r = min(mt * 16 + nl, M - 1);
-          const uint8_t* ap = a.a + size_t(r) * K + kb * 128 + g * 32;
+          const uint8_t* ap = a.a + size_t(r) * K + kb * 128 + g * 16;
           aq[u][mt][0] = *reinterpret_cast<gptr<v4i>>(as_global(ap));
-          aq[u][mt][1] = *reinterpret_cast<gptr<v4i>>(as_global(ap + 16));
+          aq[u][mt][1] = *reinterpret_cast<gptr<v4i>>(as_global(ap + 64));
           sav[u][mt] = F32S ? 1.0f : e8m0_to_f32(a.sa8[size_t(r) * KS + kb]);
         }
         if constexpr (kRowScales)
@@ -392,9 +393,9 @@ __global__ __launch_bounds__(64 * FV_WAVES) void fp8_gemv_kernel(Fp8GemmArgs a, 
 #pragma unroll
       for (int u = 0; u < FV_CHUNK; ++u) {
         const int kb = min(kc + u, b1 - 1);
-        const uint8_t* ap = xq_lds + size_t(min(nl, M - 1)) * K + kb * 128 + g * 32;
+        const uint8_t* ap = xq_lds + size_t(min(nl, M - 1)) * K + kb * 128 + g * 16;
         aq[u][0][0] = *reinterpret_cast<const v4i*>(ap);
-        aq[u][0][1] = *reinterpret_cast<const v4i*>(ap + 16);
+        aq[u][0][1] = *reinterpret_cast<const v4i*>(ap + 64);
 #pragma unroll
         for (int i = 0; i < 4; ++i) sa32v[u][i] = sl[min(4 * g + i, M - 1) * KS + kb];
       }
@@ -742,8 +743,11 @@ static size_t skinny_lds(const Fp8GemmArgs& a) {
 
 Fp8Route fp8_route(const Fp8GemmArgs& a) {
   const bool aligned = fp8_aligned(a.a, a.w);
+  // Rows that the fused and the multi-range entry points take: the K-part kernel or the GEMV, whose results are equal bit for
+  // bit (the tiled GEMM adds in another order: 65536 x 1024, M = 1 19.3 us there, 23.2 with the K-part kernel).
+  const bool same_bits = a.M <= (a.sa32 ? 16 : 32);
   if (fp8_kpart_fits(a))
-    return !fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a) ? Fp8Route::kpart : Fp8Route::tiled;
+    return same_bits || !fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a) ? Fp8Route::kpart : Fp8Route::tiled;
   if (aligned && fp8_rows_fits(a)) return Fp8Route::rows;  // weights past 4 GiB
   if (a.M <= 64) return Fp8Route::gemv;
   // (unaligned operands whose rows do not fit the row groups' LDS stay with the tiled GEMM)
