@@ -66,6 +66,48 @@ __device__ __forceinline__ void kp_reduce(const v4f (&acc)[RB][CB], uint8_t* sme
   }
 }
 
+// One operand of a tile for N direct loads of RPL rows each: `rows` rows of `stride` bytes from row row0 of b on, `width`
+// bytes of each at byte k, lane l taking the 16 bytes at piece(i) of row l / (64 / RPL) of load i. Rows past the tile repeat
+// its last, or that row's end: in bounds, and their results are not stored.
+// HOLD: an offset register per load. Without it load i's rows go into the scalar base, a few scalar instructions a load, and
+// two lane offsets serve them all (piece(i) is then piece(i % 2)): the largest tiles have no registers for 20 offsets. (With
+// them 6 x 4 and the grouped 8 x 4 spilled some, and every reload waited for the direct loads in flight: 384 x 4096 x
+// 4096 21.9 us, 19.6 so; fp32 scales, 5 x 4, 300 rows 18.7, 18.0; grouped 512 x 8192 x 4096 49.3, 47.7. The smaller
+// tiles are up to 3% faster with them.)
+template <int RPL, int N, bool HOLD>
+struct KpRows {
+  const uint8_t* base;
+  uint32_t stride, last, end, lane_off[2];
+  uint32_t off[HOLD && N ? N : 1];
+  template <class Piece>
+  __device__ __forceinline__ KpRows(const void* b, size_t row0, uint32_t stride_, int rows, int width, const Piece& piece)
+      : base(static_cast<const uint8_t*>(b) + row0 * stride_), stride(stride_) {
+    const int q = int(threadIdx.x & 63) / (64 / RPL);
+    if constexpr (HOLD) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) off[i] = uint32_t(min(i * RPL + q, rows - 1)) * stride + piece(i);
+    } else {
+      for (int i = 0; i < 2; ++i) lane_off[i] = uint32_t(q) * stride + piece(i);
+      last = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t((rows - 1) / RPL * RPL) * stride)));
+      end = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(rows - 1) * stride + uint32_t(width - 16))));
+    }
+  }
+  __device__ __forceinline__ void load(size_t k, uint32_t lds) const {
+    if constexpr (HOLD) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) dma16(base + k, off[i], lds + uint32_t(i * 1024));
+    } else {
+      uint32_t lst = last, e = end;  // opaque: the addresses are formed in this step, not ahead of the loop (in registers)
+      asm volatile("" : "+s"(lst), "+s"(e));
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const uint32_t at = min(uint32_t(i * RPL) * stride, lst);
+        dma16(base + k + at, min(lane_off[i % 2], e - at), lds + uint32_t(i * 1024));
+      }
+    }
+  }
+};
+
 // XQ (fp32 scales, one row block): A arrives as bf16 rows (a.xa), quantized here as act_quant_fp8_f32s does (s = max(amax,
 // 1e-4) * fp32(1/448), codes e4m3(x / s); 8 values per lane, a block's amax a DPP row max over 16 lanes). Each wave
 // quantizes the rows of its own K part into its own LDS, behind its first weight loads: no wave waits for another.
@@ -122,18 +164,14 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
   uint8_t* const xcodes = smem + KP_WAVES * SLOT + wave * (per * (2048 + 64));
   float* const xscale = reinterpret_cast<float*>(xcodes + per * 2048);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(slot));
-  uint32_t off[NL];
-#pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int r = 8 * i + (lane >> 3), p = (lane & 7) ^ ((r >> 1) & 7);
-    // rows and columns past the tile repeat its last (their results are not stored)
-    off[i] = (i < 2 * AB ? uint32_t(row0 + min(r, Mt - 1)) : uint32_t(min(col0 + r - 16 * AB, N - 1))) * uint32_t(K) +
-             uint32_t(p * 16);
-  }
+  const auto piece = [&](int i) { return uint32_t(((lane & 7) ^ (lane >> 4) ^ (i & 1 ? 4 : 0)) * 16); };
+  constexpr bool HOLD = RB * CB <= (F32S ? 16 : 20);
+  const KpRows<8, 2 * AB, HOLD> arows(a.a, row0, K, Mt, 128, piece);
+  const KpRows<8, 2 * CB, HOLD> wrows(a.w, col0, K, min(16 * CB, N - col0), 128, piece);
   const auto issue = [&](int c) {
     const size_t k = size_t(b0 + c) * 128;
-#pragma unroll
-    for (int i = 0; i < NL; ++i) dma16(i < 2 * AB ? a.a + k : a.w + k, off[i], lds0 + uint32_t(i * 1024));
+    arows.load(k, lds0);
+    wrows.load(k, lds0 + uint32_t(AB * 2048));
   };
   // Item it = (row, block, piece of 8 values), 16 lanes a block.
   const int xitems = M * n * 16;
@@ -306,25 +344,20 @@ __global__ __launch_bounds__(64 * KP_WAVES) __attribute__((amdgpu_waves_per_eu(2
   float swv = e8m0_to_f32(sw[size_t(col0 / 128) * KS + min(b0 + lane, KS - 1)]);
   uint8_t* const slot = smem + wave * T::SLOT;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(slot));
-  uint32_t aoff[T::NA], woff[T::NW];
-#pragma unroll
-  for (int i = 0; i < T::NA; ++i) {
-    constexpr int PR = 64 / T::AR;  // pieces per row
-    const int r = T::AR * i + lane / PR, p = (lane % PR) ^ T::aswz(r & 15);
-    aoff[i] = (uint32_t(row0 + min(r, Mt - 1)) * uint32_t(G) + uint32_t(grp)) * uint32_t(K) * 2u + uint32_t(p * 16);
-  }
-#pragma unroll
-  for (int i = 0; i < T::NW; ++i) {
-    constexpr int PR = 64 / T::WR;
-    const int r = T::WR * i + lane / PR, p = (lane % PR) ^ T::wswz(r & 15);
-    woff[i] = uint32_t(col0 + r) * uint32_t(K) + uint32_t(p * 16);
-  }
+  constexpr int AP = 64 / T::AR, WP = 64 / T::WR;  // pieces per row
+  const auto apiece = [&](int i) {
+    return uint32_t(((lane % AP) ^ T::aswz(lane / AP) ^ T::aswz(i * T::AR & 15)) * 16);
+  };
+  const auto wpiece = [&](int i) {
+    return uint32_t(((lane % WP) ^ T::wswz(lane / WP) ^ T::wswz(i * T::WR & 15)) * 16);
+  };
+  constexpr bool HOLD = RB < 8;
+  const KpRows<T::AR, T::NA, HOLD> arows(a + size_t(grp) * K, row0, uint32_t(G) * uint32_t(K) * 2u, Mt, 2 * KB, apiece);
+  const KpRows<T::WR, T::NW, HOLD> wrows(w, col0, K, 16 * CB, KB, wpiece);
   const auto issue = [&](int s) {
     const size_t k = size_t(b0) * 128 + size_t(s) * KB;
-#pragma unroll
-    for (int i = 0; i < T::NW; ++i) dma16(w + k, woff[i], lds0 + uint32_t(RB * T::AB + i * 1024));
-#pragma unroll
-    for (int i = 0; i < T::NA; ++i) dma16(a + k, aoff[i], lds0 + uint32_t(i * 1024));
+    wrows.load(k, lds0 + uint32_t(RB * T::AB));
+    arows.load(2 * k, lds0);
   };
   if (n > 0) issue(0);
   v4f acc[RB][CB];
