@@ -19,5 +19,5 @@ def test_kpart_forms_do_not_spill(tmp_path):
                     "-packed-fp32-ops", "-I", os.path.join(ROOT, "include"), "-I", csrc, "--cuda-device-only", "-S",
                     os.path.join(csrc, "fp8_kpart.hip"), "-o", str(out)], check=True, capture_output=True)
     meta = re.findall(r"\.name:\s+(_Z\S*kpart_kernel\S*).*?\.vgpr_spill_count:\s+(\d+)", out.read_text(), re.S)
-    assert len(meta) == 21
+    assert len(meta) == 22
     assert [m for m in meta if int(m[1])] == []

@@ -56,3 +56,31 @@ def test_few_rows_never_change_the_order_of_sums(routes):
              for n in (128, 1024, 4096, 8192, 32768, 65536, 129280) for k in (128, 256, 512, 1024, 2048, 4096, 8192, 9216)]
     bad = [(l, a) for l, a in zip(lines, routes(lines)) if a not in ("kpart", "gemv")]
     assert not bad, bad[:5]
+
+
+# One call with both kernels (gfx950, us, graph replays over weights that do not fit a cache): rows, N (G, R) x K, the K-part
+# kernel's best form, the tiled GEMM. Each differs by more than a tenth.
+MEASURED_DENSE = [
+    (300, 4096, 4096, 0, 17.4, 26.6), (384, 4096, 4096, 0, 19.9, 27.7), (1000, 4096, 4096, 0, 52.6, 39.3),
+    (2049, 4096, 4096, 0, 106.0, 83.2), (2176, 4096, 4096, 0, 108.9, 83.4), (2304, 4096, 4096, 0, 110.9, 83.5),
+    (2560, 4096, 4096, 0, 129.1, 85.1), (300, 4096, 4096, 1, 18.0, 27.2), (384, 4096, 4096, 1, 21.4, 27.7),
+    (2049, 4096, 4096, 1, 114.4, 96.7), (2304, 4096, 4096, 1, 121.1, 97.5), (512, 4096, 8192, 0, 46.7, 53.0),
+    (1024, 4096, 8192, 0, 89.5, 73.5), (2176, 4096, 8192, 0, 186.5, 163.8), (2560, 4096, 8192, 0, 226.4, 165.7),
+    (2304, 4096, 8192, 1, 210.9, 188.0), (64, 8192, 1024, 0, 6.0, 9.5), (300, 8192, 1024, 0, 15.7, 11.1),
+    (768, 2048, 4096, 0, 19.5, 27.7), (2304, 2048, 4096, 1, 62.5, 51.1), (64, 32768, 1024, 1, 16.3, 13.4),
+    (256, 5120, 5120, 0, 23.5, 33.0), (2100, 5120, 5120, 1, 173.7, 125.9), (1000, 1152, 4096, 0, 18.8, 24.2),
+    (2000, 1152, 4096, 0, 37.8, 33.1)]
+MEASURED_GROUPED = [
+    (384, 8, 1024, 4096, 39.5, 66.5), (1024, 8, 1024, 4096, 95.0, 76.7), (2049, 8, 1024, 4096, 260.8, 183.3),
+    (2304, 8, 1024, 4096, 276.0, 186.9), (768, 4, 1024, 4096, 37.9, 66.3), (2049, 4, 1024, 4096, 123.8, 89.2),
+    (384, 8, 1024, 2048, 24.2, 32.0), (2304, 8, 1024, 2048, 157.6, 97.6), (64, 32, 1024, 4096, 42.8, 66.8),
+    (256, 16, 512, 1024, 11.4, 17.7), (2100, 16, 512, 1024, 86.3, 54.0),
+    (2100, 2, 2048, 4096, 120.8, 89.0), (2300, 7, 1152, 4096, 240.4, 194.9)]
+
+
+def test_the_estimates_choose_the_measured_winner(routes):
+    dense = [(f"dense {m} {n} {k} {n} {f} 0 0", kp, t) for m, n, k, f, kp, t in MEASURED_DENSE]
+    grouped = [(f"grouped {m} {g} {r} {k} 0 0", kp, t) for m, g, r, k, kp, t in MEASURED_GROUPED]
+    answers = routes([l for l, _, _ in dense + grouped])
+    bad = [(l, a) for (l, kp, t), a in zip(dense + grouped, answers) if a != ("kpart" if kp < t else "tiled")]
+    assert not bad, bad

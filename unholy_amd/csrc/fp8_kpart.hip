@@ -1,4 +1,4 @@
-// Dense fp8 GEMM for up to ~700 rows: C[M, N] (bf16) = A[M, K] (e4m3) x W[N, K]^T (e4m3), per-128 scales
+// Dense fp8 GEMM for up to ~700 rows at 4096 x 4096: C[M, N] (bf16) = A[M, K] (e4m3) x W[N, K]^T (e4m3), per-128 scales
 // (e8m0 or fp32, as fp8_tiled.hip).
 //
 // What bounds these sizes is getting each CU's share of W and A to it: 4096 x 4096 weights are 64 KB per CU, and a
@@ -424,26 +424,32 @@ void launch_g(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* 
 }  // namespace
 
 namespace {
-// The forms (16-row blocks x 16-column blocks), and what a launch of each takes (us, 16 < M <= 1024 and the shapes of
-// the model's projections, with act_quant): every round of 256 workgroups reads (RB + CB) rows and columns of K; a round
-// past the first adds its start-up and the reduction, less where two or three workgroups share a CU. 64 x 4096 x 4096
-// (M x N x K) 12.1 measured, 300 x 4096 x 4096 22.2, 512 32.8, 768 46.4, 600 x 4096 x 8192 60, 200 x 8192 x 1024 16.3,
-// 20 x 32768 x 1024 14.2 as 2 x 2 and 17.9 as 4 x 4.
+// The forms (16-row blocks x 16-column blocks), and what a launch of each takes, us: `start` (the launch, the first loads and
+// the reduction) and `read` per 1,000 inputs (each workgroup's rows and columns of K) for a round of 256 workgroups, `next`
+// more for a round past the first, and `miss` per MB that an XCD's 32 workgroups in flight read from beyond its L2: their
+// row tiles (`abytes` a value) and column blocks. Fitted to 2,900 launches of the dense forms (K = 640 to 8192, N = 640 to
+// 32768, M = 17 to 4096, up to 6 rounds; fp32 scales take 1.035 times as long) and 830 of the grouped ones: rms 6% and 9%.
+// With the tiled GEMM's estimate (fp8_tiled_us) it picks a kernel that is 0.1% slower than the best on average over 990
+// dense calls measured with each, 8% at worst; grouped (tiled_us) 0.2%, 12%.
 struct KpForm {
   int rb, cb;
-  double read, next;  // RB + CB, more where the registers leave less in flight; the cost of a further round
+  double start, next, read;
 };
-constexpr KpForm kForms[] = {{1, 1, 2.0, 0.8}, {2, 1, 3.0, 1.0}, {2, 2, 4.0, 1.2}, {4, 2, 6.0, 3.0},
-                             {4, 4, 9.0, 3.5}, {5, 4, 10.5, 3.5}, {6, 4, 13.0, 3.5}};
+double launch_us(const KpForm& f, int M, size_t N, int K, int abytes, double miss) {
+  const size_t rt = (size_t(M) + 16 * f.rb - 1) / (16 * f.rb), wg = rt * cdiv(N, 16 * f.cb), rounds = (wg + 255) / 256;
+  const size_t xcd = std::min<size_t>(32, (wg + 7) / 8);
+  const double rows = 16.0 * (double(abytes * f.rb) * double(std::min(rt, xcd)) + f.cb * double((xcd + rt - 1) / rt));
+  return f.start + double(rounds - 1) * f.next + double(rounds) * K * (f.read * 1e-3 + miss * rows * 1e-6);
+}
+constexpr KpForm kForms[] = {{1, 1, 2.97, 0.0, 0.46}, {2, 1, 3.20, 0.05, 0.70}, {2, 2, 3.34, 0.46, 0.87},
+                             {4, 2, 3.63, 2.20, 1.48}, {4, 4, 4.76, 3.20, 2.03}, {5, 4, 5.64, 3.99, 2.43},
+                             {6, 4, 6.07, 4.40, 2.93}};
 double form_us(const Fp8GemmArgs& a, const KpForm& f) {
-  const size_t wg = size_t((a.M + 16 * f.rb - 1) / (16 * f.rb)) * cdiv(size_t(a.N), 16 * f.cb);
-  const double rounds = double((wg + 255) / 256);
-  return 7.0 + (rounds - 1.0) * f.next + rounds * f.read * a.K * 0.00034;
+  return launch_us(f, a.M, size_t(a.N), a.K, 1, 0.23) * (a.sa32 ? 1.035 : 1.0);
 }
 int best_form(const Fp8GemmArgs& a) {
-  const int forms = a.sa32 ? 6 : 7;  // 6 x 4 with fp32 scales spills
   int best = 0;
-  for (int i = 1; i < forms; ++i)
+  for (int i = 1; i < 7; ++i)
     if (form_us(a, kForms[i]) < form_us(a, kForms[best])) best = i;
   return best;
 }
@@ -476,7 +482,8 @@ void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
       case 2: return launch_t<true, 2, 2>(a, st);
       case 3: return launch_t<true, 4, 2>(a, st);
       case 4: return launch_t<true, 4, 4>(a, st);
-      default: return launch_t<true, 5, 4>(a, st);
+      case 5: return launch_t<true, 5, 4>(a, st);
+      default: return launch_t<true, 6, 4>(a, st);
     }
   }
   switch (best_form(a)) {
@@ -492,15 +499,11 @@ void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
 
 // ---- grouped ---------------------------------------------------------------------------------------------------------
 namespace {
-// The forms and what a launch takes (us): every round of 256 workgroups reads 16 (2 RB + CB) K bytes a workgroup. G R =
-// 8192, K = 4096: M = 16 10.1 measured (1 x 2), 32 12.9 (2 x 2), 64 14.7 (2 x 4), 128 19.6 (4 x 4), 256 30.9 (8 x 4), 512
-// 54.9 (8 x 4, two rounds).
-constexpr KpForm kGForms[] = {{1, 1, 3.0, 0.0}, {1, 2, 4.0, 0.0},  {2, 2, 6.0, 0.0}, {2, 4, 8.0, 0.0},
-                              {4, 4, 12.0, 0.0}, {6, 4, 16.0, 0.0}, {8, 4, 20.0, 0.0}};
-double gform_us(int M, int N, int K, const KpForm& f) {
-  const size_t wg = size_t((M + 16 * f.rb - 1) / (16 * f.rb)) * (N / (16 * f.cb));
-  return 4.8 + double((wg + 255) / 256) * f.read * K * 0.00032;
-}
+// As above; the rows are bf16.
+constexpr KpForm kGForms[] = {{1, 1, 3.19, 0.06, 0.57}, {1, 2, 2.93, 0.32, 0.83}, {2, 2, 3.16, 1.46, 1.15},
+                              {2, 4, 3.73, 1.26, 1.66}, {4, 4, 4.89, 1.75, 2.34}, {6, 4, 6.21, 3.10, 2.78},
+                              {8, 4, 6.75, 3.81, 3.76}};
+double gform_us(int M, int N, int K, const KpForm& f) { return launch_us(f, M, size_t(N), K, 2, 0.41); }
 int best_gform(int M, int G, int R, int K) {
   int best = 0;
   for (int i = 1; i < 7; ++i)

@@ -257,17 +257,20 @@ bool fp8_tiled_fits(const Fp8GemmArgs& a) {
   return a.N % 128 == 0 && a.K % 128 == 0 && a.ldc % 8 == 0 && FpTile<128>::lds(a.K, a.sa32 != nullptr) <= 80 * 1024;
 }
 
-// What a launch takes (us, with act_quant, K = 1024..8192; fp32 scales x 1.07): per 128-input stage 0.82 / 1.06 us (64
-// columns, up to / past 256 workgroups), 1.15 (128 columns, 256 workgroups), 1.75 up to 512, 2.06 per 512 past that.
-// 512 x 4096 x 4096 (M x N x K) 33.9 measured, 768 41.2, 1000 43.7, 1500 64.2, 2000 71.5, 300 x 8192 x 1024 14.8.
+// What a launch takes, us (K = 640 to 8192; fp32 scales 1.06 times that): a time per 128-input stage by the number w of
+// workgroups of 128 columns. Up to 255 they run as twice as many of 64 columns, 256 are one a CU, 512 two a CU; past that full
+// rounds of 512 and a last one that costs what its own workgroups do: a CU with one of them runs its stages faster than
+// with two. M x 4096 x 4096, measured / this: 512 28.2 / 26.4, 1000 38.9 / 37.9, 2000 64 / 60, 2049 84 / 83, 3000 91 / 88, 4096
+// 119 / 118.
 double fp8_tiled_us(const Fp8GemmArgs& a) {
-  const size_t w = size_t(a.N / 128) * ((a.M + 127) / 128);
-  const double stage = w <= 128   ? 0.82
-                       : w < 256  ? 1.06
-                       : w == 256 ? 1.15
-                       : w < 512  ? 1.75
-                                  : 2.06 * double((w + 511) / 512);
-  return 7.0 + a.K / 128 * stage * (a.sa32 ? 1.07 : 1.0);
+  const size_t w = size_t(a.N / 128) * ((size_t(a.M) + 127) / 128), rem = w % 512;
+  const double first = rem == 0     ? 0.0
+                       : rem <= 128 ? 0.74
+                       : rem < 256  ? 0.92 + 0.0012 * double(rem - 128)
+                       : rem == 256 ? 1.10
+                                    : 1.50 + 0.3 / 256 * double(rem - 256);
+  const double last = rem == 0 ? 0.0 : rem <= 128 ? 0.72 : rem <= 256 ? 0.85 : first;
+  return 2.7 + a.K / 128 * (w < 512 ? first : 1.8 * double(w / 512) + last) * (a.sa32 ? 1.06 : 1.0);
 }
 
 void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st) {

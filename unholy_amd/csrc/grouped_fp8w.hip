@@ -507,24 +507,29 @@ void launch_tiled_t(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c,
   kern<<<dense_grid(G * R / TN, (M + 127) / 128), 256, lds, st>>>(a, w, sw, c, M, G, R, K);
   UH_CHECK_LAUNCH();
 }
+// 256-column tiles once they leave more than 256 workgroups; before that twice the workgroups of 128 columns win
+// (DSV4 shape: 88 / 91 / 101 us at M = 512 / 768 / 1024 against 105 / 108 / 114; 157 against 197 us at M = 2048).
+bool wide_tiles(int M, int G, int R) {
+  return R % 256 == 0 && size_t((M + 127) / 128) * (size_t(G) * R / 256) > 256;
+}
 void launch_tiled(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
                   hipStream_t st) {
-  // 256-column tiles once they leave more than 256 workgroups; before that twice the workgroups of 128 columns win
-  // (DSV4 shape: 88 / 91 / 101 us at M = 512 / 768 / 1024 against 105 / 108 / 114; 157 against 197 us at M = 2048).
-  if (R % 256 == 0 && size_t((M + 127) / 128) * (size_t(G) * R / 256) > 256)
-    launch_tiled_t<256>(a, w, sw, c, M, G, R, K, st);
-  else
-    launch_tiled_t<128>(a, w, sw, c, M, G, R, K, st);
+  if (wide_tiles(M, G, R)) launch_tiled_t<256>(a, w, sw, c, M, G, R, K, st);
+  else launch_tiled_t<128>(a, w, sw, c, M, G, R, K, st);
 }
 
-// What a tiled launch takes (us, K = 4096, per 64-input stage): 1.13 up to 448 workgroups of 128 columns, 1.27 up to
-// 512, with 256 columns 1.75 up to 384 and 1.96 per 512 past that. G R = 8192: M = 512 78.8 measured, 800 79.6, 1024
-// 88.4, 1500 118, 2000 133.
+// What a tiled launch takes, us (K = 512 to 8192): a time per 64-input stage by the workgroups, 512 of which run at a time, as
+// fp8_tiled_us has it. G R = 8192, K = 4096, measured / this: M = 512 67.5 / 64.5, 1000 77 / 73, 2000 115 / 114, 2049 186 / 192,
+// 4096 269 / 270.
 double tiled_us(int M, int G, int R, int K) {
-  const size_t rt = size_t(M + 127) / 128, w128 = rt * (size_t(G) * R / 128), w256 = w128 / 2;
-  const double stage = R % 256 == 0 && w256 > 256 ? (w256 <= 384 ? 1.75 : 1.96 * double((w256 + 511) / 512))
-                                                  : (w128 <= 448 ? 1.13 : 1.27 * double((w128 + 511) / 512));
-  return 7.0 + K / 64 * stage;
+  const size_t w = (size_t(M) + 127) / 128 * (size_t(G) * R / 128);
+  const auto rounds = [](size_t n, double full, double part, double slope) {
+    return full * double(n / 512) + (n % 512 ? part + slope / 512 * double(n % 512) : 0.0);
+  };
+  const double stage = !wide_tiles(M, G, R) ? rounds(w, 1.12, 0.85, 0.27)
+                       : w / 2 <= 512       ? 1.0 + 0.75 / 512 * double(w / 2)
+                                            : rounds(w / 2, 2.1, 0.8, 1.3);
+  return 1.5 + K / 64 * stage;
 }
 }  // namespace
 
