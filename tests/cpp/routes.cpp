@@ -1,6 +1,6 @@
 // Prints the kernel that the library's dispatch chooses for each call described on stdin, one per line. Nothing is
 // launched and no pointer is read, so it runs without a GPU (tests/test_routes.py).
-//   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | rows | gemv | skinny
+//   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | gemv | skinny
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
 #include <cstdint>
 #include <iostream>
@@ -14,7 +14,7 @@ using namespace unholy::kernels;
 static const uint8_t* at(uintptr_t offset) { return reinterpret_cast<const uint8_t*>(0x100000 + offset); }
 
 int main() {
-  static const char* const kDense[] = {"kpart", "tiled", "rows", "gemv", "skinny"};
+  static const char* const kDense[] = {"kpart", "tiled", "gemv", "skinny"};
   static const char* const kGrouped[] = {"rows", "kpart", "gemv", "tiled", "ref"};
   for (std::string line; std::getline(std::cin, line);) {
     std::istringstream in(line);

@@ -165,8 +165,7 @@ def test_hazard_model_follows_a_loop_back_edge():
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
-@pytest.mark.parametrize("src,name,count,load", [("fp8_gemm.hip", "fp8_rows_kernel", 8, "global_load_dwordx4"),
-                                                 ("grouped_fp8w.hip", "grouped_fp8w_rows_kernel", 8, "global_load_dwordx4"),
+@pytest.mark.parametrize("src,name,count,load", [("grouped_fp8w.hip", "grouped_fp8w_rows_kernel", 4, "global_load_dwordx4"),
                                                  ("fp8_kpart.hip", "fp8_kpart_kernelILb1ELi1ELi1ELb1E", 1, "global_load_dwordx4"),
                                                  ("fp8_tiled.hip", "fp8_tiled_kernel", 4, "global_load_dword ")])
 def test_counted_loads_have_no_early_use(src, name, count, load, tmp_path):

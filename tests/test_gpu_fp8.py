@@ -345,3 +345,32 @@ def test_few_rows_same_bits_by_every_kernel(M, N, K, off):
     n = np.array([N], np.int32)
     call("uh_gemv_w8a8_parts", q, sa, *[v.ctypes.data for v in arr], n.ctypes.data, n.ctypes.data, 1, M, K, None)
     assert np.array_equal(c.download((M, N), np.uint16), ref.download((M, N), np.uint16))
+
+
+@pytest.mark.parametrize("M,f32,parts", [(20, True, False), (3, False, False), (40, False, False), (2, False, True)])
+def test_fp8_weights_past_4_gib(M, f32, parts):
+    """Columns whose weight rows lie past 4 GiB (K = 8192, rows 524288 on) against the oracle on those rows. The rows 2^32
+    bytes before them hold other codes, so a row offset that wraps would be seen."""
+    N0, N, K, n = 524288, 524288 + 144, 8192, 144
+    rng = np.random.default_rng(M)
+    x = randn_bf16(rng, (M, K))
+    q, sa = oracle.act_quant_fp8_f32s(x) if f32 else oracle.act_quant_fp8(x)
+    wq, sw = _w8a8_weights(rng, n, K)
+    if f32:
+        sw = (rng.random(sw.shape, np.float32) + 0.5) * np.float32(2.0 ** -6)
+    ref16, _ = oracle.gemm_w8a8(q, sa, wq, sw)
+    w = DeviceBuffer(N * K)
+    call("uh_memset", w.ptr, 0x38, N * K, None)  # e4m3 1.0
+    call("uh_memcpy_h2d", w.ptr + N0 * K, wq.ctypes.data, wq.nbytes)
+    s_all = np.ones(((N + 127) // 128, K // 128), np.float32) if f32 else np.full(((N + 127) // 128, K // 128), 127, np.uint8)
+    s_all[N0 // 128:] = sw
+    dq, dsa, dsw, c = dev(q), dev(sa), dev(s_all), DeviceBuffer(M * N * 2)
+    if parts:
+        wp, sp, cp = (np.array([v], np.uint64) for v in (w.ptr, dsw.ptr, c.ptr))
+        n_a = np.array([N], np.int32)
+        call("uh_gemv_w8a8_parts", dq, dsa, wp.ctypes.data, sp.ctypes.data, cp.ctypes.data, n_a.ctypes.data,
+             n_a.ctypes.data, 1, M, K, None)
+    else:
+        call("uh_gemm_fp8_f32s" if f32 else "uh_gemm_w8a8_wmma", dq, dsa, w, dsw, c, N, M, N, K, None)
+    got = c.download((M, N), np.uint16)[:, N0:]
+    assert max_rel(from_bf16(got), from_bf16(ref16)) <= 1e-2

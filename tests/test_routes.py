@@ -73,7 +73,7 @@ MEASURED_DENSE = [
 MEASURED_GROUPED = [
     (384, 8, 1024, 4096, 39.5, 66.5), (1024, 8, 1024, 4096, 95.0, 76.7), (2049, 8, 1024, 4096, 260.8, 183.3),
     (2304, 8, 1024, 4096, 276.0, 186.9), (768, 4, 1024, 4096, 37.9, 66.3), (2049, 4, 1024, 4096, 123.8, 89.2),
-    (384, 8, 1024, 2048, 24.2, 32.0), (2304, 8, 1024, 2048, 157.6, 97.6), (64, 32, 1024, 4096, 42.8, 66.8),
+    (384, 32, 1024, 4096, 144.0, 108.3), (384, 8, 1024, 2048, 24.2, 32.0), (2304, 8, 1024, 2048, 157.6, 97.6), (64, 32, 1024, 4096, 42.8, 66.8),
     (256, 16, 512, 1024, 11.4, 17.7), (2100, 16, 512, 1024, 86.3, 54.0),
     (2100, 2, 2048, 4096, 120.8, 89.0), (2300, 7, 1152, 4096, 240.4, 194.9)]
 
@@ -84,3 +84,10 @@ def test_the_estimates_choose_the_measured_winner(routes):
     answers = routes([l for l, _, _ in dense + grouped])
     bad = [(l, a) for (l, kp, t), a in zip(dense + grouped, answers) if a != ("kpart" if kp < t else "tiled")]
     assert not bad, bad
+
+
+def test_operands_of_any_size_keep_the_fast_kernels(routes):
+    """Weights and activations of 4 GiB and more go to the kernels that smaller ones go to."""
+    dense = [(m, n, k, f) for m in (1, 16, 40, 200) for n, k in ((1 << 20, 8192), (524352, 8192)) for f in (0, 1)]
+    assert set(routes([f"dense {m} {n} {k} {n} {f} 0 0" for m, n, k, f in dense])) <= {"kpart", "tiled"}
+    assert routes(["grouped 20000 128 64 4096 0 0", "grouped 100 128 1008 65536 0 0"]) == ["kpart", "kpart"]

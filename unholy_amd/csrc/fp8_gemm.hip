@@ -474,267 +474,7 @@ void launch_fp8_gemv_t(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts& pp)
   else fp8_gemv_kernel<F32S, 4><<<grid, 64 * FV_WAVES, 0, st>>>(a, pp);
   UH_CHECK_LAUNCH();
 }
-
-
-// ---- fp8 dense, 16 < M <= 256 with fp32 scales, weights past 4 GiB (else the K-part kernel): row tiles ----
-// A workgroup per 32 columns x 32 rows over the whole of K (<= 8,192), bf16 C written directly, one launch:
-// - 16 waves = 16 K parts of one 32 x 32 output tile (bf16 MFMA 32x32x16); part p takes block p of every 2,048-input
-//   chunk;
-// - CH = 1: each wave loads the activation codes of its own K part (32 rows x 128 codes a chunk, four 1 KB loads)
-//   into its own 2-slot LDS ring by direct global -> LDS loads, and its rows' fp32 scales into registers (lane r
-//   holds row r's; a lane-crossbar read hands each accumulator row its scale). No wave waits for another before the
-//   final reduction, so a wave computes its chunks as soon as its own loads land while the others still stream;
-//   piece q (16 bytes) of row r sits at q ^ ((r >> 1) & 7), so a 16-lane pass of 16-byte reads covers the 64 banks
-//   once. The waves of a 32-row tile share nothing but the reduction;
-// - CH = 2 (the two column halves of a K part read the same activations): the tile's activation codes go through a
-//   2-slot LDS ring of chunks (32 rows x 1,024 codes, 32 KB) by direct global -> LDS loads, filled by all 16 waves and
-//   read after a barrier; piece p (16 bytes) of row r sits at p ^ (r & 15), so a 16-lane pass of 16-byte reads
-//   covers the 64 banks once; the fp32 row scales of the tile are staged beside them;
-// - a wave's weights for all (<= 4) chunks are loaded into registers up front, interleaved with the first two
-//   activation chunks (issue order: scales, W0 A0 W1 A1 W2 W3, then A(c + 2) once chunk c is done); loads retire in
-//   order and each chunk waits for exactly the loads before its own. Weight load x (0..3) of a block: lane l reads
-//   16 bytes of column 16 (x >> 1) + l % 16 at byte 64 (x & 1) + 16 (l >> 4) (64 contiguous bytes of each of 16
-//   rows); one lane-row swap per dword pair then leaves lane l with column l % 32, load x holding piece
-//   2 h + (x >> 1) + 4 (x & 1) of the block, and the activation reads take the same pieces;
-// - per block: the raw chain of 8 MFMAs on exactly converted codes, folded as acc += raw * (sa * sw) (the reference's
-//   fp32-scale order); the 16 parts are added in LDS in part order, wave p adding accumulator element p;
-// - work item wi = column block x row tiles + row tile; XCD x takes the x-th eighth of the items, so the row tiles of
-//   a column block share one L2.
-// Against the one-tile GEMV (every 16-column workgroup reading all M rows from L2): the rows leave L2 once per 32
-// columns. A K split over workgroups (fp32 partial tiles in a workspace, added in slice order by a second launch) ran
-// 17.9 us per step at 64 x 4096 x 4096 against 14.0 here: the second launch and the partial round trip cost more
-// than the split gains.
-// Up to FR_MAXM rows (8 row tiles): at 4096 x 4096 the row tiles ran 22-43 us per step for 65 <= M <= 256 against
-// 47-53 us for the 128 x 128 tiled GEMM (too few workgroups there), which wins from M = 384 on (53 against 62 us).
-constexpr int FR_MAXCH = 4, FR_MAXM = 256;
-
-// CH column halves of 32 (workgroup width 32 CH); KP = 16 / CH K parts; chunks of KR = 128 KP inputs; NA direct loads
-// per wave per chunk (32 rows x KR codes in 1 KB loads over 16 waves). CH = 2 halves the workgroups of a wide, short
-// matrix (N / 64 column blocks), each wave then adding two accumulator elements in the reduction.
-template <int CH>
-struct Fp8Rows {
-  static constexpr int KP = 16 / CH, KR = 128 * KP, SLOT = 32 * KR, NA = SLOT / 1024 / 16, W = 32 * CH;
-  static constexpr int LS = CH == 2 ? 18 : 17;  // reduction lane stride (floats)
-  // CH = 1: each wave's own 2-slot ring of its K part (32 rows x 128 codes, 4 KB a slot); CH = 2: the shared ring
-  // of chunks and the tile's row scales.
-  static size_t lds(int K) {
-    const size_t ring = CH == 1 ? size_t(16) * 2 * 4096 : 2 * size_t(SLOT) + size_t(32) * (K / 128) * 4;
-    return std::max(ring, size_t(16) * 64 * LS * 4);
-  }
-};
-
-// NCH = the chunk count, ceil((K / 128) / KP) (1..FR_MAXCH): a template parameter, so that the issue order and every
-// counted wait are fixed at compile time and no branch depends on how many loads are outstanding.
-template <int CH, int NCH>
-__global__ __launch_bounds__(1024) void fp8_rows_kernel(Fp8GemmArgs p) {
-  using namespace pipe;
-  using T = Fp8Rows<CH>;
-  constexpr int KP = T::KP, KR = T::KR, SLOT = T::SLOT, NA = T::NA;
-  extern __shared__ __align__(16) uint8_t smem[];
-  static_assert(NCH >= 1 && NCH <= FR_MAXCH);
-  static_assert(CH == 2 || NA == 4, "CH = 1: four 1 KB activation loads per wave and chunk");
-  const int M = p.M, N = p.N, K = p.K, KS = K / 128;  // the host launches NCH = ceil(KS / KP)
-  const int nw = gridDim.x, lin = blockIdx.x;
-  const int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
-  const int RT = (M + 31) / 32, rt = wi % RT, bx = wi / RT, row0 = rt * 32;
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), chh = wave % CH, kh = wave / CH;  // column half, K part
-  const int col0 = bx * T::W, n = col0 + chh * 32 + l32;
-  const uint8_t* wld = p.w + size_t(col0 + chh * 32 + (lane & 15)) * K + (lane >> 4) * 16;
-  const float* swrow = p.sw32 + size_t((col0 + chh * 32) / 128) * KS;  // 32 columns lie in one 128-row block
-  const uint32_t lds0 = lds_addr(smem);
-  // The activation loads. CH = 1: load i of the wave covers rows 8i .. 8i + 7 of its 4 KB slot, lane j row
-  // 8i + j / 8 at piece (j % 8) ^ swz(row) of the K part. CH = 2: load i covers 1 KB of the shared chunk slot.
-  uint32_t rowoff[NA];
-  int pin[NA];
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    if constexpr (CH == 1) {
-      const int r = 8 * i + (lane >> 3);
-      rowoff[i] = uint32_t(min(row0 + r, M - 1)) * uint32_t(K);
-      pin[i] = 16 * ((lane & 7) ^ ((r >> 1) & 7));
-    } else {
-      const int slot = (wave * NA + i) * 64 + lane, r = slot / (KR / 16);
-      rowoff[i] = uint32_t(min(row0 + r, M - 1)) * uint32_t(K);
-      pin[i] = ((slot % (KR / 16)) ^ (r & 15)) * 16;
-    }
-  }
-  const auto issue_a = [&](int ch) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      if constexpr (CH == 1)
-        dma16(p.a, rowoff[i] + uint32_t(min(ch * KP + kh, KS - 1)) * 128u + uint32_t(pin[i]),
-              lds0 + uint32_t((wave * 2 + (ch & 1)) * 4096 + i * 1024));
-      else
-        dma16(p.a, rowoff[i] + uint32_t(min(ch * KR + pin[i], K - 16)),
-              lds0 + uint32_t((ch & 1) * SLOT + (wave * NA + i) * 1024));
-    }
-  };
-  v4i b[NCH][4];
-  const auto load_w = [&](int u) {
-    const uint8_t* q = wld + min(u * KP + kh, KS - 1) * 128;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) b[u][x] = vload16(q + (x >> 1) * 16 * K + (x & 1) * 64);
-  };
-  // Issue order: the scales (lane u < nch: the wave's weight scale of chunk u; CH = 1: lane r's row scale of each
-  // chunk's block; CH = 2: thread t's row scales t, t + 1024 of the tile), W0 A0 W1 A1 W2 W3, then A(c + 2).
-  uint32_t swv = vload_u32(swrow + min(min(lane, FR_MAXCH - 1) * KP + kh, KS - 1));
-  constexpr int NSA = CH == 1 ? NCH : 2;
-  uint32_t sav[NSA];
-#pragma unroll
-  for (int j = 0; j < NSA; ++j) {
-    if constexpr (CH == 1) {
-      sav[j] = vload_u32(p.sa32 + size_t(min(row0 + l32, M - 1)) * KS + min(j * KP + kh, KS - 1));
-    } else {
-      const int e = min(tid + 1024 * j, 32 * KS - 1);
-      sav[j] = vload_u32(p.sa32 + size_t(min(row0 + e / KS, M - 1)) * KS + e % KS);
-    }
-  }
-  float* const ssa = reinterpret_cast<float*>(smem + 2 * SLOT);  // CH = 2: row scales [32][KS]
-  load_w(0);
-  issue_a(0);
-  if constexpr (NCH > 1) {
-    load_w(1);
-    issue_a(1);
-  }
-  if constexpr (NCH > 2) load_w(2);
-  if constexpr (NCH > 3) load_w(3);
-  const int r = l32;
-  v16f_t acc = v16f_t{};
-  const auto chunk = [&](auto ich) {
-    constexpr int ch = decltype(ich)::value;
-    // Chunk ch, its weights and the scales have landed when only the loads issued after A(ch) are pending (4 per
-    // weight group, NA per activation group): ch = 0: W1 A1 W2 W3; ch = 1: W2 W3 A2; ch = 2: A3; each where it
-    // exists.
-    constexpr int later = ch == 0   ? 4 * ((1 < NCH) + (2 < NCH) + (3 < NCH)) + NA * (1 < NCH)
-                          : ch == 1 ? 4 * ((2 < NCH) + (3 < NCH)) + NA * (2 < NCH)
-                          : ch == 2 ? NA * (3 < NCH)
-                                    : 0;
-    wait_vm<later>();
-    vlanded(b[ch]);
-    if (ch == 0) {
-      vlanded(swv);
-#pragma unroll
-      for (int j = 0; j < NSA; ++j) vlanded(sav[j]);
-      if constexpr (CH == 2)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          if (tid + 1024 * j < 32 * KS) ssa[tid + 1024 * j] = __uint_as_float(sav[j]);
-    }
-    if constexpr (CH == 1) asm volatile("" ::: "memory");  // the wave's own activation pieces have landed in LDS
-    else __syncthreads();                                    // every wave's part of chunk ch (and the row scales)
-    const int kb = ch * KP + kh;
-    if (kb < KS) {
-      const uint8_t* sl = CH == 1 ? smem + (wave * 2 + (ch & 1)) * 4096 : smem + (ch & 1) * SLOT;
-      const float sw = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(swv), ch)));
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          // Lanes 16-31 (48-63) of load x trade with lanes 0-15 (32-47) of load x + 2.
-          const auto t = __builtin_amdgcn_permlane16_swap(uint32_t(b[ch][x][d]), uint32_t(b[ch][x + 2][d]), false,
-                                                          false);
-          b[ch][x][d] = int(t[0]);
-          b[ch][x + 2][d] = int(t[1]);
-        }
-      v16f_t raw = v16f_t{};
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int q = 2 * h + (x >> 1) + 4 * (x & 1);  // the piece of the block this load holds
-        const v4i av = CH == 1 ? *reinterpret_cast<const v4i*>(sl + r * 128 + (q ^ ((r >> 1) & 7)) * 16)
-                               : *reinterpret_cast<const v4i*>(sl + r * KR + ((kh * 8 + q) ^ (r & 15)) * 16);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const bf16x8 af = fp8x8_to_bf16(uint32_t(av[2 * e]), uint32_t(av[2 * e + 1]), 1.0f);
-          const bf16x8 bf = fp8x8_to_bf16(uint32_t(b[ch][x][2 * e]), uint32_t(b[ch][x][2 * e + 1]), 1.0f);
-          raw = mfma32_bf16(af, bf, raw);
-        }
-      }
-      // Element i of lane (l32, h) is row 8 (i / 4) + 4 h + i % 4 of the tile.
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = 8 * (i / 4) + 4 * h + (i % 4);
-        float sa;
-        if constexpr (CH == 1)
-          sa = __uint_as_float(uint32_t(__builtin_amdgcn_ds_bpermute(row * 4, int(sav[ch]))));
-        else
-          sa = ssa[row * KS + kb];
-        acc[i] += raw[i] * (sa * sw);
-      }
-    }
-    if constexpr (ch + 2 < NCH) {
-      if constexpr (CH == 2) __syncthreads();  // every wave is done with slot ch & 1
-      issue_a(ch + 2);  // CH = 1: the wave's own slot, whose reads above have returned
-    }
-  };
-  chunk(std::integral_constant<int, 0>{});
-  if constexpr (NCH > 1) chunk(std::integral_constant<int, 1>{});
-  if constexpr (NCH > 2) chunk(std::integral_constant<int, 2>{});
-  if constexpr (NCH > 3) chunk(std::integral_constant<int, 3>{});
-  // The KP parts added in part order through LDS: wave (chh, kh) adds elements CH kh .. CH kh + CH - 1 of its column
-  // half's lanes (lane stride 17 floats for 4-byte reads, 18 for 8-byte ones: a half-wave's reads cover the 64 banks
-  // once).
-  __syncthreads();
-  float* red = reinterpret_cast<float*>(smem);
-  float* mine = red + ((kh * CH + chh) * 64 + lane) * T::LS;
-  if constexpr (CH == 2) {
-#pragma unroll
-    for (int i = 0; i < 16; i += 2) *reinterpret_cast<float2*>(mine + i) = make_float2(acc[i], acc[i + 1]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mine[i] = acc[i];
-  }
-  __syncthreads();
-  float sum[CH];
-#pragma unroll
-  for (int e = 0; e < CH; ++e) sum[e] = red[(chh * 64 + lane) * T::LS + CH * kh + e];
-#pragma unroll
-  for (int q = 1; q < KP; ++q)
-#pragma unroll
-    for (int e = 0; e < CH; ++e) sum[e] += red[((q * CH + chh) * 64 + lane) * T::LS + CH * kh + e];
-  // Element i of lane (l32, h) is row 8 (i / 4) + 4 h + i % 4 of the tile.
-#pragma unroll
-  for (int e = 0; e < CH; ++e) {
-    const int i = CH * kh + e, row = row0 + 8 * (i / 4) + 4 * h + (i % 4);
-    if (row < M) p.c[size_t(row) * p.ldc + n] = f32_to_bf16(sum[e]);
-  }
-}
 }  // namespace
-
-// The wide form (CH = 2, K <= 4096) where its rounds of workgroups (256 CUs, one workgroup each) cost less: a wide
-// workgroup runs ~1.7x as long as a narrow one (~1.25x at K <= 1024, where half the narrow form's K parts idle).
-// Measured (us per call, wide / narrow): 32768 x 1024 M = 64 26.8 / 43.1, 8192 x 1024 M = 64 7.4 / 11.6, 4096 x 4096
-// M = 128 17.2 / 20.3, 129280 x 4096 M = 32 150 / 174; M = 64 at 4096 x 4096 (128 wide workgroups) 16.9 / 11.8, and
-// M = 160 (320 against 640 workgroups) 34.6 / 31.8 per step.
-static bool fp8_rows_wide(const Fp8GemmArgs& a) {
-  if (a.N % 64 || a.K > FR_MAXCH * Fp8Rows<2>::KR) return false;
-  const size_t rt = size_t(a.M + 31) / 32, nn = size_t(a.N / 32) * rt, nw = size_t(a.N / 64) * rt;
-  const double f = a.K <= 1024 ? 1.25 : 1.7;
-  return double((nw + 255) / 256) * f < double((nn + 255) / 256);
-}
-bool fp8_rows_fits(const Fp8GemmArgs& a) {
-  return a.sa32 && a.sw32 && a.M > 16 && a.M <= FR_MAXM && a.N % 32 == 0 && a.K % 128 == 0 && a.K >= 128 &&
-         a.K <= FR_MAXCH * Fp8Rows<1>::KR && size_t(a.M) * a.K < (size_t(1) << 32);
-}
-template <int CH>
-static void launch_fp8_rows_t(const Fp8GemmArgs& a, hipStream_t st) {
-  const size_t lds = Fp8Rows<CH>::lds(a.K);
-  const int nch = (a.K / 128 + Fp8Rows<CH>::KP - 1) / Fp8Rows<CH>::KP;  // 1..FR_MAXCH (fp8_rows_fits)
-  auto* kern = nch == 1   ? &fp8_rows_kernel<CH, 1>
-               : nch == 2 ? &fp8_rows_kernel<CH, 2>
-               : nch == 3 ? &fp8_rows_kernel<CH, 3>
-                          : &fp8_rows_kernel<CH, 4>;
-  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(lds)));
-  kern<<<dim3(unsigned(a.N / Fp8Rows<CH>::W * ((a.M + 31) / 32))), 1024, lds, st>>>(a);
-  UH_CHECK_LAUNCH();
-}
-void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st) {
-  if (!fp8_rows_fits(a)) throw std::runtime_error("fp8 rows: shape");
-  if (!a.a || !a.w || !a.c) throw std::runtime_error("fp8 gemm: null operand");
-  if (fp8_rows_wide(a)) launch_fp8_rows_t<2>(a, st);
-  else launch_fp8_rows_t<1>(a, st);
-}
 
 static size_t skinny_lds(const Fp8GemmArgs& a) {
   const size_t rows = std::min(a.M, DN_MAXROWS);
@@ -748,7 +488,6 @@ Fp8Route fp8_route(const Fp8GemmArgs& a) {
   const bool same_bits = a.M <= (a.sa32 ? 16 : 32);
   if (fp8_kpart_fits(a))
     return same_bits || !fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a) ? Fp8Route::kpart : Fp8Route::tiled;
-  if (aligned && fp8_rows_fits(a)) return Fp8Route::rows;  // weights past 4 GiB
   if (a.M <= 64) return Fp8Route::gemv;
   // (unaligned operands whose rows do not fit the row groups' LDS stay with the tiled GEMM)
   if (fp8_tiled_fits(a) && (aligned || skinny_lds(a) > 160 * 1024)) return Fp8Route::tiled;
@@ -759,7 +498,6 @@ void launch_fp8_gemm(const Fp8GemmArgs& a, hipStream_t st) {
   switch (fp8_route(a)) {
     case Fp8Route::kpart: return launch_fp8_kpart(a, st);
     case Fp8Route::tiled: return launch_fp8_tiled(a, st);
-    case Fp8Route::rows: return launch_fp8_rows(a, st);
     case Fp8Route::gemv: return launch_fp8_gemv(a, st);
     case Fp8Route::skinny: return launch_fp8_skinny(a, st);
   }

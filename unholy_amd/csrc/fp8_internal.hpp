@@ -36,10 +36,6 @@ struct Fp8Parts {
 void launch_fp8_skinny(const Fp8GemmArgs& a, hipStream_t st);
 // M <= 64: one workgroup per 16-column tile, K split over its 8 waves (bandwidth-shaped).
 void launch_fp8_gemv(const Fp8GemmArgs& a, hipStream_t st, const Fp8Parts* parts = nullptr);
-// 16 < M <= 256 with fp32 scales and weights past 4 GiB: one workgroup per 32 x 32 output tile over the whole of K (N % 32,
-// K <= 8192).
-bool fp8_rows_fits(const Fp8GemmArgs& a);
-void launch_fp8_rows(const Fp8GemmArgs& a, hipStream_t st);
 // The LDS-ring MFMA GEMM (N % 128, K % 128, ldc % 8; fp8_tiled_fits says whether a shape qualifies).
 bool fp8_tiled_fits(const Fp8GemmArgs& a);
 void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st);
@@ -57,10 +53,10 @@ bool grouped_kpart_fits(int M, int G, int R, int K);
 double grouped_kpart_us(int M, int G, int R, int K);
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st);
-// The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits
-// (operands past 4 GiB, K > 8192) the row tiles, the GEMV (M <= 64) or the row-group kernel. The first three load operands
-// straight into LDS, 16 bytes a lane, and are kept to 16-byte aligned operands; the GEMV and the row groups take any.
-enum class Fp8Route { kpart, tiled, rows, gemv, skinny };
+// The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits (K > 8192,
+// N % 128) the GEMV (M <= 64) or the row-group kernel. The first two load operands straight into LDS, 16 bytes a lane, and
+// are kept to 16-byte aligned operands; the GEMV and the row groups take any.
+enum class Fp8Route { kpart, tiled, gemv, skinny };
 Fp8Route fp8_route(const Fp8GemmArgs& a);
 inline bool fp8_aligned(const void* a, const void* w) {
   return (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) % 16 == 0;

@@ -457,12 +457,11 @@ int best_form(const Fp8GemmArgs& a) {
 
 bool fp8_kpart_fits(const Fp8GemmArgs& a) {
   return a.M > 0 && a.N > 0 && a.K > 0 && a.K % 128 == 0 && a.K <= 128 * KP_WAVES * 4 * NSET && fp8_aligned(a.a, a.w) &&
-         (a.sa32 || a.xa ? a.sw32 != nullptr : a.sa8 && a.sw8) && size_t(a.M) * a.K < (size_t(1) << 32) &&
-         size_t(a.N) * a.K < (size_t(1) << 32);
+         (a.sa32 || a.xa ? a.sw32 != nullptr : a.sa8 && a.sw8);
 }
 bool fp8_kpart_parts_fits(const Fp8GemmArgs& a, const Fp8Parts& pp) {
   for (int i = 0; i < pp.n; ++i)
-    if (size_t(pp.N[i]) * a.K >= (size_t(1) << 32) || !fp8_aligned(a.a, pp.w[i])) return false;
+    if (!fp8_aligned(a.a, pp.w[i])) return false;
   return a.M > 0 && a.M <= 32 && a.K <= 128 * KP_WAVES * 4 * NSET;
 }
 void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_t st) {
@@ -512,9 +511,10 @@ int best_gform(int M, int G, int R, int K) {
 }
 }  // namespace
 
+// (a tile's rows span up to 128 G K bf16 from its base, in 32-bit offsets)
 bool grouped_kpart_fits(int M, int G, int R, int K) {
   return M > 0 && R > 0 && R % 16 == 0 && K > 0 && K % 128 == 0 && K <= 128 * KP_WAVES * 64 &&
-         size_t(M) * G * K * 2 < (size_t(1) << 32) && size_t(G) * R * K < (size_t(1) << 32);
+         size_t(128) * G * K * 2 < (size_t(1) << 32);
 }
 double grouped_kpart_us(int M, int G, int R, int K) { return gform_us(M, G * R, K, kGForms[best_gform(M, G, R, K)]); }
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,

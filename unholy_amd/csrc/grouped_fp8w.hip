@@ -7,18 +7,16 @@
 // Three entry points, as the reference has them:
 //   gemm_grouped_fp8w       the reference order (ref_gemm.hip:116-125, :198-202 at G = K: one fp32 fmaf chain over k
 //                           in order), a thread per output: bit-exact against the CPU oracle, not a fast path;
-//   gemm_grouped_fp8w_wmma  the fast path: the row-tile kernel for M <= 384 (M <= 16: R % 32 == 0, K <= 8192;
-//                           else R % 64 == 0, K <= 4096), the GEMV for other shapes up to M = 160, else the tiled
-//                           MFMA GEMM;
+//   gemm_grouped_fp8w_wmma  the fast path: the row-tile kernel up to 8 rows, the K-part kernel (fp8_kpart.hip) or the tiled
+//                           MFMA GEMM past them, the GEMV for what they do not take (grouped_route);
 //   gemv_grouped_fp8w       M <= 32 as the fast path, optionally followed by act_quant_fp8 of its outputs (GemvQuant).
 //
 // GEMV (bound: HBM, 32 MB of weights at the DSV4 shape G = 8, R = 1024, K = 4096): a workgroup per 16-column tile,
 // its 8 waves splitting K in 128-input blocks, every load of a chunk issued before its first use; bf16 MFMA
 // 16x16x32 on the activations as they are and the weights dequantized with the block scale folded in; the 8
 // partial tiles added in LDS in wave order.
-// Row tiles (M <= 384): a workgroup per 64 columns x 32 rows (M <= 16: 32 columns x 16 rows) over the whole of K, the
-// activation rows staged once per workgroup in LDS (the GEMV reads them once per 16 columns), the weights held in
-// registers up to four chunks ahead.
+// Row tiles (M <= 8): a workgroup per 32 columns x 16 rows over the whole of K, each wave staging its own K part's rows in
+// LDS, the weights held in registers up to four chunks ahead.
 // GEMM (bound: MFMA at M = 4096): 128-row tiles of one group, 4 waves, 64-input stages in an LDS ring filled by direct
 // global -> LDS loads (two workgroups per CU); bf16 MFMA 32x32x16. A wave's columns lie in one 128-row weight block
 // and a stage in one 128-input block, so the weight scale is one value per stage, folded into the dequantization.
@@ -131,91 +129,60 @@ __global__ __launch_bounds__(64 * GV_W) void grouped_fp8w_gemv_kernel(const bf16
   }
 }
 
-// ---- row tiles, M <= 384 -----------------------------------------------------------------------------------------
-// A workgroup per 64 columns (one group: R % 64 == 0) x 32 rows, the whole of K (<= 4,096), bf16 C written directly
-// (M <= 16: 32 columns x 16 rows, K <= 8,192, 16 K parts of 2,048-input chunks; the parameters below):
-// - 16 waves = 2 column halves x 8 K parts, 32 x 32 output tiles (bf16 MFMA 32x32x16); part p takes block p of every
-//   1,024-input chunk;
+// ---- row tiles, up to 8 rows -----------------------------------------------------------------------------------------
+// A workgroup per 32 columns (one group: R % 32 == 0) x 16 rows, the whole of K (<= 8,192), bf16 C written directly:
+// - 16 waves = 16 K parts, 32 x 32 output tiles (bf16 MFMA 32x32x16); part p takes block p of every 2,048-input chunk;
 // - a wave's weights for all (<= 4) chunks are loaded into registers up front, interleaved with the first two
 //   activation chunks (issue order: scales, W0 A0 W1 A1 W2 W3, then A(c + 2) once chunk c is done), so chunk c starts
 //   while the later weights stream; loads retire in order and each chunk waits for exactly the loads before its own;
-// - the tile's activation rows go through a 2-slot LDS ring of chunks (32 rows x 1,024 bf16, 64 KB) by direct
-//   global -> LDS loads; piece p (16 bytes) of row r sits at p ^ (r & 15), so the 16 rows of an MFMA operand pass
-//   cover the 64 banks once (the 32-column form: each wave stages its own K part's 16 rows in its own ring and waits
-//   for no other wave until the reduction);
-// - the weights dequantize with the block scale folded in (exact); the 8 parts (16 in the 32-column form) are added
-//   in LDS in part order by all 16 waves;
-// - work item wi = column block x row tiles + row tile; XCD x takes the x-th eighth of the items, so the row tiles of
-//   a column block share one L2 (the second reads the weights from it) and a group's activation rows sit in one L2.
-// Against the GEMV (one 16-column tile per workgroup, every workgroup reading its rows from L2): the activation rows
-// leave L2 once per 64 columns. DSV4 shape: 17.6 us against 45 us at M = 64; at M = 1 8.9 us against 10.8 us (the
-// 32-column form: 256 workgroups, each wave's weights in flight at once).
-constexpr int GR_SLOT = 64 * 1024, GR_MAXCH = 4;
-
-// CH column halves of 32 (workgroup width 32 CH), TR staged rows (32, or 16 for M <= 16: the MFMA's rows 16-31 then
-// read rows 0-15 again and are not stored); KP = 16 / CH K parts, chunks of KR = 128 KP inputs, a 64 KB slot either way.
-template <int CH, int TR>
-struct GroupedRows {
-  static constexpr int KP = 16 / CH, KR = 128 * KP, PPR = KR / 8, W = 32 * CH;
-  static_assert(TR * KR * 2 == GR_SLOT, "one chunk fills a slot");
-};
+// - each wave stages its own K part's 16 activation rows in its own 2-slot LDS ring by direct global -> LDS loads and waits
+//   for no other wave until the reduction; piece p (16 bytes) of row r sits at p ^ r, so the 16 rows of an MFMA operand
+//   pass cover the 64 banks once;
+// - the weights dequantize with the block scale folded in (exact); the 16 parts are added in LDS in part order by all
+//   16 waves;
+// - XCD x takes the x-th eighth of the workgroups, so a group's activation rows sit in one L2.
+// 256 workgroups at the DSV4 shape, every wave's weights in flight at once: M = 1 8.9 us against 10.8 us for the GEMV (one
+// 16-column tile per workgroup).
+// KP K parts, chunks of KR inputs; 16 staged rows (the MFMA's rows 16-31 read rows 0-15 again and are not stored).
+constexpr int GR_MAXCH = 4, GR_TR = 16, GR_KP = 16, GR_KR = 128 * GR_KP, GR_W = 32, GR_LDS = GR_KP * 2 * 4096;
 
 // NCH = the chunk count, ceil((K / 128) / KP) (1..GR_MAXCH): a template parameter, so that the issue order and every
 // counted wait are fixed at compile time and no branch depends on how many loads are outstanding.
-template <int CH, int TR, int NCH>
+template <int NCH>
 __global__ __launch_bounds__(1024) void grouped_fp8w_rows_kernel(const bf16* a, const uint8_t* w, const uint8_t* sw,
                                                                  bf16* c, int M, int G, int R, int K) {
-  using T = GroupedRows<CH, TR>;
-  constexpr int KP = T::KP, KR = T::KR, PPR = T::PPR;
+  constexpr int KP = GR_KP, TR = GR_TR;
   extern __shared__ __align__(16) uint8_t smem[];
   static_assert(NCH >= 1 && NCH <= GR_MAXCH);
-  static_assert(CH == 2 || TR == 16, "the per-wave activation loads cover 16 rows");
   const int N = G * R, KS = K / 128;  // the host launches NCH = ceil(KS / KP)
   const int nw = gridDim.x, lin = blockIdx.x;
-  const int wi = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
-  const int RT = (M + TR - 1) / TR, rt = wi % RT, bx = wi / RT, row0 = rt * TR;
+  const int bx = nw % 8 ? lin : (lin & 7) * (nw >> 3) + (lin >> 3);
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), chh = wave % CH, kh = wave / CH;
-  const int col0 = bx * T::W, grp = col0 / R, n = col0 + chh * 32 + l32;
+  const int kh = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's K part
+  const int col0 = bx * GR_W, grp = col0 / R, n = col0 + l32;
   // Weight load x (0..3) of a block: lane l reads 16 bytes of column row 16 (x >> 1) + l % 16 at byte 64 (x & 1) +
   // 16 (l >> 4), so a load covers 64 contiguous bytes of each of 16 rows (32 bytes of 32 rows in the MFMA's own
   // layout measured 2.6 us slower at the DSV4 shape). One lane-row swap per dword pair (loads 0 <-> 2, 1 <-> 3) then
   // leaves lane l with column l % 32: load x holds piece (16 bytes) 2 h + (x >> 1) + 4 (x & 1) of the block.
-  const uint8_t* wld = w + size_t(col0 + chh * 32 + (lane & 15)) * K + (lane >> 4) * 16;
-  const uint8_t* swrow = sw + size_t((col0 + chh * 32) / 128) * KS;  // 32 columns lie in one 128-row block
+  const uint8_t* wld = w + size_t(col0 + (lane & 15)) * K + (lane >> 4) * 16;
+  const uint8_t* swrow = sw + size_t(col0 / 128) * KS;  // 32 columns lie in one 128-row block
   const uint32_t lds0 = lds_addr(smem);
-  // This wave's 4 direct loads of a chunk (rows past M repeat row M - 1; neither they nor the clamped inputs are
-  // used).
-  // - CH = 1 (16 rows): the wave's own K part, 16 rows x 128 inputs (4 KB), into its own 2-slot ring: load i covers
-  //   rows 4i .. 4i + 3, lane j row 4i + j / 16 at piece (j % 16) ^ row, so a 16-lane pass of the MFMA's 16-byte
-  //   reads (16 rows, one piece) covers the 64 banks once. No wave waits for another before the reduction: a wave
-  //   computes its chunks as soon as its own loads land while the others still stream.
-  // - CH = 2 (32 rows, the two column halves of a K part read the same activations): 1 KB pieces q = 4 wave + i of
-  //   the shared 64 KB chunk slot, read after a barrier.
+  // This wave's 4 direct loads of a chunk, its own K part of 16 rows x 128 inputs (4 KB) (rows past M repeat row M - 1;
+  // neither they nor the clamped inputs are used): load i covers rows 4i .. 4i + 3, lane j row 4i + j / 16 at piece
+  // (j % 16) ^ row.
   uint32_t rowoff[4];
   int pin[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if constexpr (CH == 1) {
-      const int r = 4 * i + (lane >> 4);
-      rowoff[i] = uint32_t(min(row0 + r, M - 1) * G + grp) * uint32_t(K) * 2u;
-      pin[i] = ((lane & 15) ^ r) * 8;
-    } else {
-      const int slot = (wave * 4 + i) * 64 + lane, r = slot / PPR;
-      rowoff[i] = uint32_t(min(row0 + r, M - 1) * G + grp) * uint32_t(K) * 2u;
-      pin[i] = ((slot % PPR) ^ (r & 15)) * 8;
-    }
+    const int r = 4 * i + (lane >> 4);
+    rowoff[i] = uint32_t(min(r, M - 1) * G + grp) * uint32_t(K) * 2u;
+    pin[i] = ((lane & 15) ^ r) * 8;
   }
   const auto issue_a = [&](int ch) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (CH == 1)
-        dma16(a, rowoff[i] + uint32_t(min(ch * KP + kh, KS - 1) * 128 + pin[i]) * 2u,
-              lds0 + uint32_t((wave * 2 + (ch & 1)) * 4096 + i * 1024));
-      else
-        dma16(a, rowoff[i] + uint32_t(min(ch * KR + pin[i], K - 8)) * 2u,
-              lds0 + uint32_t((ch & 1) * GR_SLOT + (wave * 4 + i) * 1024));
-    }
+    for (int i = 0; i < 4; ++i)
+      dma16(a, rowoff[i] + uint32_t(min(ch * KP + kh, KS - 1) * 128 + pin[i]) * 2u,
+            lds0 + uint32_t((kh * 2 + (ch & 1)) * 4096 + i * 1024));
   };
   v4i b[NCH][4];
   const auto load_w = [&](int u) {
@@ -247,10 +214,9 @@ __global__ __launch_bounds__(1024) void grouped_fp8w_rows_kernel(const bf16* a, 
     wait_vm<later>();
     vlanded(b[ch]);
     vlanded(sv);
-    if constexpr (CH == 1) asm volatile("" ::: "memory");  // the wave's own activation pieces have landed in LDS
-    else __syncthreads();                                    // every wave's part of chunk ch has landed
+    asm volatile("" ::: "memory");  // the wave's own activation pieces have landed in LDS
     if (ch * KP + kh < KS) {
-      const uint8_t* sl = CH == 1 ? smem + (wave * 2 + (ch & 1)) * 4096 : smem + (ch & 1) * GR_SLOT;
+      const uint8_t* sl = smem + (kh * 2 + (ch & 1)) * 4096;
       const float swc = __uint_as_float(uint32_t(__builtin_amdgcn_readlane(int(sv), ch)) << 23);
 #pragma unroll
       for (int x = 0; x < 2; ++x)
@@ -267,80 +233,49 @@ __global__ __launch_bounds__(1024) void grouped_fp8w_rows_kernel(const bf16* a, 
         const int x = j >> 1;
         const bf16x8 bf = fp8x8_to_bf16(uint32_t(b[ch][x][2 * (j & 1)]), uint32_t(b[ch][x][2 * (j & 1) + 1]), swc);
         const int q = 2 * (2 * h + (x >> 1) + 4 * (x & 1)) + (j & 1);  // the block's piece of this MFMA
-        const bf16x8 af = CH == 1
-            ? __builtin_bit_cast(bf16x8, *reinterpret_cast<const v4i*>(sl + (r * 16 + (q ^ r)) * 16))
-            : __builtin_bit_cast(bf16x8, *reinterpret_cast<const v4i*>(sl + (r * PPR + ((kh * 16 + q) ^ (r & 15))) * 16));
+        const bf16x8 af = __builtin_bit_cast(bf16x8, *reinterpret_cast<const v4i*>(sl + (r * 16 + (q ^ r)) * 16));
         acc = mfma32_bf16(af, bf, acc);
       }
     }
-    if constexpr (ch + 2 < NCH) {
-      if constexpr (CH == 2) __syncthreads();  // every wave is done with slot ch & 1
-      issue_a(ch + 2);  // CH = 1: the wave's own slot, whose reads above have returned
-    }
+    if constexpr (ch + 2 < NCH) issue_a(ch + 2);  // the wave's own slot, whose reads above have returned
   };
   chunk(std::integral_constant<int, 0>{});
   if constexpr (NCH > 1) chunk(std::integral_constant<int, 1>{});
   if constexpr (NCH > 2) chunk(std::integral_constant<int, 2>{});
   if constexpr (NCH > 3) chunk(std::integral_constant<int, 3>{});
-  // The KP parts added in part order through LDS, shared by all waves: wave (chh, kh) adds elements CH kh ..
-  // CH kh + CH - 1 of its column half's lanes. Lane stride 18 floats for 8-byte reads (CH 2), 17 for 4-byte ones
-  // (CH 1): a half-wave's reads cover the 64 banks once.
+  // The KP parts added in part order through LDS, shared by all waves: wave kh adds element kh of every lane. Lane stride 17
+  // floats: a half-wave's reads cover the 64 banks once.
   __syncthreads();
   float* red = reinterpret_cast<float*>(smem);
-  constexpr int LS = CH == 2 ? 18 : 17;
-  float* mine = red + ((kh * CH + chh) * 64 + lane) * LS;
-  if constexpr (CH == 2) {
+  constexpr int LS = 17;
+  static_assert(KP * 64 * LS * 4 <= GR_LDS);
+  float* mine = red + (kh * 64 + lane) * LS;
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) *reinterpret_cast<float2*>(mine + i) = make_float2(acc[i], acc[i + 1]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mine[i] = acc[i];
-  }
+  for (int i = 0; i < 16; ++i) mine[i] = acc[i];
   __syncthreads();
-  float sum[CH];
+  float sum = red[lane * LS + kh];
 #pragma unroll
-  for (int e = 0; e < CH; ++e) sum[e] = red[(chh * 64 + lane) * LS + CH * kh + e];
-#pragma unroll
-  for (int q = 1; q < KP; ++q)
-#pragma unroll
-    for (int e = 0; e < CH; ++e) sum[e] += red[((q * CH + chh) * 64 + lane) * LS + CH * kh + e];
-  // Element i of lane (l32, h) is row 8 (i / 4) + 4 h + i % 4 of the tile, column l32 of the half.
-#pragma unroll
-  for (int e = 0; e < CH; ++e) {
-    const int i = CH * kh + e, rr = 8 * (i / 4) + 4 * h + (i % 4);
-    if (rr < TR && row0 + rr < M) c[size_t(row0 + rr) * N + n] = f32_to_bf16(sum[e]);
-  }
+  for (int q = 1; q < KP; ++q) sum += red[(q * 64 + lane) * LS + kh];
+  // Element i of lane (l32, h) is row 8 (i / 4) + 4 h + i % 4 of the tile, column l32.
+  const int rr = 8 * (kh / 4) + 4 * h + (kh % 4);
+  if (rr < M) c[size_t(rr) * N + n] = f32_to_bf16(sum);
 }
 
-// M <= 16: 32-column workgroups of 16 staged rows (256 workgroups at the DSV4 shape, every wave's weights in flight at
-// once); 16 < M <= GR_MAXM: 64-column workgroups of 32-row tiles. At the DSV4 shape the row tiles ran 44 / 58 / 86 us
-// at M = 192 / 256 / 384 against 100-106 us for the tiled GEMM (128 workgroups or fewer there), which wins from
-// M = 512 on (107 against 116 us).
-constexpr int GR_MAXM = 384;
+// Up to 8 rows while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part kernel, 8 9.28 / 9.43, 16 10.9 / 10.1).
 bool rows_fits(int M, int G, int R, int K) {
-  if (M < 1 || M > GR_MAXM || size_t(M) * G * K * 2 >= (size_t(1) << 32)) return false;
-  return M <= 16 ? R % 32 == 0 && K <= GR_MAXCH * GroupedRows<1, 16>::KR
-                 : R % 64 == 0 && K <= GR_MAXCH * GroupedRows<2, 32>::KR;
-}
-template <int CH, int TR>
-void launch_rows_t(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
-                   hipStream_t st) {
-  const size_t lds = 2 * size_t(GR_SLOT);
-  const int nch = (K / 128 + GroupedRows<CH, TR>::KP - 1) / GroupedRows<CH, TR>::KP;  // 1..GR_MAXCH (rows_fits)
-  auto* kern = nch == 1   ? &grouped_fp8w_rows_kernel<CH, TR, 1>
-               : nch == 2 ? &grouped_fp8w_rows_kernel<CH, TR, 2>
-               : nch == 3 ? &grouped_fp8w_rows_kernel<CH, TR, 3>
-                          : &grouped_fp8w_rows_kernel<CH, TR, 4>;
-  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(lds)));
-  kern<<<dim3(unsigned(G * R / GroupedRows<CH, TR>::W * ((M + TR - 1) / TR))), 1024, lds, st>>>(a, w, sw, c, M, G, R,
-                                                                                                 K);
-  UH_CHECK_LAUNCH();
+  return M >= 1 && M <= 8 && R % 32 == 0 && K <= GR_MAXCH * GR_KR && size_t(G) * R / GR_W >= 256 &&
+         size_t(M) * G * K * 2 < (size_t(1) << 32);
 }
 void launch_rows(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
                  hipStream_t st) {
-  if (M <= 16) launch_rows_t<1, 16>(a, w, sw, c, M, G, R, K, st);
-  else launch_rows_t<2, 32>(a, w, sw, c, M, G, R, K, st);
+  const int nch = (K / 128 + GR_KP - 1) / GR_KP;  // 1..GR_MAXCH (rows_fits)
+  auto* kern = nch == 1   ? &grouped_fp8w_rows_kernel<1>
+               : nch == 2 ? &grouped_fp8w_rows_kernel<2>
+               : nch == 3 ? &grouped_fp8w_rows_kernel<3>
+                          : &grouped_fp8w_rows_kernel<4>;
+  UH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GR_LDS));
+  kern<<<dim3(unsigned(G * R / GR_W)), 1024, GR_LDS, st>>>(a, w, sw, c, M, G, R, K);
+  UH_CHECK_LAUNCH();
 }
 
 // ---- tiled GEMM ------------------------------------------------------------------------------------------------------
@@ -483,8 +418,8 @@ void launch_ref(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int
   UH_CHECK_LAUNCH();
 }
 
-// The GEMV for up to 160 rows (32-row chunks side by side) where the row-tile kernel does not take the shape, the tiled
-// GEMM above: at the DSV4 shape M = 64 the GEMV ran 46 us as two chunks, the tiled kernel 69 us (64 workgroups).
+// The GEMV for up to 160 rows (32-row chunks side by side), what the K-part kernel does not take: at the DSV4 shape M = 64 it
+// ran 46 us as two chunks, the tiled kernel 69 us (64 workgroups).
 constexpr int GV_MAX_ROWS = 160;
 bool gemv_fits(int M, int R) { return M <= GV_MAX_ROWS && R % 16 == 0; }
 void launch_gemv(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
@@ -533,18 +468,17 @@ double tiled_us(int M, int G, int R, int K) {
 }
 }  // namespace
 
-// Up to 8 rows the row tiles' 32-column form while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part
-// kernel, 8 9.28 / 9.43, 16 10.9 / 10.1); else the K-part kernel or the tiled GEMM by their estimated times; then the
-// kernels for what neither takes (operands past 4 GiB, R % 16 != 0). All but the GEMV and the reference order load
-// operands straight into LDS, 16 bytes a lane: operands that are not 16-byte aligned take those two.
+// Up to 8 rows the row tiles; else the K-part kernel or the tiled GEMM by their estimated times; then what the K-part
+// kernel does not take (R % 16, a row of G K past 2^24): the GEMV, the tiled GEMM, the reference order. The GEMV and the
+// reference order read their operands with plain loads and take those that are not 16-byte aligned, the others load
+// them straight into LDS, 16 bytes a lane.
 GroupedRoute grouped_route(const void* a, const void* w, int M, int G, int R, int K) {
   if (!fp8_aligned(a, w)) return R % 16 == 0 ? GroupedRoute::gemv : GroupedRoute::ref;
-  const bool few = M <= 8 && size_t(G) * R / 32 >= 256 && rows_fits(M, G, R, K), tiled = tiled_fits(G, R, K);
-  if (!few && grouped_kpart_fits(M, G, R, K) && (!tiled || grouped_kpart_us(M, G, R, K) < tiled_us(M, G, R, K)))
-    return GroupedRoute::kpart;
   if (rows_fits(M, G, R, K)) return GroupedRoute::rows;
-  if (gemv_fits(M, R) && !grouped_kpart_fits(M, G, R, K)) return GroupedRoute::gemv;
-  return tiled ? GroupedRoute::tiled : GroupedRoute::ref;
+  const bool tiled = tiled_fits(G, R, K);
+  if (grouped_kpart_fits(M, G, R, K))
+    return !tiled || grouped_kpart_us(M, G, R, K) < tiled_us(M, G, R, K) ? GroupedRoute::kpart : GroupedRoute::tiled;
+  return gemv_fits(M, R) ? GroupedRoute::gemv : tiled ? GroupedRoute::tiled : GroupedRoute::ref;
 }
 
 namespace {
