@@ -1,6 +1,7 @@
 // Prints the kernel that the library's dispatch chooses for each call described on stdin, one per line. Nothing is
 // launched and no pointer is read, so it runs without a GPU (tests/test_routes.py).
 //   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | gemv | skinny
+//   form  M N K ldc f32 a_offset w_offset       -> the K-part kernel's tile, row x column blocks of 16
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
 #include <cstdint>
 #include <iostream>
@@ -20,7 +21,7 @@ int main() {
     std::istringstream in(line);
     std::string kind;
     in >> kind;
-    if (kind == "dense") {
+    if (kind == "dense" || kind == "form") {
       Fp8GemmArgs a{};
       int f32 = 0;
       uintptr_t ao = 0, wo = 0;
@@ -30,7 +31,12 @@ int main() {
       a.c = reinterpret_cast<uint16_t*>(0x100000);
       if (f32) a.sa32 = a.sw32 = reinterpret_cast<const float*>(0x100000);
       else a.sa8 = a.sw8 = at(0);
-      std::cout << kDense[int(fp8_route(a))] << "\n";
+      if (kind == "form") {
+        const auto [rb, cb] = fp8_kpart_form(a);
+        std::cout << rb << "x" << cb << "\n";
+      } else {
+        std::cout << kDense[int(fp8_route(a))] << "\n";
+      }
     } else if (kind == "grouped") {
       int M, G, R, K;
       uintptr_t ao = 0, wo = 0;

@@ -86,6 +86,20 @@ def test_the_estimates_choose_the_measured_winner(routes):
     assert not bad, bad
 
 
+# The K-part kernel's fastest tile (gfx950, us, M, N, K, fp32 scales): one-tile workgroups take longer with e8m0 scales.
+MEASURED_FORMS = [
+    (1, 8192, 1024, 0, "2x2"), (16, 8192, 1024, 0, "2x2"), (8, 7168, 2048, 0, "2x2"), (1, 8192, 1024, 1, "1x1"),
+    (16, 32768, 1024, 0, "1x1"), (1, 4096, 4096, 0, "1x1"), (32, 4096, 4096, 1, "2x1"), (64, 4096, 4096, 0, "2x2"),
+    (128, 4096, 4096, 0, "4x2"), (256, 4096, 4096, 1, "4x4"), (300, 4096, 4096, 0, "5x4"), (384, 4096, 4096, 1, "6x4"),
+    (700, 2048, 4096, 0, "6x4"), (17, 2560, 640, 0, "2x1")]
+
+
+def test_the_estimates_choose_the_measured_tile(routes):
+    answers = routes([f"form {m} {n} {k} {n} {f} 0 0" for m, n, k, f, _ in MEASURED_FORMS])
+    bad = [(c, a) for c, a in zip(MEASURED_FORMS, answers) if a != c[4]]
+    assert not bad, bad
+
+
 def test_operands_of_any_size_keep_the_fast_kernels(routes):
     """Weights and activations of 4 GiB and more go to the kernels that smaller ones go to."""
     dense = [(m, n, k, f) for m in (1, 16, 40, 200) for n, k in ((1 << 20, 8192), (524352, 8192)) for f in (0, 1)]

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <utility>
 
 namespace unholy::kernels {
 
@@ -43,6 +44,7 @@ void launch_fp8_tiled(const Fp8GemmArgs& a, hipStream_t st);
 // ranges of gemv_w8a8_parts (M <= 32), and bf16 rows quantized in the kernel (fp32 scales, M <= 16).
 bool fp8_kpart_fits(const Fp8GemmArgs& a);
 double fp8_kpart_us(const Fp8GemmArgs& a);
+std::pair<int, int> fp8_kpart_form(const Fp8GemmArgs& a);  // the tile it would use, in 16-row and 16-column blocks
 void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st);
 bool fp8_kpart_parts_fits(const Fp8GemmArgs& a, const Fp8Parts& pp);
 void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_t st);

@@ -20,6 +20,7 @@
 // e8m0 M = 1 10.5 -> 8.7, 16 12.2 -> 9.6, 16 x 32768 x 1024 36 -> 14; the fused form M = 1 7.2 -> 6.3, 4 10.5 -> 8.7.
 #include <algorithm>
 #include <stdexcept>
+#include <utility>
 
 #include "common.hpp"
 #include "numerics.hpp"
@@ -429,7 +430,7 @@ namespace {
 // more for a round past the first, and `miss` per MB that an XCD's 32 workgroups in flight read from beyond its L2: their
 // row tiles (`abytes` a value) and column blocks. Fitted to 2,900 launches of the dense forms (K = 640 to 8192, N = 640 to
 // 32768, M = 17 to 4096, up to 6 rounds; fp32 scales take 1.035 times as long) and 830 of the grouped ones: rms 6% and 9%.
-// With the tiled GEMM's estimate (fp8_tiled_us) it picks a kernel that is 0.1% slower than the best on average over 990
+// With the tiled GEMM's estimate (fp8_tiled_us) it picks a form that is 0.1% slower than the best on average over 1,200
 // dense calls measured with each, 8% at worst; grouped (tiled_us) 0.2%, 12%.
 struct KpForm {
   int rb, cb;
@@ -441,11 +442,13 @@ double launch_us(const KpForm& f, int M, size_t N, int K, int abytes, double mis
   const double rows = 16.0 * (double(abytes * f.rb) * double(std::min(rt, xcd)) + f.cb * double((xcd + rt - 1) / rt));
   return f.start + double(rounds - 1) * f.next + double(rounds) * K * (f.read * 1e-3 + miss * rows * 1e-6);
 }
-constexpr KpForm kForms[] = {{1, 1, 2.97, 0.0, 0.46}, {2, 1, 3.20, 0.05, 0.70}, {2, 2, 3.34, 0.46, 0.87},
+constexpr KpForm kForms[] = {{1, 1, 2.97, 0.05, 0.46}, {2, 1, 3.20, 0.2, 0.70}, {2, 2, 3.34, 0.46, 0.87},
                              {4, 2, 3.63, 2.20, 1.48}, {4, 4, 4.76, 3.20, 2.03}, {5, 4, 5.64, 3.99, 2.43},
                              {6, 4, 6.07, 4.40, 2.93}};
+// (Workgroups of one 16 x 16 tile take longer with e8m0 scales than with fp32 ones: 1 x 8192 x 1024 5.0 / 4.3 us, 2 x 2 4.7.)
 double form_us(const Fp8GemmArgs& a, const KpForm& f) {
-  return launch_us(f, a.M, size_t(a.N), a.K, 1, 0.23) * (a.sa32 ? 1.035 : 1.0);
+  const double us = launch_us(f, a.M, size_t(a.N), a.K, 1, 0.23);
+  return a.sa32 ? 1.035 * us : f.rb * f.cb == 1 ? us + 0.35 : us;
 }
 int best_form(const Fp8GemmArgs& a) {
   int best = 0;
@@ -470,6 +473,7 @@ void launch_fp8_kpart_parts(const Fp8GemmArgs& a, const Fp8Parts& pp, hipStream_
 }
 void launch_fp8_kpart_xq(const Fp8GemmArgs& a, hipStream_t st) { launch_t<true, 1, 1, true>(a, st); }
 double fp8_kpart_us(const Fp8GemmArgs& a) { return form_us(a, kForms[best_form(a)]); }
+std::pair<int, int> fp8_kpart_form(const Fp8GemmArgs& a) { return {kForms[best_form(a)].rb, kForms[best_form(a)].cb}; }
 
 void launch_fp8_kpart(const Fp8GemmArgs& a, hipStream_t st) {
   if (!fp8_kpart_fits(a)) throw std::runtime_error("fp8 kpart: shape");
