@@ -2,6 +2,7 @@
 // launched and no pointer is read, so it runs without a GPU (tests/test_routes.py).
 //   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | gemv | skinny
 //   form  M N K ldc f32 a_offset w_offset       -> the K-part kernel's tile, row x column blocks of 16
+//   token T K E D I                             -> token (two launches) | general
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
 #include <cstdint>
 #include <iostream>
@@ -9,6 +10,7 @@
 #include <string>
 
 #include "fp8_internal.hpp"
+#include "mx_internal.hpp"
 
 using namespace unholy::kernels;
 
@@ -42,6 +44,10 @@ int main() {
       uintptr_t ao = 0, wo = 0;
       in >> M >> G >> R >> K >> ao >> wo;
       std::cout << kGrouped[int(grouped_route(at(ao), at(wo), M, G, R, K))] << "\n";
+    } else if (kind == "token") {
+      MoeTokenArgs a{};
+      in >> a.T >> a.K >> a.E >> a.D >> a.I;
+      std::cout << (moe_token_fits(a) ? "token" : "general") << "\n";
     } else {
       return 1;
     }

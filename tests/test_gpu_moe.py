@@ -337,7 +337,8 @@ def test_moe_forward_tile_sizes(T, E, K, D, I):
 
 @pytest.mark.parametrize("T,E,K,D,I", [(1, 16, 6, 1024, 512), (1, 8, 2, 4096, 256), (3, 24, 6, 4096, 2048),
                                        (2, 16, 6, 1024, 512), (1, 300, 8, 256, 128), (2, 24, 5, 384, 640),
-                                       (2, 8, 1, 128, 128), (1, 6, 6, 1152, 2304), (4, 6, 2, 512, 256)])
+                                       (2, 8, 1, 128, 128), (1, 6, 6, 1152, 2304), (4, 6, 2, 512, 256),
+                                       (1, 6, 5, 1152, 2304), (1, 6, 6, 512, 2048)])
 def test_moe_forward_few_tokens(T, E, K, D, I):
     """Steps of one and two tokens (two launches: the router's wide form past 256 experts, one and eight picks, the same
     expert for both tokens, units that do not fill the last workgroup, fewer 128-blocks than K parts), and of three and

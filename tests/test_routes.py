@@ -105,3 +105,19 @@ def test_operands_of_any_size_keep_the_fast_kernels(routes):
     dense = [(m, n, k, f) for m in (1, 16, 40, 200) for n, k in ((1 << 20, 8192), (524352, 8192)) for f in (0, 1)]
     assert set(routes([f"dense {m} {n} {k} {n} {f} 0 0" for m, n, k, f in dense])) <= {"kpart", "tiled"}
     assert routes(["grouped 20000 128 64 4096 0 0", "grouped 100 128 1008 65536 0 0"]) == ["kpart", "kpart"]
+
+
+# The forward of one or two tokens in two launches and by the general path (gfx950, us): T, K, E, D, I.
+MEASURED_TOKEN = [
+    (1, 1, 256, 4096, 2048, 15.4, 24.5), (1, 6, 256, 4096, 2048, 25.0, 30.7), (1, 7, 256, 4096, 2048, 35.6, 32.3),
+    (1, 8, 256, 4096, 2048, 37.3, 34.5), (2, 3, 256, 4096, 2048, 24.4, 30.1), (2, 4, 256, 4096, 2048, 34.6, 33.4),
+    (2, 7, 256, 4096, 2048, 56.1, 45.6), (2, 8, 32, 4096, 2048, 57.3, 46.1), (2, 6, 64, 2048, 1024, 17.7, 22.7),
+    (2, 7, 64, 2048, 1024, 25.4, 23.7), (1, 6, 16, 7168, 2048, 34.3, 42.2), (1, 7, 16, 7168, 2048, 51.9, 44.1),
+    (2, 3, 16, 7168, 2048, 32.7, 42.2), (2, 6, 16, 7168, 2048, 61.2, 55.1), (1, 2, 8, 4096, 6144, 24.6, 35.8),
+    (1, 5, 8, 4096, 6144, 54.1, 48.0), (2, 6, 8, 4096, 6144, 108.3, 64.3), (2, 8, 128, 1024, 512, 14.7, 19.6)]
+
+
+def test_few_tokens_take_the_faster_path(routes):
+    answers = routes([f"token {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_TOKEN])
+    bad = [(c, a) for c, a in zip(MEASURED_TOKEN, answers) if a != ("token" if c[5] < c[6] else "general")]
+    assert not bad, bad

@@ -9,7 +9,12 @@
 //   bf16 sums are added in LDS in ascending expert order, as moe_combine does. 256 workgroups at D = 4096.
 // Whole forward, us, general path / this: E = 256, D = 4096, I = 2048: T = 1 29.8 / 23.8, 2 41.9 / 41.0, 3 58.4 / 58.7, 4
 // 66.9 / 74.3; E = 32: T = 1 29.8 / 23.4, 2 40.9 / 39.7, 3 46.4 / 55.3; E = 64, D = 2048, I = 1024: T = 1 21.4 / 14.0, 2
-// 22.5 / 15.8, 3 23.9 / 24.7. So up to two tokens.
+// 22.5 / 15.8, 3 23.9 / 24.7. So up to two tokens, and only while the first launch is one round of workgroups: in a second
+// one most of the chip waits for a few, and full or not it is the general path's measure at best (T, picks K, us, general
+// / this; E = 256, D = 4096, I = 2048: T = 1 K = 6 (256 workgroups) 30.7 / 25.0, 7 (299) 32.3 / 35.6, 8 34.5 / 37.3; T = 2
+// K = 3 30.1 / 24.4, 4 33.4 / 34.6, 6 (512) 41.9 / 41.4, 7 45.6 / 56.1; E = 16, D = 7168: T = 2 K = 3 42.2 / 32.7, 6 55.1 /
+// 61.2; E = 8, I = 6144: T = 1 K = 2 35.8 / 24.6, 5 48.0 / 54.1; E = 64, D = 2048, I = 1024: T = 2 K = 6 22.7 / 17.7, 7 23.7 /
+// 25.4).
 // The arithmetic is the GEMV's (exact dequantization, one bf16 MFMA per 32-input block), a K part's blocks in input order,
 // the parts added in order. A pick streams its expert's weights whether or not another token picked it too.
 #include <algorithm>
@@ -235,7 +240,8 @@ size_t down_lds(const MoeTokenArgs& a) { return size_t(a.K + 1) * (a.I + 8) * 2;
 
 bool moe_token_fits(const MoeTokenArgs& a) {
   return a.T >= 1 && a.T <= kTokenMaxT && a.K >= 1 && a.K <= 8 && a.K <= a.E && a.E <= 1024 && a.D % 128 == 0 &&
-         a.I % 128 == 0 && up_lds(a) <= 96 * 1024 && down_lds(a) <= 96 * 1024;
+         a.I % 128 == 0 && size_t(a.T) * a.K * (a.I / 16) <= size_t(256) * TU_UNITS &&  // one round of workgroups
+         up_lds(a) <= 96 * 1024 && down_lds(a) <= 96 * 1024;
 }
 void launch_moe_token_up(const MoeTokenArgs& a, hipStream_t st) {
   if (!moe_token_fits(a)) throw std::runtime_error("moe token: shape");
