@@ -3,7 +3,9 @@
 //   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | gemv | skinny
 //   form  M N K ldc f32 a_offset w_offset       -> the K-part kernel's tile, row x column blocks of 16
 //   token T K E D I                             -> token (two launches) | general
+//   shape T K E D I                             -> w4 | w8, the forward's w1 / w3 GEMV
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
+#include <algorithm>
 #include <cstdint>
 #include <iostream>
 #include <sstream>
@@ -48,6 +50,11 @@ int main() {
       MoeTokenArgs a{};
       in >> a.T >> a.K >> a.E >> a.D >> a.I;
       std::cout << (moe_token_fits(a) ? "token" : "general") << "\n";
+    } else if (kind == "shape") {
+      int T, K, E, D, I;
+      in >> T >> K >> E >> D >> I;
+      const size_t n = size_t(moe_live_tiles(T, K, E, 16)) * size_t(I / 128);
+      std::cout << (gemv_four_waves(n, std::min(16, T), D) ? "w4" : "w8") << "\n";
     } else {
       return 1;
     }

@@ -121,3 +121,20 @@ def test_few_tokens_take_the_faster_path(routes):
     answers = routes([f"token {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_TOKEN])
     bad = [(c, a) for c, a in zip(MEASURED_TOKEN, answers) if a != ("token" if c[5] < c[6] else "general")]
     assert not bad, bad
+
+
+# The forward's w1 / w3 GEMV in workgroups of 4 and of 8 waves (gfx950, whole forward, us): T, K, E, D, I. An expert with
+# more rows than a tile is several tiles (E = 8, T = 64); rows that do not fit a third of the LDS keep 8 waves.
+MEASURED_SHAPE = [
+    (1, 2, 4, 4096, 2048, 26.4, 30.1), (5, 4, 4, 4096, 2048, 35.4, 37.1), (8, 4, 4, 4096, 2048, 42.7, 40.4),
+    (16, 4, 4, 4096, 2048, 57.1, 50.0), (24, 2, 4, 4096, 2048, 52.5, 47.2), (8, 4, 8, 2048, 1024, 25.5, 26.8),
+    (16, 4, 8, 2048, 1024, 31.4, 30.1), (4, 6, 32, 4096, 2048, 61.6, 68.2), (5, 2, 32, 4096, 2048, 38.9, 37.4),
+    (3, 6, 256, 4096, 2048, 63.7, 69.2), (4, 6, 256, 4096, 2048, 68.4, 71.5), (12, 2, 256, 4096, 2048, 69.6, 73.0),
+    (2, 4, 16, 7168, 2048, 44.3, 48.9), (12, 4, 16, 7168, 2048, 100.4, 82.5), (16, 4, 8, 4096, 4096, 66.7, 60.8),
+    (24, 2, 8, 4096, 4096, 63.7, 58.1), (16, 4, 8, 4096, 6144, 105.2, 95.3), (64, 8, 8, 4096, 6144, 339.7, 266.5)]
+
+
+def test_the_gemv_workgroup_shape_is_the_measured_one(routes):
+    answers = routes([f"shape {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_SHAPE])
+    bad = [(c, a) for c, a in zip(MEASURED_SHAPE, answers) if a != ("w4" if c[5] < c[6] else "w8")]
+    assert not bad, bad

@@ -887,10 +887,8 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
       gh.h = w.h;
       const int rows = std::min(tile_rows, T);
       mark(2);
-      // The distinct experts that T K uniform picks hit, about the live tiles of the launch.
-      const int live = int(std::lround(E * (1.0 - std::pow(1.0 - double(K) / E, T))));
       k::launch_mx_gemv_x(x, D, w.eidx, D, tiles, w.max_tiles, t(0, 0), t(0, 1), nullptr, I, I, st, ntd, t(1, 0),
-                          t(1, 1), nullptr, rows, gh, std::max(1, live));
+                          t(1, 1), nullptr, rows, gh, k::moe_live_tiles(T, K, E, tile_rows));
       mark(3);
       k::mx_grouped_gemv_x(w.h, I, nullptr, I, tiles, w.max_tiles, t(2, 0), t(2, 1), w.pair_out, D, D, st, ntd,
                            nullptr, nullptr, nullptr, rows, k::MxGlu{});

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "unholy/kernels/exl3_moe.hpp"
@@ -99,6 +101,14 @@ struct MoeTokenArgs {
   uint16_t* out;
 };
 bool moe_token_fits(const MoeTokenArgs& a);
+// About the live tiles of a step: the distinct experts that T K uniform picks hit, each with its rows in tiles of tile_rows.
+inline int moe_live_tiles(int T, int K, int E, int tile_rows) {
+  const double hit = E * (1.0 - std::pow(1.0 - double(K) / E, T)), rows = double(T) * K / hit;
+  const double per = std::min(std::max(1.0, rows / tile_rows + 0.5), double((T + tile_rows - 1) / tile_rows));
+  return std::max(1, int(std::lround(hit * per)));
+}
+// The workgroup shape of the forward's w1 / w3 GEMV: 4 waves, or 8 (launch_gemv_t).
+bool gemv_four_waves(size_t workgroups8, int rows, int K);
 void launch_moe_token_up(const MoeTokenArgs& a, hipStream_t st);
 void launch_moe_token_down(const MoeTokenArgs& a, hipStream_t st);
 
