@@ -4,6 +4,7 @@
 //   form  M N K ldc f32 a_offset w_offset       -> the K-part kernel's tile, row x column blocks of 16
 //   token T K E D I                             -> token (two launches) | general
 //   shape T K E D I                             -> w4 | w8, the forward's w1 / w3 GEMV
+//   moe T K E D I                               -> gemm | gemv, the forward up to 64 tokens
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
 #include <algorithm>
 #include <cstdint>
@@ -55,6 +56,10 @@ int main() {
       in >> T >> K >> E >> D >> I;
       const size_t n = size_t(moe_live_tiles(T, K, E, 16)) * size_t(I / 128);
       std::cout << (gemv_four_waves(n, std::min(16, T), D) ? "w4" : "w8") << "\n";
+    } else if (kind == "moe") {
+      int T, K, E, D, I;
+      in >> T >> K >> E >> D >> I;
+      std::cout << (moe_gemm_pays(T, K, E, D, I) ? "gemm" : "gemv") << "\n";
     } else {
       return 1;
     }

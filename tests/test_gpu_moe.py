@@ -310,9 +310,11 @@ def test_forward_matches_composed_entry_points(T, E, K, D, I):
 
 @pytest.mark.parametrize("T,E,K,D,I", [(9, 16, 2, 256, 128), (40, 32, 6, 512, 256), (64, 64, 8, 256, 128),
                                        (40, 16, 2, 256, 256), (380, 80, 2, 512, 256), (380, 16, 2, 512, 256),
-                                       (100, 16, 1, 512, 128)])
+                                       (100, 16, 1, 512, 128), (9, 64, 8, 1792, 896), (40, 256, 6, 512, 256),
+                                       (64, 192, 8, 512, 256)])
 def test_moe_forward_tile_sizes(T, E, K, D, I):
-    """The forward's GEMM steps over skewed routing: experts with 1 to 130 rows (every count of 16-row blocks of a
+    """The forward's GEMM steps (past 64 tokens, and the last three sizes: enough workgroups for it; the others of up to 64
+    tokens take the GEMVs) over skewed routing: experts with 1 to 130 rows (every count of 16-row blocks of a
     workgroup, a tile past 64 rows where the few-rows kernel takes two groups, tiles past 128 rows), the one-block and
     the many-block dispatch, 2 I > D (no room for hh in the workspace of a small step: the GEMVs), one pick per token
     (bf16 token rows larger than the pair rows' codes, whose workspace bytes they share). Against the oracle, max-rel

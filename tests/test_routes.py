@@ -138,3 +138,20 @@ def test_the_gemv_workgroup_shape_is_the_measured_one(routes):
     answers = routes([f"shape {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_SHAPE])
     bad = [(c, a) for c, a in zip(MEASURED_SHAPE, answers) if a != ("w4" if c[5] < c[6] else "w8")]
     assert not bad, bad
+
+
+# The forward of up to 64 tokens by the GEMM on bf16 rows and by the GEMV (gfx950, us): T, K, E, D, I.
+MEASURED_MOE = [
+    (8, 6, 256, 4096, 2048, 114, 111), (9, 6, 256, 4096, 2048, 112.8, 118.6), (64, 6, 256, 4096, 2048, 337, 353),
+    (9, 4, 32, 4096, 2048, 65.4, 70.4), (9, 4, 64, 2048, 1024, 35.0, 32.0), (16, 4, 64, 2048, 1024, 38.1, 40.9),
+    (9, 6, 64, 2048, 1024, 39.6, 40.8), (9, 4, 8, 4096, 2048, 51.1, 42.6), (32, 4, 8, 4096, 2048, 65.5, 56.0),
+    (64, 4, 8, 4096, 2048, 78.2, 87.3), (48, 8, 8, 4096, 2048, 75.2, 97.3), (64, 4, 4, 4096, 2048, 81.0, 59.7),
+    (64, 8, 8, 2048, 1024, 54.9, 43.2), (12, 4, 24, 3072, 1536, 50.1, 41.6), (12, 4, 16, 7168, 2048, 77.1, 100.2),
+    (9, 4, 128, 1024, 512, 24.8, 21.6), (20, 8, 128, 1024, 512, 35.3, 40.8), (9, 4, 256, 2048, 768, 35.1, 31.8),
+    (10, 6, 256, 2048, 768, 42.9, 46.1)]
+
+
+def test_the_forward_takes_the_faster_of_gemm_and_gemv(routes):
+    answers = routes([f"moe {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_MOE])
+    bad = [(c, a) for c, a in zip(MEASURED_MOE, answers) if a != ("gemm" if c[5] < c[6] else "gemv")]
+    assert not bad, bad
