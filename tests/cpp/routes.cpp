@@ -5,6 +5,7 @@
 //   token T K E D I                             -> token (two launches) | general
 //   shape T K E D I                             -> w4 | w8, the forward's w1 / w3 GEMV
 //   moe T K E D I                               -> gemm | gemv, the forward up to 64 tokens
+//   split tiles N K                             -> split | whole, a single-projection GEMV
 //   grouped M G R K a_offset w_offset           -> rows | kpart | gemv | tiled | ref
 #include <algorithm>
 #include <cstdint>
@@ -60,6 +61,10 @@ int main() {
       int T, K, E, D, I;
       in >> T >> K >> E >> D >> I;
       std::cout << (moe_gemm_pays(T, K, E, D, I) ? "gemm" : "gemv") << "\n";
+    } else if (kind == "split") {
+      int tiles, N, K;
+      in >> tiles >> N >> K;
+      std::cout << (gemv_splits_k(size_t(tiles), size_t(N / 16), K) ? "split" : "whole") << "\n";
     } else {
       return 1;
     }

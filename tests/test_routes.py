@@ -155,3 +155,17 @@ def test_the_forward_takes_the_faster_of_gemm_and_gemv(routes):
     answers = routes([f"moe {t} {k} {e} {d} {i}" for t, k, e, d, i, _, _ in MEASURED_MOE])
     bad = [(c, a) for c, a in zip(MEASURED_MOE, answers) if a != ("gemm" if c[5] < c[6] else "gemv")]
     assert not bad, bad
+
+
+# A forward whose w2 launch (tiles, N, K) splits K over the waves of a workgroup, and does not (gfx950, whole forward, us).
+MEASURED_SPLIT = [
+    (1, 4096, 1024, 22.8, 23.8), (3, 4096, 1024, 27.5, 24.6), (1, 4096, 2048, 23.3, 25.6), (3, 4096, 2048, 29.9, 27.1),
+    (6, 4096, 2048, 37.1, 30.2), (2, 7168, 2048, 39.1, 34.9), (6, 1024, 4096, 24.7, 26.1), (8, 1024, 4096, 26.8, 27.9),
+    (4, 2048, 4096, 26.0, 27.9), (8, 2048, 4096, 39.2, 35.4), (2, 7168, 4096, 43.2, 40.1), (2, 4096, 6144, 31.9, 36.0),
+    (3, 4096, 6144, 38.2, 40.9), (6, 4096, 6144, 66.2, 57.1), (6, 2048, 8192, 48.7, 50.2)]
+
+
+def test_the_gemv_splits_k_where_measured(routes):
+    answers = routes([f"split {t} {n} {k}" for t, n, k, _, _ in MEASURED_SPLIT])
+    bad = [(c, a) for c, a in zip(MEASURED_SPLIT, answers) if a != ("split" if c[3] < c[4] else "whole")]
+    assert not bad, bad

@@ -119,6 +119,8 @@ inline bool moe_gemm_pays(int T, int K, int E, int D, int I) {
   const double mb = 3.0 * D * I * (17.0 / 32.0) * 1e-6;  // an expert's weights
   return T > 8 && (moe_experts_hit(T, K, E) * (I / 128) >= 280.0 || moe_live_tiles(T, K, E, 16) * mb >= 260.0);
 }
+// Whether a single-projection GEMV of ntiles x column_tiles tiles splits K over a workgroup's waves.
+bool gemv_splits_k(size_t ntiles, size_t column_tiles, int K);
 // The workgroup shape of the forward's w1 / w3 GEMV: 4 waves, or 8 (launch_gemv_t).
 bool gemv_four_waves(size_t workgroups8, int rows, int K);
 void launch_moe_token_up(const MoeTokenArgs& a, hipStream_t st);

@@ -587,6 +587,17 @@ static bool ksplit_enabled() {
 
 }  // namespace
 
+// Whether a single-projection launch splits each 16-column tile's K over the 8 waves of a workgroup of its own: while 8-tile
+// workgroups would leave CUs idle and the split ones' rounds (12 waves per CU) cost less in start-ups than their shorter
+// K saves. Whole forward, us, not split / split (the w2 launch): K = I = 1024, 0.7 rounds 23.8 / 22.8, 2 24.6 / 27.5; K =
+// 2048, 0.7 25.6 / 23.3, 1.3 26.5 / 26.5, 2 27.1 / 29.9; K = 4096, 1.3 27.9 / 26.0, 2 31.7 / 33.2; K = 6144, 1.3 36.0 /
+// 31.9, 2 40.9 / 38.2, 2.7 42.0 / 43.3; K = 8192, 2 46.0 / 41.7, 2.7 50.8 / 48.1, 3.3 56.7 / 59.8.
+bool gemv_splits_k(size_t ntiles, size_t column_tiles, int K) {
+  constexpr size_t W = GV_WAVES;
+  return ntiles * cdiv(column_tiles, W) < 256 && K % int(128 * W) == 0 &&
+         double(ntiles * column_tiles * W) <= 256 * 12 * std::max(1.0, K / 2560.0);
+}
+
 // Workgroup shape: 8 waves (128 outputs), one workgroup per CU by its registers. A requantizing epilogue needs a whole
 // 128-output block. 4 waves (three per CU, while three fit the LDS):
 // - where 8-wave workgroups would leave half the CUs idle (up to 128) and the rows fit as bf16: whole forward, w1 / w3 with 8 / 4
@@ -627,13 +638,8 @@ void launch_gemv_t(const MxGemvArgs& a, int ntiles, hipStream_t st) {
   constexpr int W = GV_WAVES;
   const size_t lds = size_t(a.rows_cap) * (a.K + GV_PAD) + size_t(a.rows_cap) * (a.K / 128);
   const size_t ntn = a.split ? size_t(a.split) : size_t(a.N) / 16;
-  [[maybe_unused]] const size_t n8 = size_t(ntiles) * cdiv(ntn, W);
   if constexpr (GM == 0 && NP == 1) {
-    // So few column tiles that one round of workgroups (12 waves per CU) takes a workgroup for each: split each tile's K
-    // over its 8 waves. (Past that the split only multiplies the workgroups' start-ups: the w2 launch of T = 1, 1,536
-    // tiles, took 15 us split and 6 not.)
-    const size_t tiles = size_t(ntiles) * ntn;
-    if (n8 < 256 && tiles * W <= 256 * 12 && a.K % (128 * W) == 0 && !a.out32 && ksplit_enabled()) {
+    if (gemv_splits_k(size_t(ntiles), ntn, a.K) && !a.out32 && ksplit_enabled()) {
       auto* kern = &mx_gemv_kernel<NP, GM, AM, W, true>;
       const size_t l = std::max<size_t>(lds, size_t(W) * NP * 64 * 16);
       set_lds_limit(kern, l);
