@@ -47,7 +47,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   int bx, by;
   const int K = a.K, KS = K / 128, M = a.M;
   const int rt = (M + 127) / 128;
-  if (!dense_block(a.N / TN, rt, rt == 8, bx, by)) return;  // eight row tiles: one per XCD
+  // Eight row tiles of few columns: one per XCD (us, M = 900 x N x K, one per XCD / groups: 1152 x 4096 24.1 / 24.7, 1024 x 7168
+  // 42.8 / 43.7, 2048 x 4096 26.8 / 26.8, but 4096 x 4096 37.2 / 35.9, 8192 x 1024 19.5 / 18.5, 5120 x 5120 63.9 / 62.4).
+  if (!dense_block(a.N / TN, rt, rt == 8 && a.N <= 2048, bx, by)) return;
   const int row0 = by * 128;
   const int Mt = min(128, M - row0), col0 = bx * TN;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;

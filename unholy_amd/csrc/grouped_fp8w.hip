@@ -301,9 +301,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   using T = GroupedTile<TN>;
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
-  // Row tiles on XCDs of their own where they divide evenly (M = 4096, G R = 8192: 259 us against 263).
+  // Row tiles on XCDs of their own where they divide evenly and the columns are few (us, own XCDs / groups, K = 4096: G R = 4096,
+  // M = 1000 66.2 / 68.8, 2048 71.3 / 73.6; 8192, M = 1000 79.7 / 78.5, 3000 222 / 214, 4096 248 / 259; 16384, M = 1000 127 /
+  // 122, 4096 540 / 513; K = 1024, 8192, M = 1000 24.9 / 23.6).
   const int rt = (M + 127) / 128;
-  if (!dense_block(G * R / TN, rt, rt % 8 == 0, bx, by)) return;
+  if (!dense_block(G * R / TN, rt, rt % 8 == 0 && G * R <= 4096, bx, by)) return;
   const int row0 = by * 128;
   const int KS = K / 64, N = G * R, Mt = min(128, M - row0), col0 = bx * TN, grp = col0 / R;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
