@@ -2,6 +2,7 @@
 // launched and no pointer is read, so it runs without a GPU (tests/test_routes.py).
 //   dense M N K ldc f32 a_offset w_offset       -> kpart | tiled | gemv | skinny
 //   form  M N K ldc f32 a_offset w_offset       -> the K-part kernel's tile, row x column blocks of 16
+//   gform M G R K                               -> the grouped K-part kernel's tile
 //   token T K E D I                             -> token (two launches) | general
 //   shape T K E D I                             -> w4 | w8, the forward's w1 / w3 GEMV
 //   moe T K E D I                               -> gemm | gemv, the forward up to 64 tokens
@@ -48,6 +49,11 @@ int main() {
       uintptr_t ao = 0, wo = 0;
       in >> M >> G >> R >> K >> ao >> wo;
       std::cout << kGrouped[int(grouped_route(at(ao), at(wo), M, G, R, K))] << "\n";
+    } else if (kind == "gform") {
+      int M, G, R, K;
+      in >> M >> G >> R >> K;
+      const auto [rb, cb] = grouped_kpart_form(M, G, R, K);
+      std::cout << rb << "x" << cb << "\n";
     } else if (kind == "token") {
       MoeTokenArgs a{};
       in >> a.T >> a.K >> a.E >> a.D >> a.I;

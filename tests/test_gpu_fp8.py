@@ -22,10 +22,9 @@ def _weights_f32s(rng, N, K):
     return q.download((N, K), np.uint8), s.download(((N + 127) // 128, K // 128), np.float32), w
 
 
-# 16 < M <= 256 with N % 32 == 0 takes the row-tile kernel: one to four 2,048-input chunks, ragged last chunks (K = 640,
-# 2,176), one 32-column block (N = 32), a weight-scale row shared by fewer than 128 columns (N = 96), 1 to 8 row tiles;
-# (200, 4096, 1024): the 64-column form over 7 row tiles. Past 256 rows the tiled GEMM, whose last row tile leaves a
-# wave one or no live 32-row block: 300 (44 rows), 400 (16 rows), 480 (96 rows).
+# All of these are the K-part kernel's (tiles of 1 x 1, 2 x 1, 2 x 2 and 4 x 4 blocks of 16): K from one to 64
+# 128-blocks, ragged K parts, two column blocks to 256, a weight-scale row shared by fewer than 128 columns (N = 96), row
+# remainders.
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (5, 384, 1024), (64, 512, 1024), (300, 256, 512), (3, 136, 384),
                                    (1000, 768, 1024), (129, 200, 256), (17, 32, 640), (33, 1024, 8192), (64, 96, 6144),
                                    (48, 256, 2176), (40, 200, 512), (200, 128, 1024), (256, 96, 2176), (129, 64, 384),
@@ -100,12 +99,11 @@ def test_fp8_f32s_fused_quant_is_bit_identical(M, N, K, pad):
         call("uh_gemm_fp8_f32s_x", dx, ldx, dwq, dws, c, N, 17, N, K, None)
 
 
-# (40, 16384, 2048) and (48, 20480, 1152) leave >= 512 workgroups of 64 columns: the wide form (two chunks, the second
-# ragged at K = 1152).
+# (40, 16384, 2048): 4 x 4 tiles; (48, 20480, 1152): more than one round of 2 x 2 ones, K parts of two blocks and of one.
 @pytest.mark.parametrize("M,N,K,pad", [(17, 512, 1024, 0), (64, 1024, 2048, 8), (40, 4096, 1024, 0), (64, 128, 256, 0),
                                        (33, 640, 4096, 64), (40, 16384, 2048, 0), (48, 20480, 1152, 0)])
 def test_fp8_f32s_row_tiles_ldc(M, N, K, pad):
-    """gemm_fp8_f32s at 16 < M <= 64 (the row-tile kernel) with a C row stride wider than N: against the oracle within
+    """gemm_fp8_f32s at 16 < M <= 64 (the K-part kernel) with a C row stride wider than N: against the oracle within
     the bf16 bar, and C columns past N untouched."""
     rng = np.random.default_rng(5 * M + K)
     ldx, ldc = K + pad, N + 8
@@ -120,7 +118,7 @@ def test_fp8_f32s_row_tiles_ldc(M, N, K, pad):
     assert np.all(g[:, N:] == 0x7FC1)
     ref16, _ = oracle.gemm_w8a8(q_ref, sa_ref, wq, ws)
     mr = max_rel(from_bf16(g[:, :N]), from_bf16(ref16))
-    print(f"fp8 f32s row tiles M={M} N={N} K={K} ldc={ldc}: max_rel {mr:.3e}")
+    print(f"fp8 f32s M={M} N={N} K={K} ldc={ldc}: max_rel {mr:.3e}")
     assert mr <= 1e-2
 
 
@@ -233,14 +231,19 @@ def test_fp8_gemm_refuses_narrow_ldc():
         call("uh_gemm_fp8_f32s", q, sa, w, sw, c, N - 32, M, N, K, None)
 
 
-# The K-part kernel's forms (1 x 1 .. 6 x 4 row x column blocks of 16): row and column remainders, fewer 128-blocks than
-# waves, uneven parts, two sets of scales (K > 4096); the tiled kernel's block mapping (1, 3, 5, 8 and 9 row tiles); and
-# K > 8192, which the GEMV takes.
+# The K-part kernel's forms (1 x 1 .. 6 x 4 row x column blocks of 16; test_routes.py checks that every one is here): row
+# and column remainders, fewer 128-blocks than waves, uneven parts, two sets of scales (K > 4096); the tiled kernel (both
+# tile widths, a last row tile of 18 to 122 rows, 1, 2, 3, 5, 6, 8, 9 and 10 row tiles); and K > 8192: the GEMV, the row
+# groups and the tiled GEMM.
+MID_SIZES = [(17, 48, 128), (33, 80, 1152), (47, 4096, 256), (100, 4096, 256), (250, 4096, 256), (300, 4096, 384),
+             (384, 4096, 256), (65, 192, 8192), (18, 32, 5248), (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256),
+             (1100, 1024, 256), (1, 200, 640), (16, 48, 8192), (9, 32768, 128), (70, 200, 256), (20, 64, 9216),
+             (1170, 4096, 128), (250, 4096, 640), (299, 4096, 1152), (300, 4072, 1024), (383, 4096, 1536),
+             (383, 4072, 1536), (699, 2048, 1536), (70, 200, 9216), (100, 256, 9216), (31, 4096, 1024), (61, 4096, 640)]
+
+
 @pytest.mark.parametrize("f32", [False, True])
-@pytest.mark.parametrize("M,N,K", [(17, 48, 128), (33, 80, 1152), (47, 4096, 256), (100, 4096, 256), (250, 4096, 256),
-                                   (300, 4096, 384), (384, 4096, 256), (65, 192, 8192), (18, 32, 5248),
-                                   (128, 32768, 128), (700, 4096, 128), (1000, 2048, 256), (1100, 1024, 256),
-                                   (1, 200, 640), (16, 48, 8192), (9, 32768, 128), (70, 200, 256), (20, 64, 9216), (1170, 4096, 128)])
+@pytest.mark.parametrize("M,N,K", MID_SIZES)
 def test_fp8_mid_sizes(M, N, K, f32):
     """gemm_w8a8_wmma / gemm_fp8_f32s against the oracle within the bf16 bar, C with a row stride past N
     and its columns past N untouched."""

@@ -11,8 +11,8 @@ the sizes the reference's own kernel tests run at (tools/kernel_test/mx_moe.hip:
 - configs[4] fp8 dense 4096 x 4096 at M = 64 and M = 4096 (fp32 scales), against the oracle (M = 4096: a sample of
   512 rows, the first and last included).
 - The DSV4 W8A8 projection shapes (e8m0 scales) at M = 1 / 8 / 64 through every W8A8 entry point.
-- DSV4 projection shapes with fp32 scales through the row-tile kernel (M = 64, and 200 for wo_b): the widest N, the
-  longest K, K = 1,024.
+- DSV4 projection shapes with fp32 scales through the K-part kernel and the tiled GEMM (M = 64, and 200 for
+  wo_b): the widest N, the longest K, K = 1,024.
 Weights are made on the device (splitmix64 bytes, e8m0 scales in [119, 125]) and the touched experts copied back for
 the oracle."""
 import numpy as np
@@ -356,9 +356,8 @@ def test_dsv4_w8a8_shapes(name, N, Kd):
             assert np.array_equal(o, outs[0])
 
 
-# fp32-scale fp8 dense at DSV4 projection shapes through the row-tile kernel (16 < M <= 256): the widest N (head_fp8,
-# 4,040 column blocks), the longest K (wo_b, four 2,048-input chunks; also at M = 200, seven row tiles) and K = 1,024
-# (wq_b: one chunk with 8 of the 16 K parts busy).
+# fp32-scale fp8 dense at DSV4 projection shapes, by the K-part kernel or the tiled GEMM as estimated: the widest N
+# (head_fp8), the longest K (wo_b, eight 128-blocks a wave; also at M = 200) and K = 1,024 (wq_b: one block a wave).
 @pytest.mark.parametrize("name,N,Kd,M", [("wq_b", 32768, 1024, 64), ("wo_b", 4096, 8192, 64), ("wo_b", 4096, 8192, 200),
                                          ("sw2", 4096, 2048, 64), ("head_fp8", 129280, 4096, 64)],
                          ids=["wq_b-64", "wo_b-64", "wo_b-200", "sw2-64", "head_fp8-64"])

@@ -15,7 +15,7 @@ def dev(a):
     return DeviceBuffer.from_array(np.ascontiguousarray(a))
 
 
-# M = 4: the GEMV; 64 and 200: the row-tile kernel (asm-issued loads, counted waits).
+# The K-part kernel: one, several and many row blocks.
 @pytest.mark.parametrize("M", [4, 64, 200])
 def test_graph_replays_fp8_dense_step(M):
     rng = np.random.default_rng(3 + M)
@@ -47,7 +47,7 @@ def test_graph_replays_fp8_dense_step(M):
 
 @pytest.mark.parametrize("M", [1, 64])
 def test_graph_replays_grouped_fp8w(M):
-    """The grouped fp8-weight GEMM (M = 1: the GEMV; 64: the row-tile kernel) replayed: every replay equals eager."""
+    """The grouped fp8-weight GEMM (the K-part kernel) replayed: every replay equals eager."""
     rng = np.random.default_rng(11 + M)
     G, R, K = 4, 512, 4096
     a = dev(randn_bf16(rng, (M, G, K)))

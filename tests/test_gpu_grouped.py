@@ -36,18 +36,16 @@ def test_grouped_fp8w_reference_order_bit_exact(M, G, R, K):
     assert np.array_equal(got, ref16)
 
 
-# M <= 16: the row-tile kernel's 32-column form (R % 32 == 0, K <= 8192: one to four 2,048-input chunks, ragged K);
-# 16 < M <= 384: its 64-column form (R % 64 == 0, K <= 4096: one to four 1,024-input chunks, a ragged last chunk at
-# K = 640 and 1,152, 1 to 12 row tiles, the DSV4 shape); other shapes up to M = 160 the GEMV in 32-row chunks (R = 200
-# is the reference-order kernel; K = 9,216 the GEMV); larger M: the tiled GEMM (128-column tiles, M = 385, 400, 520;
-# 256-column ones for R % 256 == 0 once they make more than 256 workgroups: M = 400, G R = 16,896).
+# The row-tile kernel (up to 8 rows of at least 256 workgroups, G R = 8,192: one to four 2,048-input chunks, ragged K), the
+# K-part kernel (ragged K, row remainders, the DSV4 shape), the reference order (R = 200), the tiled GEMM in 256-column
+# tiles (more than 256 workgroups: M = 400, G R = 16,896).
 @pytest.mark.parametrize("M,G,R,K", [(1, 8, 1024, 4096), (16, 2, 512, 1024), (32, 3, 256, 640), (7, 2, 200, 256),
                                      (33, 2, 256, 512), (100, 2, 256, 512), (200, 3, 128, 384), (300, 2, 384, 1024),
                                      (257, 2, 256, 512), (200, 3, 512, 384), (65, 2, 200, 256), (64, 8, 1024, 4096),
                                      (17, 2, 128, 768), (160, 2, 192, 3072), (48, 3, 64, 1152), (95, 1, 64, 9216),
                                      (4, 3, 96, 640), (16, 1, 32, 8192), (9, 2, 160, 5120), (1, 2, 64, 128),
                                      (384, 1, 64, 256), (385, 1, 128, 384), (400, 2, 256, 512), (520, 2, 384, 1024),
-                                     (400, 1, 16896, 128)])
+                                     (400, 1, 16896, 128), (7, 8, 1024, 640), (8, 8, 1024, 6144), (2, 8, 1024, 8192)])
 def test_grouped_fp8w_fast_path(M, G, R, K):
     rng = np.random.default_rng(M * 7 + G * R + K)
     a, w, sw = _case(rng, M, G, R, K)
@@ -97,13 +95,16 @@ def test_grouped_fp8w_shape_errors():
 
 
 
-# The K-part kernel's forms (1 x 1 .. 8 x 4 row x column blocks of 16, 128- and 64-input slots) at the sizes that select
-# them: row remainders, R a multiple of 16 or 32 only, one 128-block, uneven K parts, more than eight blocks a wave
-# (K = 9,216); the tiled kernel past it with row tiles that do and do not divide over the XCDs.
-@pytest.mark.parametrize("M,G,R,K", [(9, 8, 512, 256), (16, 8, 1024, 128), (30, 8, 1024, 256), (61, 8, 1024, 384),
-                                     (100, 8, 1024, 128), (180, 8, 1024, 128), (250, 8, 1024, 256), (23, 5, 48, 1152),
-                                     (70, 3, 96, 640), (12, 2, 16, 9216), (600, 8, 1024, 256), (1030, 16, 512, 128),
-                                     (1000, 8, 1024, 128), (1170, 4, 1024, 128)])
+# The K-part kernel's forms (1 x 1 .. 8 x 4 row x column blocks of 16, 128- and 64-input slots; test_routes.py checks that
+# every one is here): row remainders, R a multiple of 16 or 32 only, one 128-block, uneven K parts, more than eight blocks
+# a wave (K = 9,216); the tiled kernel with row tiles that do and do not divide over the XCDs.
+MID_SIZES = [(9, 8, 512, 256), (16, 8, 1024, 128), (30, 8, 1024, 256), (61, 8, 1024, 384), (100, 8, 1024, 128),
+             (180, 8, 1024, 128), (250, 8, 1024, 256), (23, 5, 48, 1152), (70, 3, 96, 640), (12, 2, 16, 9216),
+             (600, 8, 1024, 256), (1030, 16, 512, 128), (1000, 8, 1024, 128), (1170, 4, 1024, 128), (100, 8, 1024, 384),
+             (180, 8, 1024, 512), (250, 8, 1024, 640), (500, 4, 1024, 640), (1000, 4, 1024, 128)]
+
+
+@pytest.mark.parametrize("M,G,R,K", MID_SIZES)
 def test_grouped_fp8w_mid_sizes(M, G, R, K):
     rng = np.random.default_rng(M * 5 + G * R + K)
     a, w, sw = _case(rng, M, G, R, K)

@@ -58,8 +58,8 @@ def test_few_rows_never_change_the_order_of_sums(routes):
     assert not bad, bad[:5]
 
 
-# One call with both kernels (gfx950, us, graph replays over weights that do not fit a cache): rows, N (G, R) x K, the K-part
-# kernel's best form, the tiled GEMM. Each differs by more than a tenth.
+# One call with both kernels (gfx950, us, graph replays over weights that do not fit a cache): rows, N (G, R) x K, the
+# K-part kernel's best form, the tiled GEMM. Each differs by more than a tenth.
 MEASURED_DENSE = [
     (300, 4096, 4096, 0, 17.4, 26.6), (384, 4096, 4096, 0, 19.9, 27.7), (1000, 4096, 4096, 0, 52.6, 39.3),
     (2049, 4096, 4096, 0, 106.0, 83.2), (2176, 4096, 4096, 0, 108.9, 83.4), (2304, 4096, 4096, 0, 110.9, 83.5),
@@ -169,3 +169,18 @@ def test_the_gemv_splits_k_where_measured(routes):
     answers = routes([f"split {t} {n} {k}" for t, n, k, _, _ in MEASURED_SPLIT])
     bad = [(c, a) for c, a in zip(MEASURED_SPLIT, answers) if a != ("split" if c[3] < c[4] else "whole")]
     assert not bad, bad
+
+
+def test_every_kpart_form_has_a_gpu_test(routes):
+    from tests.test_gpu_fp8 import MID_SIZES as dense
+    from tests.test_gpu_grouped import MID_SIZES as grouped
+
+    for f32 in (0, 1):
+        route = routes([f"dense {m} {n} {k} {n + 8} {f32} 0 0" for m, n, k in dense])
+        form = routes([f"form {m} {n} {k} {n + 8} {f32} 0 0" for m, n, k in dense])
+        assert {f for f, r in zip(form, route) if r == "kpart"} == {"1x1", "2x1", "2x2", "4x2", "4x4", "5x4", "6x4"}
+        assert set(route) == {"kpart", "tiled", "gemv", "skinny"}
+    route = routes([f"grouped {m} {g} {r} {k} 0 0" for m, g, r, k in grouped])
+    form = routes([f"gform {m} {g} {r} {k}" for m, g, r, k in grouped])
+    assert {f for f, r in zip(form, route) if r == "kpart"} == {"1x1", "1x2", "2x2", "2x4", "4x4", "6x4", "8x4"}
+    assert "tiled" in route

@@ -53,6 +53,7 @@ double fp8_tiled_us(const Fp8GemmArgs& a);
 // The same for the grouped projection (R % 16, K <= 65536).
 bool grouped_kpart_fits(int M, int G, int R, int K);
 double grouped_kpart_us(int M, int G, int R, int K);
+std::pair<int, int> grouped_kpart_form(int M, int G, int R, int K);
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st);
 // The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits (K > 8192,

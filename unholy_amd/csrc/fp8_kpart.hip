@@ -521,6 +521,10 @@ bool grouped_kpart_fits(int M, int G, int R, int K) {
          size_t(128) * G * K * 2 < (size_t(1) << 32);
 }
 double grouped_kpart_us(int M, int G, int R, int K) { return gform_us(M, G * R, K, kGForms[best_gform(M, G, R, K)]); }
+std::pair<int, int> grouped_kpart_form(int M, int G, int R, int K) {
+  const KpForm& f = kGForms[best_gform(M, G, R, K)];
+  return {f.rb, f.cb};
+}
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st) {
   if (!grouped_kpart_fits(M, G, R, K)) throw std::runtime_error("grouped kpart: shape");
