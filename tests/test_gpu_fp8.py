@@ -365,7 +365,7 @@ def test_fp8_weights_past_4_gib(M, f32, parts):
     w = DeviceBuffer(N * K)
     call("uh_memset", w.ptr, 0x38, N * K, None)  # e4m3 1.0
     call("uh_memcpy_h2d", w.ptr + N0 * K, wq.ctypes.data, wq.nbytes)
-    s_all = np.ones(((N + 127) // 128, K // 128), np.float32) if f32 else np.full(((N + 127) // 128, K // 128), 127, np.uint8)
+    s_all = np.full(((N + 127) // 128, K // 128), 1.0 if f32 else 127, np.float32 if f32 else np.uint8)
     s_all[N0 // 128:] = sw
     dq, dsa, dsw, c = dev(q), dev(sa), dev(s_all), DeviceBuffer(M * N * 2)
     if parts:

@@ -73,7 +73,8 @@ MEASURED_DENSE = [
 MEASURED_GROUPED = [
     (384, 8, 1024, 4096, 39.5, 66.5), (1024, 8, 1024, 4096, 95.0, 76.7), (2049, 8, 1024, 4096, 260.8, 183.3),
     (2304, 8, 1024, 4096, 276.0, 186.9), (768, 4, 1024, 4096, 37.9, 66.3), (2049, 4, 1024, 4096, 123.8, 89.2),
-    (384, 32, 1024, 4096, 144.0, 108.3), (384, 8, 1024, 2048, 24.2, 32.0), (2304, 8, 1024, 2048, 157.6, 97.6), (64, 32, 1024, 4096, 42.8, 66.8),
+    (384, 32, 1024, 4096, 144.0, 108.3), (384, 8, 1024, 2048, 24.2, 32.0), (2304, 8, 1024, 2048, 157.6, 97.6),
+    (64, 32, 1024, 4096, 42.8, 66.8),
     (256, 16, 512, 1024, 11.4, 17.7), (2100, 16, 512, 1024, 86.3, 54.0),
     (2100, 2, 2048, 4096, 120.8, 89.0), (2300, 7, 1152, 4096, 240.4, 194.9)]
 

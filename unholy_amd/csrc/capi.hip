@@ -842,10 +842,12 @@ int uh_mx_moe_forward_ev(const uint16_t* x, const float* logits, int T, int K, i
     // Dispatch in one single-block launch up to 512 picks; the routing in that launch too while every token has a
     // wave of its own (T <= 8), else a wave per token over many workgroups first.
     const bool one_block = P <= k::kMoeMidMaxPicks, route_in = one_block && T <= 8;
-    // The GEMM on bf16 rows where it pays (moe_gemm_pays), always past 64 tokens; else the GEMV. Up to 64 tokens the fp8-code
-    // and block-scaled GEMMs are not used, whatever the switches say, and a workspace without room for hh keeps the GEMV.
+    // The GEMM on bf16 rows where it pays (moe_gemm_pays), always past 64 tokens; else the GEMV. Up to 64 tokens the
+    // fp8-code and block-scaled GEMMs are not used, whatever the switches say, and a workspace without room for hh
+    // keeps the GEMV.
     const bool bf16_rows = !prefill_fp8() && k::mx_gemm_exact();
-    const bool rows16 = bf16_rows && (T > 64 || (w.hh && k::mx_gemm_pipe_on() && k::moe_gemm_pays(T, K, E, D, I))), gemv = T <= 64 && !rows16;
+    const bool pays = T > 64 || (w.hh && k::mx_gemm_pipe_on() && k::moe_gemm_pays(T, K, E, D, I));
+    const bool rows16 = bf16_rows && pays, gemv = T <= 64 && !rows16;
     const int tile_rows = gemv ? 16 : k::kExl3TileRows;
     const bool few_rows = size_t(P) <= size_t(10) * E;  // at most 10 rows per expert on average: tiles of few rows
     if (rows16) k::launch_route_xform(logits, s_sel, s_wt, T, E, K, x, w.xa, D, st);

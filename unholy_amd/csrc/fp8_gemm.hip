@@ -270,15 +270,15 @@ __global__ __launch_bounds__(DN_NT) void fp8_skinny_kernel(Fp8GemmArgs a) {
   }
 }
 
-// ---- fp8 dense, small M (<= 64 rows), what the K-part kernel does not take (K > 8192): bandwidth-shaped ----
-// One workgroup per 16-column tile; its 8 waves split K (wave w takes 128-blocks w * per .. + per - 1), so the grid
-// covers every CU and each CU keeps 8 waves x 64 lanes x 128 B of weights in flight (four 128-blocks per wave are
-// loaded before any is used). Lane (nl, g) reads 32 weight bytes of column n0 + nl, inputs 16 g .. + 15 and 64 + 16 g .. + 15
-// of a block, and the same inputs of activation row nl (row tile mt: rows 16 mt + nl) from global memory (A is small and
-// cache-resident), dequantizes both exactly to bf16 (e8m0 scales folded in) and issues 16x16x32 bf16 MFMAs. With fp32
-// scales each block's MFMA chain starts from zero and is folded as acc += raw * (sa * sw). The 8 partial tiles are
-// summed in wave order through LDS. K parts, inputs of an MFMA and order of sums are those of fp8_kpart_kernel: the two give
-// the same bits, and a call that one of them takes may be compared with a call that the other takes.
+// ---- fp8 dense, small M (<= 64 rows), what the K-part kernel does not take (K > 8192, unaligned operands) ----
+// Bandwidth-shaped. One workgroup per 16-column tile; its 8 waves split K (wave w takes 128-blocks w * per ..
+// + per - 1), so the grid covers every CU and each CU keeps 8 waves x 64 lanes x 128 B of weights in flight (four 128-blocks per wave are loaded
+// before any is used). Lane (nl, g) reads 32 weight bytes of column n0 + nl, inputs 16 g .. + 15 and 64 + 16 g .. + 15
+// of a block, and the same inputs of activation row nl (row tile mt: rows 16 mt + nl) from global memory (A is small
+// and cache-resident), dequantizes both exactly to bf16 (e8m0 scales folded in) and issues 16x16x32 bf16 MFMAs. With
+// fp32 scales each block's MFMA chain starts from zero and is folded as acc += raw * (sa * sw). The 8 partial tiles
+// are summed in wave order through LDS. K parts, inputs of an MFMA and order of sums are those of fp8_kpart_kernel:
+// the two give the same bits, and a call that one of them takes may be compared with a call that the other takes.
 constexpr int FV_WAVES = 8, FV_CHUNK = 4;
 
 // XQ: A arrives as bf16 rows (a.xa). The workgroup first quantizes its M rows into LDS as act_quant_fp8_f32s does
@@ -483,8 +483,9 @@ static size_t skinny_lds(const Fp8GemmArgs& a) {
 
 Fp8Route fp8_route(const Fp8GemmArgs& a) {
   const bool aligned = fp8_aligned(a.a, a.w);
-  // Rows that the fused and the multi-range entry points take: the K-part kernel or the GEMV, whose results are equal bit for
-  // bit (the tiled GEMM adds in another order: 65536 x 1024, M = 1 19.3 us there, 23.2 with the K-part kernel).
+  // Rows that the fused and the multi-range entry points take: the K-part kernel or the GEMV, whose results are equal
+  // bit for bit (the tiled GEMM adds in another order: 65536 x 1024, M = 1 19.3 us there, 23.2 with the K-part
+  // kernel).
   const bool same_bits = a.M <= (a.sa32 ? 16 : 32);
   if (fp8_kpart_fits(a))
     return same_bits || !fp8_tiled_fits(a) || fp8_kpart_us(a) < fp8_tiled_us(a) ? Fp8Route::kpart : Fp8Route::tiled;

@@ -56,9 +56,9 @@ double grouped_kpart_us(int M, int G, int R, int K);
 std::pair<int, int> grouped_kpart_form(int M, int G, int R, int K);
 void launch_grouped_kpart(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* c, int M, int G, int R, int K,
                           hipStream_t st);
-// The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits (K > 8192,
-// N % 128) the GEMV (M <= 64) or the row-group kernel. The first two load operands straight into LDS, 16 bytes a lane, and
-// are kept to 16-byte aligned operands; the GEMV and the row groups take any.
+// The kernel of a dense product: the K-part kernel or the tiled GEMM, by their estimated times; where neither fits (K
+// > 8192, unaligned operands) the GEMV (M <= 64) or the row-group kernel. The first two load operands straight into LDS, 16 bytes
+// a lane, and are kept to 16-byte aligned operands; the GEMV and the row groups take any.
 enum class Fp8Route { kpart, tiled, gemv, skinny };
 Fp8Route fp8_route(const Fp8GemmArgs& a);
 inline bool fp8_aligned(const void* a, const void* w) {

@@ -425,13 +425,14 @@ void launch_g(const uint16_t* a, const uint8_t* w, const uint8_t* sw, uint16_t* 
 }  // namespace
 
 namespace {
-// The forms (16-row blocks x 16-column blocks), and what a launch of each takes, us: `start` (the launch, the first loads and
-// the reduction) and `read` per 1,000 inputs (each workgroup's rows and columns of K) for a round of 256 workgroups, `next`
-// more for a round past the first, and `miss` per MB that an XCD's 32 workgroups in flight read from beyond its L2: their
-// row tiles (`abytes` a value) and column blocks. Fitted to 2,900 launches of the dense forms (K = 640 to 8192, N = 640 to
-// 32768, M = 17 to 4096, up to 6 rounds; fp32 scales take 1.035 times as long) and 830 of the grouped ones: rms 6% and 9%.
-// With the tiled GEMM's estimate (fp8_tiled_us) it picks a form that is 0.1% slower than the best on average over 1,200
-// dense calls measured with each, 8% at worst; grouped (tiled_us) 0.2%, 12%.
+// The forms (16-row blocks x 16-column blocks), and what a launch of each takes, us: `start` (the launch, the first
+// loads and the reduction) and `read` per 1,000 inputs (each workgroup's rows and columns of K) for a round of 256
+// workgroups, `next` more for a round past the first, and `miss` per MB that an XCD's 32 workgroups in flight read
+// from beyond its L2: their row tiles (`abytes` a value) and column blocks. Fitted to 2,900 launches of the dense
+// forms (K = 640 to 8192, N = 640 to 32768, M = 17 to 4096, up to 6 rounds; fp32 scales take 1.035 times as long) and
+// 830 of the grouped ones: rms 6% and 9%. With the tiled GEMM's estimate (fp8_tiled_us) it picks a form that is 0.1%
+// slower than the best on average over 1,200 dense calls measured with each, 8% at worst; grouped (tiled_us) 0.2%,
+// 12%.
 struct KpForm {
   int rb, cb;
   double start, next, read;
@@ -445,7 +446,8 @@ double launch_us(const KpForm& f, int M, size_t N, int K, int abytes, double mis
 constexpr KpForm kForms[] = {{1, 1, 2.97, 0.05, 0.46}, {2, 1, 3.20, 0.2, 0.70}, {2, 2, 3.34, 0.46, 0.87},
                              {4, 2, 3.63, 2.20, 1.48}, {4, 4, 4.76, 3.20, 2.03}, {5, 4, 5.64, 3.99, 2.43},
                              {6, 4, 6.07, 4.40, 2.93}};
-// (Workgroups of one 16 x 16 tile take longer with e8m0 scales than with fp32 ones: 1 x 8192 x 1024 5.0 / 4.3 us, 2 x 2 4.7.)
+// (Workgroups of one 16 x 16 tile take longer with e8m0 scales than with fp32 ones: 1 x 8192 x 1024 5.0 / 4.3 us, 2 x
+// 2 4.7.)
 double form_us(const Fp8GemmArgs& a, const KpForm& f) {
   const double us = launch_us(f, a.M, size_t(a.N), a.K, 1, 0.23);
   return a.sa32 ? 1.035 * us : f.rb * f.cb == 1 ? us + 0.35 : us;

@@ -47,8 +47,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   int bx, by;
   const int K = a.K, KS = K / 128, M = a.M;
   const int rt = (M + 127) / 128;
-  // Eight row tiles of few columns: one per XCD (us, M = 900 x N x K, one per XCD / groups: 1152 x 4096 24.1 / 24.7, 1024 x 7168
-  // 42.8 / 43.7, 2048 x 4096 26.8 / 26.8, but 4096 x 4096 37.2 / 35.9, 8192 x 1024 19.5 / 18.5, 5120 x 5120 63.9 / 62.4).
+  // Eight row tiles of few columns: one per XCD (us, M = 900 x N x K, one per XCD / groups: 1152 x 4096 24.1 / 24.7,
+  // 1024 x 7168 42.8 / 43.7, 2048 x 4096 26.8 / 26.8, but 4096 x 4096 37.2 / 35.9, 8192 x 1024 19.5 / 18.5, 5120 x
+  // 5120 63.9 / 62.4).
   if (!dense_block(a.N / TN, rt, rt == 8 && a.N <= 2048, bx, by)) return;
   const int row0 = by * 128;
   const int Mt = min(128, M - row0), col0 = bx * TN;
@@ -259,11 +260,11 @@ bool fp8_tiled_fits(const Fp8GemmArgs& a) {
   return a.N % 128 == 0 && a.K % 128 == 0 && a.ldc % 8 == 0 && FpTile<128>::lds(a.K, a.sa32 != nullptr) <= 80 * 1024;
 }
 
-// What a launch takes, us (K = 640 to 8192; fp32 scales 1.06 times that): a time per 128-input stage by the number w of
-// workgroups of 128 columns. Up to 255 they run as twice as many of 64 columns, 256 are one a CU, 512 two a CU; past that full
-// rounds of 512 and a last one that costs what its own workgroups do: a CU with one of them runs its stages faster than
-// with two. M x 4096 x 4096, measured / this: 512 28.2 / 26.4, 1000 38.9 / 37.9, 2000 64 / 60, 2049 84 / 83, 3000 91 / 88, 4096
-// 119 / 118.
+// What a launch takes, us (K = 640 to 8192; fp32 scales 1.06 times that): a time per 128-input stage by the number w
+// of workgroups of 128 columns. Up to 255 they run as twice as many of 64 columns, 256 are one a CU, 512 two a CU;
+// past that full rounds of 512 and a last one that costs what its own workgroups do: a CU with one of them runs its
+// stages faster than with two. M x 4096 x 4096, measured / this: 512 28.2 / 26.4, 1000 38.9 / 37.9, 2000 64 / 60, 2049
+// 84 / 83, 3000 91 / 88, 4096 119 / 118.
 double fp8_tiled_us(const Fp8GemmArgs& a) {
   const size_t w = size_t(a.N / 128) * ((size_t(a.M) + 127) / 128), rem = w % 512;
   const double first = rem == 0     ? 0.0

@@ -261,7 +261,8 @@ __global__ __launch_bounds__(1024) void grouped_fp8w_rows_kernel(const bf16* a, 
   if (rr < M) c[size_t(rr) * N + n] = f32_to_bf16(sum);
 }
 
-// Up to 8 rows while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part kernel, 8 9.28 / 9.43, 16 10.9 / 10.1).
+// Up to 8 rows while it makes 256 workgroups (M = 1 9.05 us against 9.13 for the K-part kernel, 8 9.28 / 9.43, 16 10.9
+// / 10.1).
 bool rows_fits(int M, int G, int R, int K) {
   return M >= 1 && M <= 8 && R % 32 == 0 && K <= GR_MAXCH * GR_KR && size_t(G) * R / GR_W >= 256 &&
          size_t(M) * G * K * 2 < (size_t(1) << 32);
@@ -301,9 +302,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   using T = GroupedTile<TN>;
   extern __shared__ __align__(16) uint8_t smem[];
   int bx, by;
-  // Row tiles on XCDs of their own where they divide evenly and the columns are few (us, own XCDs / groups, K = 4096: G R = 4096,
-  // M = 1000 66.2 / 68.8, 2048 71.3 / 73.6; 8192, M = 1000 79.7 / 78.5, 3000 222 / 214, 4096 248 / 259; 16384, M = 1000 127 /
-  // 122, 4096 540 / 513; K = 1024, 8192, M = 1000 24.9 / 23.6).
+  // Row tiles on XCDs of their own where they divide evenly and the columns are few (us, own XCDs / groups, K = 4096:
+  // G R = 4096, M = 1000 66.2 / 68.8, 2048 71.3 / 73.6; 8192, M = 1000 79.7 / 78.5, 3000 222 / 214, 4096 248 / 259;
+  // 16384, M = 1000 127 / 122, 4096 540 / 513; K = 1024, 8192, M = 1000 24.9 / 23.6).
   const int rt = (M + 127) / 128;
   if (!dense_block(G * R / TN, rt, rt % 8 == 0 && G * R <= 4096, bx, by)) return;
   const int row0 = by * 128;
@@ -420,8 +421,8 @@ void launch_ref(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int
   UH_CHECK_LAUNCH();
 }
 
-// The GEMV for up to 160 rows (32-row chunks side by side), what the K-part kernel does not take: at the DSV4 shape M = 64 it
-// ran 46 us as two chunks, the tiled kernel 69 us (64 workgroups).
+// The GEMV for up to 160 rows (32-row chunks side by side), what the K-part kernel does not take: at the DSV4 shape M
+// = 64 it ran 46 us as two chunks, the tiled kernel 69 us (64 workgroups).
 constexpr int GV_MAX_ROWS = 160;
 bool gemv_fits(int M, int R) { return M <= GV_MAX_ROWS && R % 16 == 0; }
 void launch_gemv(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, int M, int G, int R, int K,
@@ -455,9 +456,9 @@ void launch_tiled(const bf16* a, const uint8_t* w, const uint8_t* sw, bf16* c, i
   else launch_tiled_t<128>(a, w, sw, c, M, G, R, K, st);
 }
 
-// What a tiled launch takes, us (K = 512 to 8192): a time per 64-input stage by the workgroups, 512 of which run at a time, as
-// fp8_tiled_us has it. G R = 8192, K = 4096, measured / this: M = 512 67.5 / 64.5, 1000 77 / 73, 2000 115 / 114, 2049 186 / 192,
-// 4096 269 / 270.
+// What a tiled launch takes, us (K = 512 to 8192): a time per 64-input stage by the workgroups, 512 of which run at a
+// time, as fp8_tiled_us has it. G R = 8192, K = 4096, measured / this: M = 512 67.5 / 64.5, 1000 77 / 73, 2000 115 /
+// 114, 2049 186 / 192, 4096 269 / 270.
 double tiled_us(int M, int G, int R, int K) {
   const size_t w = (size_t(M) + 127) / 128 * (size_t(G) * R / 128);
   const auto rounds = [](size_t n, double full, double part, double slope) {

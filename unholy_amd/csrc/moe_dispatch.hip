@@ -1159,23 +1159,23 @@ void route_fast(const float* logits, const float* bias, const int32_t* tid2eid, 
                 int vocab) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_fast: E <= 1024, K in [1, 8]");
-  (E <= 256 ? &route_wave_kernel<0, 4> : &route_wave_kernel<0, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, tid2eid, ids, sel, weights, T, E, K,
-                                                            route_scale, bias_vl, vocab);
+  auto* kern = E <= 256 ? &route_wave_kernel<0, 4> : &route_wave_kernel<0, 16>;
+  kern<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, tid2eid, ids, sel, weights, T, E, K, route_scale, bias_vl, vocab);
   UH_CHECK_LAUNCH();
 }
 void route_glm(const float* logits, const float* bias, int32_t* sel, float* weights, int T, int E, int K,
                float route_scale, hipStream_t st) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_glm: E <= 1024, K in [1, 8]");
-  (E <= 256 ? &route_wave_kernel<1, 4> : &route_wave_kernel<1, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, nullptr, nullptr, sel, weights, T, E, K,
-                                                            route_scale, nullptr, 0);
+  auto* kern = E <= 256 ? &route_wave_kernel<1, 4> : &route_wave_kernel<1, 16>;
+  kern<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, bias, nullptr, nullptr, sel, weights, T, E, K, route_scale, nullptr, 0);
   UH_CHECK_LAUNCH();
 }
 void route_softmax(const float* logits, int32_t* sel, float* weights, int T, int E, int K, hipStream_t st) {
   if (T <= 0) return;
   if (E > 1024 || K <= 0 || K > kMaxK || K > E) throw std::runtime_error("route_softmax: E <= 1024, K in [1, 8]");
-  (E <= 256 ? &route_wave_kernel<2, 4> : &route_wave_kernel<2, 16>)<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, nullptr, nullptr, nullptr, sel, weights, T, E, K,
-                                                            1.0f, nullptr, 0);
+  auto* kern = E <= 256 ? &route_wave_kernel<2, 4> : &route_wave_kernel<2, 16>;
+  kern<<<cdiv(size_t(T), 4), 256, 0, st>>>(logits, nullptr, nullptr, nullptr, sel, weights, T, E, K, 1.0f, nullptr, 0);
   UH_CHECK_LAUNCH();
 }
 

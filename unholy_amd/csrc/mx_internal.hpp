@@ -108,13 +108,14 @@ inline int moe_live_tiles(int T, int K, int E, int tile_rows) {
   const double per = std::min(std::max(1.0, rows / tile_rows + 0.5), double((T + tile_rows - 1) / tile_rows));
   return std::max(1, int(std::lround(hit * per)));
 }
-// Up to 64 tokens: whether the GEMM on bf16 rows beats the GEMV. Its workgroups (a tile x 128 columns of w1 / w3) stream the
-// weights no faster than their chain of stages, so it needs more than one a CU, or weights that take the GEMV longer:
-// the GEMV reads an expert once per 16 rows. us per forward, GEMV / GEMM: E = 256, D = 4096, I = 2048, 6 picks (workgroups past
-// 280): T = 8 111 / 114, 9 119 / 113, 16 173 / 162, 64 353 / 337; E = 64, D = 2048, I = 1024, 4 picks: T = 9 (226) 32.0 / 35.0,
-// 12 (277) 34.7 / 35.5, 16 (330) 40.9 / 38.1; E = 8, D = 4096, I = 2048 (128), 4 picks: T = 9 (107 MB) 42.6 / 51.1, 32 (161) 56.0 /
-// 65.5, 64 (268) 87.3 / 78.2; 8 picks, T = 48 (375) 97.3 / 75.2; E = 16, D = 7168, 4 picks, T = 12 (364) 100 / 77. Over 460
-// calls timed with both the choice is 0.1% slower than the best on average, 8% at worst.
+// Up to 64 tokens: whether the GEMM on bf16 rows beats the GEMV. Its workgroups (a tile x 128 columns of w1 / w3)
+// stream the weights no faster than their chain of stages, so it needs more than one a CU, or weights that take the
+// GEMV longer: the GEMV reads an expert once per 16 rows. us per forward, GEMV / GEMM: E = 256, D = 4096, I = 2048, 6
+// picks (workgroups past 280): T = 8 111 / 114, 9 119 / 113, 16 173 / 162, 64 353 / 337; E = 64, D = 2048, I = 1024, 4
+// picks: T = 9 (226) 32.0 / 35.0, 12 (277) 34.7 / 35.5, 16 (330) 40.9 / 38.1; E = 8, D = 4096, I = 2048 (128), 4
+// picks: T = 9 (107 MB) 42.6 / 51.1, 32 (161) 56.0 / 65.5, 64 (268) 87.3 / 78.2; 8 picks, T = 48 (375) 97.3 / 75.2; E
+// = 16, D = 7168, 4 picks, T = 12 (364) 100 / 77. Over 517 calls timed with both the choice is 0.1% slower than the
+// best on average, 8% at worst.
 inline bool moe_gemm_pays(int T, int K, int E, int D, int I) {
   const double mb = 3.0 * D * I * (17.0 / 32.0) * 1e-6;  // an expert's weights
   return T > 8 && (moe_experts_hit(T, K, E) * (I / 128) >= 280.0 || moe_live_tiles(T, K, E, 16) * mb >= 260.0);

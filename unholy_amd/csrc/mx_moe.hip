@@ -600,13 +600,13 @@ bool gemv_splits_k(size_t ntiles, size_t column_tiles, int K) {
 
 // Workgroup shape: 8 waves (128 outputs), one workgroup per CU by its registers. A requantizing epilogue needs a whole
 // 128-output block. 4 waves (three per CU, while three fit the LDS):
-// - where 8-wave workgroups would leave half the CUs idle (up to 128) and the rows fit as bf16: whole forward, w1 / w3 with 8 / 4
-//   waves, us, D = 4096, I = 2048: E = 256, T = 1 (96 workgroups of 8) 32.9 / 29.8; E = 4, T = 5, 4 picks 37.1 / 35.4; but with
-//   the rows as codes T = 8 40.4 / 42.7, T = 16 50.0 / 57.1;
+// - where 8-wave workgroups would leave half the CUs idle (up to 128) and the rows fit as bf16: whole forward, w1 / w3
+//   with 8 / 4 waves, us, D = 4096, I = 2048: E = 256, T = 1 (96 workgroups of 8) 32.9 / 29.8; E = 4, T = 5, 4 picks
+//   37.1 / 35.4; but with the rows as codes T = 8 40.4 / 42.7, T = 16 50.0 / 57.1;
 // - where they would make a second round for at most half of the CUs (257 to 384), with K >= 4096 and the rows' codes
-//   fitting: E = 256, 6 picks: T = 2 (192) 41.8 / 44.6, 3 (281) 61.7 / 58.2, 4 (366) 70.4 / 66.6, 5 (453) 77.3 / 80.9, 8 110 /
-//   115; 2 picks, T = 12 (368) 73.0 / 69.6; but D = 2048, I = 1024, E = 64, T = 8 (278) 32.5 / 33.3, and E = 8, I = 6144, T = 16, 4
-//   picks (384; 67 KB of codes) 95 / 105.
+//   fitting: E = 256, 6 picks: T = 2 (192) 41.8 / 44.6, 3 (281) 61.7 / 58.2, 4 (366) 70.4 / 66.6, 5 (453) 77.3 / 80.9,
+//   8 110 / 115; 2 picks, T = 12 (368) 73.0 / 69.6; but D = 2048, I = 1024, E = 64, T = 8 (278) 32.5 / 33.3, and E =
+//   8, I = 6144, T = 16, 4 picks (384; 67 KB of codes) 95 / 105.
 bool gemv_four_waves(size_t workgroups8, int rows, int K) {
   constexpr size_t kThird = 52 * 1024;
   if (workgroups8 <= 128) return size_t(rows + 1) * (K + 8) * 2 <= kThird;

@@ -1,22 +1,22 @@
-// The routed-expert FFN of a step of very few tokens (uh_mx_moe_forward) in two launches. At one token the weights of its
-// picks are 80 MB, 10 us of HBM, and the general path (dispatch, w1 / w3 GEMV, w2 GEMV, combine) took 29.5 us: 5 + 4.5
-// us of launches with next to nothing in them, and GEMVs whose workgroups (64 or 128 columns of one expert) do not divide over
-// 256 CUs. Here
+// The routed-expert FFN of a step of very few tokens (uh_mx_moe_forward) in two launches. At one token the weights of
+// its picks are 80 MB, 10 us of HBM, and the general path (dispatch, w1 / w3 GEMV, w2 GEMV, combine) took 29.5 us: 5 +
+// 4.5 us of launches with next to nothing in them, and GEMVs whose workgroups (64 or 128 columns of one expert) do not
+// divide over 256 CUs. Here
 // - moe_token_up_kernel routes each token in every workgroup (a wave per token, ~1 us, instead of a launch), quantizes the
 //   token rows, and streams w1 / w3: a unit is a 16-column tile of one pick, a workgroup three units with K split over
 //   four waves each. One token with 6 picks of I = 2048: 768 units, 256 workgroups of 12 waves, one per CU;
-// - moe_token_down_kernel streams w2 and combines: a workgroup is 16 output columns of one token, two waves per pick; the picks'
-//   bf16 sums are added in LDS in ascending expert order, as moe_combine does. 256 workgroups at D = 4096.
-// Whole forward, us, general path / this: E = 256, D = 4096, I = 2048: T = 1 29.8 / 23.8, 2 41.9 / 41.0, 3 58.4 / 58.7, 4
-// 66.9 / 74.3; E = 32: T = 1 29.8 / 23.4, 2 40.9 / 39.7, 3 46.4 / 55.3; E = 64, D = 2048, I = 1024: T = 1 21.4 / 14.0, 2
-// 22.5 / 15.8, 3 23.9 / 24.7. So up to two tokens, and only while the first launch is one round of workgroups: in a second
-// one most of the chip waits for a few, and full or not it is the general path's measure at best (T, picks K, us, general
-// / this; E = 256, D = 4096, I = 2048: T = 1 K = 6 (256 workgroups) 30.7 / 25.0, 7 (299) 32.3 / 35.6, 8 34.5 / 37.3; T = 2
-// K = 3 30.1 / 24.4, 4 33.4 / 34.6, 6 (512) 41.9 / 41.4, 7 45.6 / 56.1; E = 16, D = 7168: T = 2 K = 3 42.2 / 32.7, 6 55.1 /
-// 61.2; E = 8, I = 6144: T = 1 K = 2 35.8 / 24.6, 5 48.0 / 54.1; E = 64, D = 2048, I = 1024: T = 2 K = 6 22.7 / 17.7, 7 23.7 /
-// 25.4).
-// The arithmetic is the GEMV's (exact dequantization, one bf16 MFMA per 32-input block), a K part's blocks in input order,
-// the parts added in order. A pick streams its expert's weights whether or not another token picked it too.
+// - moe_token_down_kernel streams w2 and combines: a workgroup is 16 output columns of one token, two waves per pick;
+//   the picks' bf16 sums are added in LDS in ascending expert order, as moe_combine does. 256 workgroups at D = 4096.
+// Whole forward, us, general path / this: E = 256, D = 4096, I = 2048: T = 1 29.8 / 23.8, 2 41.9 / 41.0, 3 58.4 /
+// 58.7, 4 66.9 / 74.3; E = 32: T = 1 29.8 / 23.4, 2 40.9 / 39.7, 3 46.4 / 55.3; E = 64, D = 2048, I = 1024: T = 1 21.4
+// / 14.0, 2 22.5 / 15.8, 3 23.9 / 24.7. So up to two tokens, and only while the first launch is one round of
+// workgroups: in a second one most of the chip waits for a few, and full or not it is the general path's measure at
+// best (T, picks K, us, general / this; E = 256, D = 4096, I = 2048: T = 1 K = 6 (256 workgroups) 30.7 / 25.0, 7 (299)
+// 32.3 / 35.6, 8 34.5 / 37.3; T = 2 K = 3 30.1 / 24.4, 4 33.4 / 34.6, 6 (512) 41.9 / 41.4, 7 45.6 / 56.1; E = 16, D =
+// 7168: T = 2 K = 3 42.2 / 32.7, 6 55.1 / 61.2; E = 8, I = 6144: T = 1 K = 2 35.8 / 24.6, 5 48.0 / 54.1; E = 64, D =
+// 2048, I = 1024: T = 2 K = 6 22.7 / 17.7, 7 23.7 / 25.4).
+// The arithmetic is the GEMV's (exact dequantization, one bf16 MFMA per 32-input block), a K part's blocks in input
+// order, the parts added in order. A pick streams its expert's weights whether or not another token picked it too.
 #include <algorithm>
 #include <stdexcept>
 
@@ -31,8 +31,8 @@ using namespace uh;
 
 namespace {
 
-// 128-input steps in flight per wave; a dword of scales covers 4 (8 measured slower: w1 / w3 15.6 -> 15.8 us, w2 8.6 -> 10.1,
-// the unrolled steps run once from a cold instruction cache).
+// 128-input steps in flight per wave; a dword of scales covers 4 (8 measured slower: w1 / w3 15.6 -> 15.8 us, w2 8.6
+// -> 10.1, the unrolled steps run once from a cold instruction cache).
 constexpr int TK_PF = 4, TK_SW = TK_PF / 4;
 
 // Steps [sb, se) of one 16-column tile nt of NP matrices against the bf16 row at ap (lane (nl, g): inputs 8 g .. + 7 of
@@ -208,7 +208,8 @@ __global__ __launch_bounds__(1024) void moe_token_down_kernel(MoeTokenArgs a) {
   const uint8_t* const wp[1] = {a.tab[4 * a.E + e]};
   const uint8_t* const sp[1] = {a.tab[5 * a.E + e]};
   const int per_part = (KS + TD_PARTS - 1) / TD_PARTS, sb = min(KS, part * per_part);
-  const int se = wp[0] && sp[0] ? min(KS, sb + per_part) : sb;  // an expert that is not here: nothing (its rows are undefined)
+  // (an expert that is not here: nothing, its rows are undefined)
+  const int se = wp[0] && sp[0] ? min(KS, sb + per_part) : sb;
   v4f acc[1] = {v4f{0.0f, 0.0f, 0.0f, 0.0f}};
   token_stream<1>(wp, sp, ntn, nt, sb, se, KS, rows + (nl == 0 ? j : K) * ldh + g * 8, acc, [&] {
     const int nthr = blockDim.x, per = I / 8;

@@ -120,14 +120,16 @@ __device__ __forceinline__ void tile_block(int nbx, int& bx, int& by) {
 }
 inline dim3 tile_grid(int nbx, int ntiles) { return dim3(unsigned(nbx), unsigned((ntiles + 7) / 8 * 8)); }
 
-// Block -> (column block bx, row tile by) of a dense GEMM of nbx x rt tiles; false: nothing to do. XCD x (blocks x, x + 8,
-// ...) runs the x-th eighth of the tiles, whatever their counts, in groups of up to 8 row tiles, rows inner: the tiles
-// an XCD has in flight then share few row and column blocks in its L2. (Row tile r on XCD r % 8 throughout, as tile_block does for expert tiles, leaves XCDs idle unless rt is a multiple of 8: M = 512 ran on
-// four of them. Dense fp8 step, 4096 x 4096, row r % 8 / this: M = 128 38.9 / 32.1 us, 512 42.8 / 33.9, 1500 68.4 /
-// 64.2, 2000 75.7 / 71.5, 4096 140 / 134; 100 x 32768 x 1024 62 / 18; 1000 x 2048 x 4096 33.2 / 34.6.)
+// Block -> (column block bx, row tile by) of a dense GEMM of nbx x rt tiles; false: nothing to do. XCD x (blocks x, x
+// + 8, ...) runs the x-th eighth of the tiles, whatever their counts, in groups of up to 8 row tiles, rows inner: the
+// tiles an XCD has in flight then share few row and column blocks in its L2. (Row tile r on XCD r % 8 throughout, as
+// tile_block does for expert tiles, leaves XCDs idle unless rt is a multiple of 8: M = 512 ran on four of them. Dense
+// fp8 step, 4096 x 4096, row r % 8 / this: M = 128 38.9 / 32.1 us, 512 42.8 / 33.9, 1500 68.4 / 64.2, 2000 75.7 /
+// 71.5, 4096 140 / 134; 100 x 32768 x 1024 62 / 18; 1000 x 2048 x 4096 33.2 / 34.6.)
 // A last group of one to three row tiles would read its columns' weights for those few: the groups are of equal size
-// there (grouped step, G R = 4096, K = 4096, M = 1200, groups of 8 + 2 / 5 + 5 row tiles: 69.0 / 67.8 us; 8192, 114.0 / 111.6;
-// from a remainder of 4 on either is better by turns: K = 4096, M = 1500 68.8 / 67.6; K = 2048, M = 2500 53.9 / 54.9).
+// there (grouped step, G R = 4096, K = 4096, M = 1200, groups of 8 + 2 / 5 + 5 row tiles: 69.0 / 67.8 us; 8192, 114.0
+// / 111.6; from a remainder of 4 on either is better by turns: K = 4096, M = 1500 68.8 / 67.6; K = 2048, M = 2500 53.9
+// / 54.9).
 // rows_apart: row tile r on XCD r % 8 (for the caller's cases where that is better, rt a multiple of 8).
 __device__ __forceinline__ bool dense_block(int nbx, int rt, bool rows_apart, int& bx, int& by) {
   const int nw = nbx * rt, x = blockIdx.x & 7, i0 = int(int64_t(x) * nw >> 3), i1 = int(int64_t(x + 1) * nw >> 3);

@@ -18,7 +18,9 @@ __device__ __forceinline__ float sigmoid(float x) {
 #pragma clang fp contract(off)
   return 1.0f / (1.0f + uh::exp_f32(-x));
 }
-__device__ __forceinline__ float lane_f32(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+__device__ __forceinline__ float lane_f32(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
 
 // One token's routing by one wave (MODE 0: DSV4 sqrt-softplus + bias or the hash row, 1: GLM sigmoid + bias, 2:
 // softmax top-K; E <= 64 * NV). Lane l holds the keys of experts l + 64 i. Top-K with ties to the lower index, in
